@@ -50,6 +50,14 @@ struct Traits<float> {
 
 constexpr int kBK = 16;
 
+// One BM x BN tile.  Slices of BK = 16 inner indices go through two LDS
+// buffers: the next slice's global loads are issued before the products of
+// the current one and written to the other buffer after them, so a slice
+// costs its products (64 f64 MFMAs of 64 cycles per wave in a 64 x 64 tile)
+// and one barrier, with the memory latency behind them.  theta of chi = 500
+// (1000 x 978 x 511 in FP64, 256 tiles, one workgroup per CU) took 151 us
+// with the loads between two barriers and takes 98 us; 2048^3 went from 49.6
+// to 59.4 TF/s (57.8 before the tiles of an XCD were made neighbours).
 template <typename R, int OPA, int OPB, int TM, int TN>
 __device__ __forceinline__ void gemm_tile(
     int64_t M, int64_t N, int64_t K, typename Traits<R>::c_t alpha,
@@ -62,10 +70,11 @@ __device__ __forceinline__ void gemm_tile(
   constexpr int BM = 2 * TM * 16;
   constexpr int BN = 2 * TN * 16;
   constexpr int BK = kBK;
-  __shared__ R As_re[BK][BM + 1];
-  __shared__ R As_im[BK][BM + 1];
-  __shared__ R Bs_re[BK][BN + 1];
-  __shared__ R Bs_im[BK][BN + 1];
+  constexpr int UA = BM * BK / 256, UB = BN * BK / 256;  // loads per thread
+  __shared__ R As_re[2][BK][BM + 1];
+  __shared__ R As_im[2][BK][BM + 1];
+  __shared__ R Bs_re[2][BK][BN + 1];
+  __shared__ R Bs_im[2][BK][BN + 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -88,94 +97,72 @@ __device__ __forceinline__ void gemm_tile(
   const R sgnA = (OPA == 2) ? R(-1) : R(1);
   const R sgnB = (OPB == 2) ? R(-1) : R(1);
 
-  for (int64_t k0 = 0; k0 < K; k0 += BK) {
-    // ---- stage op(A)[m0:m0+BM, k0:k0+BK] ----
-    if (OPA == 0) {
-      // element (i,k) at A[i + k*lda]; i fastest -> coalesced
-      constexpr int KSTEP = 256 / BM;
-      const int i = tid % BM;
+  // Load u of a slice: op(A) row ai + u AI, inner index ak + u AK (the
+  // operand's unit-stride index runs along consecutive threads), likewise B.
+  constexpr int AI = OPA == 0 ? 0 : 256 / BK, AK = OPA == 0 ? 256 / BM : 0;
+  constexpr int BJ = OPB == 0 ? 256 / BK : 0, BKS = OPB == 0 ? 0 : 256 / BN;
+  const int ai = OPA == 0 ? tid % BM : tid / BK;
+  const int ak = OPA == 0 ? tid / BM : tid % BK;
+  const int bj = OPB == 0 ? tid / BK : tid % BN;
+  const int bk = OPB == 0 ? tid % BK : tid / BN;
+  const c_t* pa = OPA == 0 ? A + (m0 + ai) + ak * lda
+                           : A + ak + (m0 + ai) * lda;
+  const c_t* pb = OPB == 0 ? B + bk + (n0 + bj) * ldb
+                           : B + (n0 + bj) + bk * ldb;
+  const int64_t step_a = OPA == 0 ? BK * lda : BK;
+  const int64_t step_b = OPB == 0 ? BK : BK * ldb;
+  const int64_t ua = OPA == 0 ? AK * lda : AI * lda;
+  const int64_t ub = OPB == 0 ? BJ * ldb : BKS * ldb;
+  c_t va[UA], vb[UB];
+  auto load = [&](int64_t k0) {
 #pragma unroll
-      for (int kk = tid / BM; kk < BK; kk += KSTEP) {
-        const int64_t gi = m0 + i, gk = k0 + kk;
-        c_t v;
-        if (gi < M && gk < K) {
-          v = A[gi + gk * lda];
-        } else {
-          v.x = R(0);
-          v.y = R(0);
-        }
-        As_re[kk][i] = v.x;
-        As_im[kk][i] = v.y;
-      }
-    } else {
-      // element (i,k) at A[k + i*lda]; k fastest -> coalesced
-      constexpr int ISTEP = 256 / BK;
-      const int kk = tid % BK;
-#pragma unroll
-      for (int i = tid / BK; i < BM; i += ISTEP) {
-        const int64_t gi = m0 + i, gk = k0 + kk;
-        c_t v;
-        if (gi < M && gk < K) {
-          v = A[gk + gi * lda];
-        } else {
-          v.x = R(0);
-          v.y = R(0);
-        }
-        As_re[kk][i] = v.x;
-        As_im[kk][i] = sgnA * v.y;
-      }
+    for (int u = 0; u < UA; ++u) {
+      va[u].x = va[u].y = R(0);
+      if (m0 + ai + u * AI < M && k0 + ak + u * AK < K) va[u] = pa[u * ua];
     }
-    // ---- stage op(B)[k0:k0+BK, n0:n0+BN] ----
-    if (OPB == 0) {
-      // element (k,j) at B[k + j*ldb]; k fastest
-      constexpr int JSTEP = 256 / BK;
-      const int kk = tid % BK;
 #pragma unroll
-      for (int j = tid / BK; j < BN; j += JSTEP) {
-        const int64_t gj = n0 + j, gk = k0 + kk;
-        c_t v;
-        if (gj < N && gk < K) {
-          v = B[gk + gj * ldb];
-        } else {
-          v.x = R(0);
-          v.y = R(0);
-        }
-        Bs_re[kk][j] = v.x;
-        Bs_im[kk][j] = v.y;
-      }
-    } else {
-      // element (k,j) at B[j + k*ldb]; j fastest
-      constexpr int KSTEP = 256 / BN;
-      const int j = tid % BN;
-#pragma unroll
-      for (int kk = tid / BN; kk < BK; kk += KSTEP) {
-        const int64_t gj = n0 + j, gk = k0 + kk;
-        c_t v;
-        if (gj < N && gk < K) {
-          v = B[gj + gk * ldb];
-        } else {
-          v.x = R(0);
-          v.y = R(0);
-        }
-        Bs_re[kk][j] = v.x;
-        Bs_im[kk][j] = sgnB * v.y;
-      }
+    for (int u = 0; u < UB; ++u) {
+      vb[u].x = vb[u].y = R(0);
+      if (n0 + bj + u * BJ < N && k0 + bk + u * BKS < K) vb[u] = pb[u * ub];
     }
-    __syncthreads();
+    pa += step_a;
+    pb += step_b;
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int u = 0; u < UA; ++u) {
+      As_re[buf][ak + u * AK][ai + u * AI] = va[u].x;
+      As_im[buf][ak + u * AK][ai + u * AI] = sgnA * va[u].y;
+    }
+#pragma unroll
+    for (int u = 0; u < UB; ++u) {
+      Bs_re[buf][bk + u * BKS][bj + u * BJ] = vb[u].x;
+      Bs_im[buf][bk + u * BKS][bj + u * BJ] = sgnB * vb[u].y;
+    }
+  };
 
+  if (K > 0) {
+    load(0);
+    store(0);
+    __syncthreads();
+  }
+  int buf = 0;
+  for (int64_t k0 = 0; k0 < K; k0 += BK) {
+    const bool more = k0 + BK < K;
+    if (more) load(k0 + BK);
 #pragma unroll
     for (int ks = 0; ks < BK; ks += 4) {
       const int kr = ks + (lane >> 4);
       R a_re[TM], a_im[TM], b_re[TN], b_im[TN];
 #pragma unroll
       for (int i = 0; i < TM; ++i) {
-        a_re[i] = As_re[kr][wm + i * 16 + (lane & 15)];
-        a_im[i] = As_im[kr][wm + i * 16 + (lane & 15)];
+        a_re[i] = As_re[buf][kr][wm + i * 16 + (lane & 15)];
+        a_im[i] = As_im[buf][kr][wm + i * 16 + (lane & 15)];
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        b_re[j] = Bs_re[kr][wn + j * 16 + (lane & 15)];
-        b_im[j] = Bs_im[kr][wn + j * 16 + (lane & 15)];
+        b_re[j] = Bs_re[buf][kr][wn + j * 16 + (lane & 15)];
+        b_im[j] = Bs_im[buf][kr][wn + j * 16 + (lane & 15)];
       }
 #pragma unroll
       for (int i = 0; i < TM; ++i)
@@ -187,7 +174,9 @@ __device__ __forceinline__ void gemm_tile(
           acc_im[i][j] = Traits<R>::mfma(a_im[i], b_re[j], acc_im[i][j]);
         }
     }
+    if (more) store(buf ^ 1);
     __syncthreads();
+    buf ^= 1;
   }
 
   // ---- epilogue: lane holds column lane%16, rows Traits<R>::row(lane, e) ----
@@ -225,10 +214,17 @@ __global__ __launch_bounds__(256) void gemm_kernel(
     typename Traits<R>::c_t beta, typename Traits<R>::c_t* __restrict__ C,
     int64_t ldc, int64_t sC) {
   const int64_t bz = blockIdx.z;
+  // Consecutive workgroups go to the 8 XCDs in turn: give each XCD (its own
+  // L2) a contiguous run of the tiles, which share columns of B and the
+  // whole of A, instead of every eighth tile.
+  const uint32_t nt = gridDim.x * gridDim.y;
+  uint32_t t = blockIdx.x + gridDim.x * blockIdx.y;
+  const uint32_t q = nt / 8, r = nt % 8, x = t % 8;
+  t = x * q + min(x, r) + t / 8;
   gemm_tile<R, OPA, OPB, TM, TN>(M, N, K, alpha, A + bz * sA, lda, B + bz * sB,
                                  ldb, beta, C + bz * sC, ldc,
-                                 (int64_t)blockIdx.x * (32 * TM),
-                                 (int64_t)blockIdx.y * (32 * TN));
+                                 (int64_t)(t % gridDim.x) * (32 * TM),
+                                 (int64_t)(t / gridDim.x) * (32 * TN));
 }
 
 // Grouped form: problem blockIdx.z described by desc[blockIdx.z]; tiles
@@ -244,6 +240,19 @@ __global__ __launch_bounds__(256) void gemm_grouped_kernel(
                                  d.ldb, d.beta, d.C, d.ldc, m0, n0);
 }
 
+// Whether `count` problems of m x n take 64x64 tiles rather than 32x32: the
+// tiles of a CU run one after the other on its matrix cores, so the time is
+// that of the fullest CU, ceil(tiles / 256) tiles.  A 64x64 tile is four
+// 32x32 ones of work at about 10% less cost each (half the operand traffic);
+// it loses where its last round of tiles leaves CUs idle (5 products of 512
+// x 512 x 512: 320 big tiles, two rounds, 163 us; 1280 small ones, five
+// quarter rounds, 133 us).
+bool big_tiles(int64_t m, int64_t n, int64_t count) {
+  const int64_t big = ((m + 63) / 64) * ((n + 63) / 64) * count;
+  const int64_t small = ((m + 31) / 32) * ((n + 31) / 32) * count;
+  return 40 * ((big + 255) / 256) <= 11 * ((small + 255) / 256);
+}
+
 template <typename R, int OPA, int OPB>
 int32_t launch_ops(hipStream_t s, int64_t m, int64_t n, int64_t k,
                    typename Traits<R>::c_t alpha,
@@ -251,9 +260,7 @@ int32_t launch_ops(hipStream_t s, int64_t m, int64_t n, int64_t k,
                    const typename Traits<R>::c_t* B, int64_t ldb, int64_t sB,
                    typename Traits<R>::c_t beta, typename Traits<R>::c_t* C,
                    int64_t ldc, int64_t sC, int64_t batch) {
-  // 64x64 tiles when they alone give a few hundred workgroups, else 32x32.
-  const int64_t big_tiles = ((m + 63) / 64) * ((n + 63) / 64) * batch;
-  if (big_tiles >= 256) {
+  if (big_tiles(m, n, batch)) {
     dim3 grid((unsigned)((m + 63) / 64), (unsigned)((n + 63) / 64),
               (unsigned)batch);
     hipLaunchKernelGGL((gemm_kernel<R, OPA, OPB, 2, 2>), grid, dim3(256), 0, s,
@@ -307,8 +314,7 @@ int32_t launch_gemm(hipStream_t s, int opA, int opB, int64_t m, int64_t n,
 template <typename R, int OPA, int OPB>
 int32_t launch_grouped_ops(hipStream_t s, const GemmDesc<R>* d, int count,
                            int64_t maxM, int64_t maxN) {
-  const int64_t big_tiles = ((maxM + 63) / 64) * ((maxN + 63) / 64) * count;
-  if (big_tiles >= 256) {
+  if (big_tiles(maxM, maxN, count)) {
     dim3 grid((unsigned)((maxM + 63) / 64), (unsigned)((maxN + 63) / 64),
               (unsigned)count);
     hipLaunchKernelGGL((gemm_grouped_kernel<R, OPA, OPB, 2, 2>), grid,
