@@ -266,13 +266,31 @@ struct Rot {
   bool on;
 };
 
+// Whether a pair can be rotated, and the product a d its off-diagonal is
+// scaled by.  FP64: both columns above the zero threshold zt.  FP32: one of
+// them, with the other's norm taken as the threshold at least: a column
+// below the FP32 floor has no direction of its own, but what it shares with
+// a large column is resolved, and left in place it would stay in the kept
+// vectors (up to the floor, 2e-5 |X|_F, per column).
+template <typename R>
+__device__ __forceinline__ bool pair_open(R a, R d, R zt) {
+  if (sizeof(R) == sizeof(float)) return a > zt || d > zt;
+  return a > zt && d > zt;
+}
+template <typename R>
+__device__ __forceinline__ R pair_scale(R a, R d, R zt) {
+  if (sizeof(R) == sizeof(float))
+    return (a > zt ? a : zt) * (d > zt ? d : zt);
+  return a * d;
+}
+
 template <typename R>
 __device__ __forceinline__ Rot<R> make_rot(R a, R d,
                                            typename JT<R>::c_t g, R zt,
                                            R tol2) {
   Rot<R> o;
   const R absc2 = g.x * g.x + g.y * g.y;
-  o.on = (a > zt && d > zt && absc2 > tol2 * a * d);
+  o.on = pair_open<R>(a, d, zt) && absc2 > tol2 * pair_scale<R>(a, d, zt);
   const R s2 = o.on ? absc2 : (R)1;
   const R inv = JT<R>::rsq_r(s2);
   const R absc = s2 * inv;
@@ -417,9 +435,9 @@ __device__ __forceinline__ int inner_solve(
     const int r = idx % W, c = idx / W;
     if (r < c) {
       const R a = Gp[gpos<NP>(r, r)].x, d = Gp[gpos<NP>(c, c)].x;
-      if (a > zt && d > zt) {
+      if (pair_open<R>(a, d, zt)) {
         const c_t g = Gp[gpos<NP>(r, c)];
-        const R o2 = (g.x * g.x + g.y * g.y) / (a * d);
+        const R o2 = (g.x * g.x + g.y * g.y) / pair_scale<R>(a, d, zt);
         omax = fmax(omax, (double)o2);
         // the sweep can only reduce the pairs it rotates
         off = off || (o2 > tol2 && (!cross || (r < NP && c >= NP)));
@@ -1896,9 +1914,9 @@ int32_t JacobiEngine::run32(qtn_ctx* ctx, float2* X, int64_t ldx, int64_t sX,
 
 // FP64: tol = sqrt(rows) eps / 2 and zero columns below rows eps |X|_F
 // (before the sweeps: never rotated; after them: exact zeros in sig).
-// FP32 (the chosen form's sweeps): tol = sqrt(rows) eps32 and columns below
+// FP32 (the chosen form's sweeps): tol = sqrt(rows) eps32, and columns below
 // 8 sqrt(rows) eps32 |X|_F (the rounding noise a column gathers over the
-// sweeps) are left alone.
+// sweeps) are only rotated against larger ones (pair_open).
 template <typename R>
 int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
                             int64_t ldx, int64_t sX,
@@ -1921,8 +1939,10 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   int n_inner_big = 1;
   if (const char* e = getenv("QTN_JACOBI_INNER")) n_inner_big = std::max(1, atoi(e));
   const int n_inner = (p == 1) ? 40 : n_inner_big;
-  // stop once a sweep's largest scaled off-diagonal is below sqrt(tol)
-  const double conv2 = tol;
+  // Stop once a sweep's largest scaled off-diagonal is below sqrt(conv2):
+  // sqrt(tol), so that the sweep's own rotations leave it converged, unless
+  // the caller refines the vectors (conv2_refined).
+  const double conv2 = conv2_refined > 0.0 ? conv2_refined : tol;
   const int nchunk_x = (int)(rows_p / 64);
   const int nchunk_w = (int)(cols_p / 64);
 

@@ -35,6 +35,9 @@ struct JacobiEngine {
   bool cross_rounds = false;
   int64_t ldw = 0;     // leading dimension of W (0: cols_p)
   const int64_t* chimax_per = nullptr;  // host, per-problem cap (optional)
+  // > 0: the sweeps stop at this square of the largest scaled off-diagonal
+  // (for a caller that refines the vectors itself) instead of at tol
+  double conv2_refined = 0.0;
   int64_t* chimax_dev = nullptr;
   // device arrays (valid after reserve); Gram partials and rotation blocks
   // are complex double, or complex float when `single`
