@@ -701,6 +701,266 @@ __global__ __launch_bounds__(256) void jac_inner(
 }
 
 // ---------------------------------------------------------------------------
+// 2b. The inner solve of a problem that is one block pair (at most 64
+// columns): sweeps to convergence on the whole Gram.  The cyclic order runs
+// over the columns that are there: np = ceil(eff / 2) slot pairs for the
+// eff leading columns up to the last one that can be rotated (padding never
+// is), so a sweep takes 2 np - 1 rounds of np^2 blocks instead of 63 of 1024.
+// Bound by the latency of its dependent rounds: a 12-qubit chi-32 circuit,
+// one gate at a time, spent 426 us per solve (84% of it) in the 63-round
+// solve of 256 threads, run until a sweep rotated nothing; the circuit took
+// 50.9 ms and takes 17.2 ms.
+//
+// One thread per 2x2 block: up to 32 columns 256 threads on double-buffered
+// G and Q planes (one barrier a round), above that 1024 threads with G
+// rewritten in place between two barriers (two buffers of the 64-column
+// planes do not fit the LDS; Q moves within a wave either way, see
+// inner_solve).
+constexpr int kWholeThreads = 1024;
+
+// Sweeps on the planes of np <= NP slot pairs (row stride NP) until a sweep
+// meets no scaled off-diagonal above conv2 (its own rotations then leave
+// them at O(conv2): the fresh Gram of the next outer pass decides), or
+// max_sweeps.  Called by the whole workgroup; the first NP^2 threads own the
+// blocks.  Returns the rotations made; the final Q planes are Qc's.
+template <typename R, int NP>
+__device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
+                                            typename JT<R>::c_t* Gn,
+                                            typename JT<R>::c_t*& Qc, int np,
+                                            R zt, R tol2, R conv2,
+                                            int max_sweeps, int* big,
+                                            int* nrot) {
+  using c_t = typename JT<R>::c_t;
+  constexpr int NBLK = NP * NP;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int P = tid / NP, pc = tid % NP;
+  const bool mine = tid < NBLK && P < np && pc < np;
+  const int blk = P * NP + pc;
+  c_t* Qp = Qc;
+  auto next = [&](int a, int side) {  // slot_next on np pairs
+    if (np == 1) return side;
+    if (side == 0)
+      return a == 0 ? 0 : a == np - 1 ? 2 * (np - 1) + 1 : 2 * (a + 1);
+    return a == 0 ? 2 : 2 * (a - 1) + 1;
+  };
+  int gd[4], qd[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int rs = next(P, q >> 1), cs = next(pc, q & 1);
+    gd[q] = ((rs & 1) * 2 + (cs & 1)) * NBLK + (rs >> 1) * NP + (cs >> 1);
+    qd[q] = ((q >> 1) * 2 + (cs & 1)) * NBLK + P * NP + (cs >> 1);
+  }
+  if (mine) {
+    // Q = the identity: row 2P + side, index np-slot of the column
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int idx = (q & 1) ? 2 * np - 1 - pc : pc;
+      Qp[q * NBLK + blk] =
+          JT<R>::mk(2 * P + (q >> 1) == idx ? (R)1 : (R)0, (R)0);
+    }
+  }
+  if (tid == 0) *nrot = 0;
+  const bool dbuf = Gn != Gc;
+  int rot = 0;
+  for (int sweep = 0; sweep < max_sweeps; ++sweep) {
+    if (tid == 0) *big = 0;
+    __syncthreads();
+    bool any_big = false;
+    for (int round = 0; round < 2 * np - 1; ++round) {
+      c_t b[4], q[4];
+      R ga = 0, gdd = 0;
+      c_t gg = JT<R>::mk((R)0, (R)0);
+      if (mine) {
+        const int dcol = pc * (NP + 1);
+        ga = Gc[dcol].x;
+        gdd = Gc[3 * NBLK + dcol].x;
+        gg = Gc[NBLK + dcol];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          b[u] = Gc[u * NBLK + blk];
+          q[u] = Qp[u * NBLK + blk];
+        }
+      }
+      if (!dbuf) __syncthreads();
+      else __builtin_amdgcn_wave_barrier();
+      const Rot<R> jc = make_rot<R>(ga, gdd, gg, zt, tol2);
+      Rot<R> jr;
+      const int src = (lane & ~(NP - 1)) | (P & (NP - 1));
+      jr.cs = __shfl(jc.cs, src, 64);
+      jr.sn = __shfl(jc.sn, src, 64);
+      jr.er = __shfl(jc.er, src, 64);
+      jr.ei = __shfl(jc.ei, src, 64);
+      if (mine) {
+        rot_right<R>(jc, b[0], b[1]);
+        rot_right<R>(jc, b[2], b[3]);
+        rot_left<R>(jr, b[0], b[2]);
+        rot_left<R>(jr, b[1], b[3]);
+        if (P == pc && jc.on) {
+          any_big = any_big ||
+                    gg.x * gg.x + gg.y * gg.y >
+                        conv2 * pair_scale<R>(ga, gdd, zt);
+          b[0] = JT<R>::mk(jc.ap, (R)0);
+          b[1] = JT<R>::mk((R)0, (R)0);
+          b[2] = JT<R>::mk((R)0, (R)0);
+          b[3] = JT<R>::mk(jc.dq, (R)0);
+          ++rot;
+        }
+        rot_right<R>(jc, q[0], q[1]);
+        rot_right<R>(jc, q[2], q[3]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          Gn[gd[u]] = b[u];
+          Qp[qd[u]] = q[u];
+        }
+      }
+      __syncthreads();
+      c_t* t = Gc;
+      Gc = Gn;
+      Gn = t;
+    }
+    if (any_big) *big = 1;
+    __syncthreads();
+    const int go = *big;
+    __syncthreads();
+    if (!go) break;
+  }
+  if (rot) atomicAdd(nrot, rot);
+  __syncthreads();
+  return *nrot;
+}
+
+// Plane position of the Gram entry (r, c) and of the rotation entry (r, c)
+// on np slot pairs with row stride NP (gpos / qpos for np = NP).
+template <int NP>
+__device__ __forceinline__ int gpos_n(int r, int c, int np) {
+  const int sr = r >= np ? 1 : 0, sc = c >= np ? 1 : 0;
+  const int pr = sr ? 2 * np - 1 - r : r, pc = sc ? 2 * np - 1 - c : c;
+  return (2 * sr + sc) * NP * NP + pr * NP + pc;
+}
+template <int NP>
+__device__ __forceinline__ int qpos_n(int r, int c, int np) {
+  const int sc = c >= np ? 1 : 0, pc = sc ? 2 * np - 1 - c : c;
+  return (2 * (r & 1) + sc) * NP * NP + (r >> 1) * NP + pc;
+}
+
+// grid (1, batch), kWholeThreads threads; arguments as jac_inner's.
+template <typename R>
+__global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
+    const typename JT<R>::c_t* __restrict__ Gp, int nchunk, double tol,
+    double conv2, const double* __restrict__ zthr, int max_sweeps,
+    typename JT<R>::c_t* __restrict__ Qout, int* __restrict__ flags,
+    int* __restrict__ counters, const int* __restrict__ active,
+    double* __restrict__ offmax, int* __restrict__ qpairs,
+    const int* __restrict__ want, int w_mode) {
+  using c_t = typename JT<R>::c_t;
+  constexpr int W = 64, IPT = W * W / kWholeThreads;
+  const int bz = blockIdx.y;
+  if (!active[bz]) return;
+  __shared__ c_t pool[2 * W * W];
+  __shared__ R dg[W];
+  __shared__ int s_eff, s_off, s_big, s_rot;
+  __shared__ double wmax[kWholeThreads / 64];
+  const int tid = threadIdx.x;
+  const R zt = (R)zthr[bz];
+  const R tol2 = (R)(tol * tol);
+  const c_t* src = Gp + (int64_t)bz * nchunk * (W * W);
+  // the lower-left quadrant of the partial Grams is not filled (jac_gram):
+  // its entries are the adjoints of the upper-right one
+  c_t g[IPT];
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const int idx = tid + kWholeThreads * i;
+    const int r = idx % W, c = idx / W;
+    const bool ll = r >= W / 2 && c < W / 2;
+    const int at = ll ? c + W * r : idx;
+    R re = 0, im = 0;
+    for (int ch = 0; ch < nchunk; ++ch) {
+      const c_t v = src[(int64_t)ch * (W * W) + at];
+      re += v.x;
+      im += v.y;
+    }
+    g[i] = JT<R>::mk(re, ll ? -im : im);
+    if (r == c) dg[r] = re;
+  }
+  if (tid == 0) {
+    s_eff = 0;
+    s_off = 0;
+  }
+  __syncthreads();
+  if (tid < W && dg[tid] > (sizeof(R) == sizeof(float) ? (R)0 : zt))
+    atomicMax(&s_eff, tid + 1);
+  // largest scaled off-diagonal, and whether any pair needs a rotation
+  double omax = 0.0;
+  bool off = false;
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const int idx = tid + kWholeThreads * i;
+    const int r = idx % W, c = idx / W;
+    if (r < c && pair_open<R>(dg[r], dg[c], zt)) {
+      const R o2 = (g[i].x * g[i].x + g[i].y * g[i].y) /
+                   pair_scale<R>(dg[r], dg[c], zt);
+      omax = fmax(omax, (double)o2);
+      off = off || o2 > tol2;
+    }
+  }
+#pragma unroll
+  for (int sh = 32; sh > 0; sh >>= 1)
+    omax = fmax(omax, __shfl_xor(omax, sh, 64));
+  if (off) s_off = 1;
+  if ((tid & 63) == 0) wmax[tid >> 6] = omax;
+  __syncthreads();
+  if (tid == 0) {
+    double bm = 0.0;
+    for (int w = 0; w < kWholeThreads / 64; ++w) bm = fmax(bm, wmax[w]);
+    // positive doubles order like their bit patterns
+    if (bm > 0.0)
+      atomicMax((unsigned long long*)&offmax[bz],
+                (unsigned long long)__double_as_longlong(bm));
+  }
+  const int eff = s_eff;
+  if (!s_off) {
+    if (tid == 0) flags[bz] = 0;
+    return;
+  }
+  const int np = (eff + 1) / 2;
+  const bool narrow = np <= 16;
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const int idx = tid + kWholeThreads * i;
+    const int r = idx % W, c = idx / W;
+    if (r < 2 * np && c < 2 * np)
+      pool[narrow ? gpos_n<16>(r, c, np) : gpos_n<32>(r, c, np)] = g[i];
+  }
+  c_t* Qp = narrow ? pool + 2048 : pool + W * W;
+  int total;
+  if (narrow)
+    total = whole_sweeps<R, 16>(pool, pool + 1024, Qp, np, zt, tol2,
+                                (R)conv2, max_sweeps, &s_big, &s_rot);
+  else
+    total = whole_sweeps<R, 32>(pool, pool, Qp, np, zt, tol2, (R)conv2,
+                                max_sweeps, &s_big, &s_rot);
+  if (tid == 0) {
+    flags[bz] = total > 0 ? 1 : 0;
+    if (total > 0) {
+      atomicAdd(&counters[bz], total);
+      atomicAdd(qpairs, 1);
+      if (w_mode == 1 || (w_mode == 2 && want[bz])) atomicAdd(qpairs + 1, 1);
+    }
+  }
+  if (total == 0) return;
+  c_t* q = Qout + (int64_t)bz * (W * W);
+#pragma unroll
+  for (int i = 0; i < IPT; ++i) {
+    const int idx = tid + kWholeThreads * i;
+    const int r = idx % W, c = idx / W;
+    c_t v = JT<R>::mk(r == c ? (R)1 : (R)0, (R)0);
+    if (r < 2 * np && c < 2 * np)
+      v = Qp[narrow ? qpos_n<16>(r, c, np) : qpos_n<32>(r, c, np)];
+    q[idx] = v;
+  }
+}
+
+// ---------------------------------------------------------------------------
 // 3. X_IJ <- X_IJ Q (and W_IJ <- W_IJ Q) for one 64-row chunk.  grid
 // (nchunk_x + nchunk_w, p, batch): chunks below nchunk_x are X's, the rest
 // W's (Wm non-null; only for the problems with want[bz] != 0 when want is
@@ -1760,14 +2020,16 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
       prof_events.push_back(ev[i]);
     }
   }
-#define QTN_TIMED_LAUNCH(e0, e1, kern, grid, ...)                           \
+#define QTN_TIMED_LAUNCH_N(e0, e1, kern, grid, threads, ...)                \
   do {                                                                      \
     if (e0)                                                                 \
-      hipExtLaunchKernelGGL(kern, grid, dim3(256), 0, s, e0, e1, 0,         \
+      hipExtLaunchKernelGGL(kern, grid, dim3(threads), 0, s, e0, e1, 0,     \
                             __VA_ARGS__);                                   \
     else                                                                    \
-      hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, __VA_ARGS__);         \
+      hipLaunchKernelGGL(kern, grid, dim3(threads), 0, s, __VA_ARGS__);     \
   } while (0)
+#define QTN_TIMED_LAUNCH(e0, e1, kern, grid, ...) \
+  QTN_TIMED_LAUNCH_N(e0, e1, kern, grid, 256, __VA_ARGS__)
   if (fused && WW == 32) {
     if constexpr (std::is_same<R, float>::value) {
       if (res_round(nchunk_x, Wm ? nchunk_w : 0)) {
@@ -1789,6 +2051,12 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
   QTN_TIMED_LAUNCH(ev[0], ev[1], (jac_gram<R, WW>), dim3(npart, p, batch),
                    (const c_t*)X, ldx, sX, p, r, nchunk_x, gram_cpw(nchunk_x),
                    G, active);
+  if (WW == 64 && p == 1) {
+    QTN_TIMED_LAUNCH_N(ev[2], ev[3], (jac_inner_whole<R>), dim3(1, batch),
+                       kWholeThreads, (const c_t*)G, npart, tol, tol, zthr,
+                       n_inner, Qc, flags, counters, active, offmax, misc + 2,
+                       (const int*)want_w, Wm ? (per_problem_w ? 2 : 1) : 0);
+  } else
   QTN_TIMED_LAUNCH(ev[2], ev[3], (jac_inner<R, WW>), dim3(p, batch),
                    (const c_t*)G, npart, p, tol, zthr, n_inner, Qc, flags,
                    counters, active, offmax, misc + 2,
@@ -1800,6 +2068,7 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
                    (const c_t*)Qc, flags, active,
                    (const int*)(per_problem_w ? want_w : nullptr));
 #undef QTN_TIMED_LAUNCH
+#undef QTN_TIMED_LAUNCH_N
   return QTN_OK;
 }
 
@@ -1990,22 +2259,29 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   }
   int* host_flags = nullptr;
   QTN_TRY(ctx->pinned_buffer(4 * sizeof(int), (void**)&host_flags));
+  // A problem of one block pair is solved whole by its first pass and
+  // checked on a fresh Gram by the second, so the two go out together (a
+  // read-back less per solve; a problem done after the first skips the
+  // second on the device).  Counted per pass while profiling.
+  const int passes = (p == 1 && !ctx->prof) ? 2 : 1;
   // One sweep: every round, then the convergence bookkeeping.
   auto enqueue_sweep = [&]() -> int32_t {
-    for (int r = 0; r < rounds; ++r) {
-      if (this->W == 64)
-        QTN_TRY((launch_round<R, 64>(s, X, ldx, sX, Wm, sW, r, tol, n_inner,
-                                     nchunk_x, nchunk_w,
-                                     want_w_host != nullptr)));
-      else
-        QTN_TRY((launch_round<R, 32>(s, X, ldx, sX, Wm, sW, r, tol, n_inner,
-                                     nchunk_x, nchunk_w,
-                                     want_w_host != nullptr)));
+    for (int pass = 0; pass < passes; ++pass) {
+      for (int r = 0; r < rounds; ++r) {
+        if (this->W == 64)
+          QTN_TRY((launch_round<R, 64>(s, X, ldx, sX, Wm, sW, r, tol, n_inner,
+                                       nchunk_x, nchunk_w,
+                                       want_w_host != nullptr)));
+        else
+          QTN_TRY((launch_round<R, 32>(s, X, ldx, sX, Wm, sW, r, tol, n_inner,
+                                       nchunk_x, nchunk_w,
+                                       want_w_host != nullptr)));
+      }
+      QTN_CHECK_HIP(hipGetLastError());
+      hipLaunchKernelGGL(jac_sweep_end, dim3(1), dim3(256), 0, s, active,
+                         counters, offmax, conv2, batch, misc);
+      QTN_CHECK_HIP(hipGetLastError());
     }
-    QTN_CHECK_HIP(hipGetLastError());
-    hipLaunchKernelGGL(jac_sweep_end, dim3(1), dim3(256), 0, s, active,
-                       counters, offmax, conv2, batch, misc);
-    QTN_CHECK_HIP(hipGetLastError());
     return QTN_OK;
   };
   // The sweep's launches are captured once into a graph (kernel nodes
@@ -2040,7 +2316,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   }
   int sweep = 0;
   bool converged = false;
-  for (; sweep < max_sweeps; ++sweep) {
+  for (; sweep < max_sweeps; sweep += passes) {
     if (exec)
       QTN_CHECK_HIP(hipGraphLaunch(exec, s));
     else
@@ -2058,7 +2334,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     }
     if (host_flags[0] == 0) {
       converged = true;
-      ++sweep;
+      sweep += passes;
       break;
     }
   }
