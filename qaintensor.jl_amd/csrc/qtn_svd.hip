@@ -79,27 +79,16 @@ struct JT<double> {
   static __device__ __forceinline__ double dv(double a, double b) {
     return a / b;
   }
-  // Rotation parameters (make_rot): the hardware v_rsq_f64 / v_rcp_f64
-  // estimates refined by two Newton steps each (quadratic convergence from
-  // their ~2^-26 relative error to below FP64 rounding), which shortens the
-  // dependent chain of the inner sweep's rounds against the correctly
-  // rounded library sequences.  Arguments are positive and normal (the
-  // rotation guards them).
+  // 1 / sqrt(x) for the rotation parameters (make_rot): the hardware
+  // v_rsq_f64 estimate (relative error e about 2^-26) and one third-order
+  // step, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2, whose error e^3 is
+  // below FP64 rounding: a shorter dependent chain than the correctly
+  // rounded library sequence or two Newton steps, and the inner sweep is
+  // bound by that chain.  x is positive and normal (the rotation guards it).
   static __device__ __forceinline__ double rsq_r(double x) {
-    double y = __builtin_amdgcn_rsq(x);
-    const double hx = 0.5 * x;
-    y = y * fma(-hx * y, y, 1.5);
-    y = y * fma(-hx * y, y, 1.5);
-    return y;
-  }
-  static __device__ __forceinline__ double sq_r(double x) {
-    return x * rsq_r(x);
-  }
-  static __device__ __forceinline__ double dv_r(double a, double b) {
-    double r = __builtin_amdgcn_rcp(b);
-    r = fma(r, fma(-b, r, 1.0), r);
-    r = fma(r, fma(-b, r, 1.0), r);
-    return a * r;
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(e, 0.375, 0.5), y);
   }
 };
 template <>
@@ -131,10 +120,6 @@ struct JT<float> {
     return a * __builtin_amdgcn_rcpf(b);
   }
   static __device__ __forceinline__ float rsq_r(float x) { return rsq(x); }
-  static __device__ __forceinline__ float sq_r(float x) { return sq(x); }
-  static __device__ __forceinline__ float dv_r(float a, float b) {
-    return dv(a, b);
-  }
 };
 
 // Round-robin (circle method) position -> block for 2p blocks.
@@ -253,16 +238,17 @@ inline int gram_parts(int nchunk) {
 
 // Rotation of the pair (p, q) from the Gram entries a = G_pp, d = G_qq and
 // g = G_pq (Golub & Van Loan 8.5, complex Hermitian form):
-//   J = [[cs, sn], [-sn e, cs e]], e = e^{-i phi} = conj(g) / |g|,
-// J^H [[a, g], [conj g, d]] J = diag(ap, dq).  With zeta = (d - a) / (2|g|)
-// and tau = |zeta| + sqrt(1 + zeta^2) (so t = tan = sign(zeta) / tau):
-// cs = tau / sqrt(1 + tau^2), sn = sign(zeta) / sqrt(1 + tau^2).  Computed
-// without branches; a pair that already meets the tolerance (or has a
-// column below the zero threshold) gets cs = 1, sn = 0, e = 1, which
-// leaves every entry it touches unchanged bit for bit.
+//   J = [[cs, conj(s)], [-s, cs]],  J^H [[a, g], [conj g, d]] J = diag(ap, dq)
+// with the smaller of the two angles.  With h = d - a and
+// r = sqrt(h^2 + 4 |g|^2): cos(2 theta) = |h| / r, so cs^2 = (1 + |h| / r) / 2
+// and s = sign(h) conj(g) / (r cs); t = |g| tan(theta) = |g|^2 / (r cs^2).
+// Two reciprocal square roots in sequence, no division and no |g|.  Computed
+// without branches; a pair that already meets the tolerance (or cannot be
+// rotated, pair_open) gets cs = 1, s = 0, which leaves every entry it
+// touches unchanged bit for bit.
 template <typename R>
 struct Rot {
-  R cs, sn, er, ei, ap, dq;
+  R cs, sx, sy, ap, dq;
   bool on;
 };
 
@@ -291,47 +277,46 @@ __device__ __forceinline__ Rot<R> make_rot(R a, R d,
   Rot<R> o;
   const R absc2 = g.x * g.x + g.y * g.y;
   o.on = pair_open<R>(a, d, zt) && absc2 > tol2 * pair_scale<R>(a, d, zt);
-  const R s2 = o.on ? absc2 : (R)1;
-  const R inv = JT<R>::rsq_r(s2);
-  const R absc = s2 * inv;
-  const R zeta = (R)0.5 * (d - a) * inv;
-  const R tau = JT<R>::ab(zeta) + JT<R>::sq_r((R)1 + zeta * zeta);
-  const R rr = JT<R>::rsq_r((R)1 + tau * tau);
-  const R sgn = zeta >= (R)0 ? (R)1 : (R)-1;
-  const R tt = JT<R>::dv_r(sgn, tau);
-  o.cs = o.on ? tau * rr : (R)1;
-  o.sn = o.on ? sgn * rr : (R)0;
-  o.er = o.on ? g.x * inv : (R)1;
-  o.ei = o.on ? -g.y * inv : (R)0;
-  o.ap = o.on ? a - tt * absc : a;
-  o.dq = o.on ? d + tt * absc : d;
+  const R h = d - a;
+  const R ir = JT<R>::rsq_r(o.on ? h * h + (R)4 * absc2 : (R)1);
+  const R c2 = o.on ? (R)0.5 + (R)0.5 * JT<R>::ab(h) * ir : (R)1;
+  const R ic = JT<R>::rsq_r(c2);
+  const R f = h >= (R)0 ? ir * ic : -(ir * ic);
+  const R t = absc2 * f * ic;
+  o.cs = o.on ? c2 * ic : (R)1;
+  o.sx = o.on ? g.x * f : (R)0;
+  o.sy = o.on ? -g.y * f : (R)0;
+  o.ap = o.on ? a - t : a;
+  o.dq = o.on ? d + t : d;
   return o;
 }
 
 // [u v] <- [u v] J (a row of two entries in the columns p, q of the pair)
 template <typename R>
+__device__ __forceinline__ void rot_right(R cs, R sx, R sy,
+                                          typename JT<R>::c_t& u,
+                                          typename JT<R>::c_t& v) {
+  const typename JT<R>::c_t nu =
+      JT<R>::mk(cs * u.x - sx * v.x + sy * v.y,
+                cs * u.y - sx * v.y - sy * v.x);
+  v = JT<R>::mk(cs * v.x + sx * u.x + sy * u.y,
+                cs * v.y + sx * u.y - sy * u.x);
+  u = nu;
+}
+template <typename R>
 __device__ __forceinline__ void rot_right(const Rot<R>& j,
                                           typename JT<R>::c_t& u,
                                           typename JT<R>::c_t& v) {
-  const R yr = j.er * v.x - j.ei * v.y;
-  const R yi = j.er * v.y + j.ei * v.x;
-  const typename JT<R>::c_t nu =
-      JT<R>::mk(j.cs * u.x - j.sn * yr, j.cs * u.y - j.sn * yi);
-  v = JT<R>::mk(j.sn * u.x + j.cs * yr, j.sn * u.y + j.cs * yi);
-  u = nu;
+  rot_right<R>(j.cs, j.sx, j.sy, u, v);
 }
 
-// [u; v] <- J^H [u; v], J^H = [[cs, -sn conj(e)], [sn, cs conj(e)]]
+// [u; v] <- J^H [u; v], J^H = [[cs, -conj(s)], [s, cs]]: the right rotation
+// with conj(s)
 template <typename R>
 __device__ __forceinline__ void rot_left(const Rot<R>& j,
                                          typename JT<R>::c_t& u,
                                          typename JT<R>::c_t& v) {
-  const R yr = j.er * v.x + j.ei * v.y;
-  const R yi = j.er * v.y - j.ei * v.x;
-  const typename JT<R>::c_t nu =
-      JT<R>::mk(j.cs * u.x - j.sn * yr, j.cs * u.y - j.sn * yi);
-  v = JT<R>::mk(j.sn * u.x + j.cs * yr, j.sn * u.y + j.cs * yi);
-  u = nu;
+  rot_right<R>(j.cs, j.sx, -j.sy, u, v);
 }
 
 // Round-robin slots of the inner sweep.  The W indices of the block pair
@@ -524,9 +509,8 @@ __device__ __forceinline__ int inner_solve(
         // the lane of this wave whose column pair is this row pair
         const int src = (lane & ~(NP - 1)) | (pr0 + RS * k);
         jr[k].cs = __shfl(jc.cs, src, 64);
-        jr[k].sn = __shfl(jc.sn, src, 64);
-        jr[k].er = __shfl(jc.er, src, 64);
-        jr[k].ei = __shfl(jc.ei, src, 64);
+        jr[k].sx = __shfl(jc.sx, src, 64);
+        jr[k].sy = __shfl(jc.sy, src, 64);
       }
       // --- transform, then write each entry to its next-round slot
 #pragma unroll
@@ -787,9 +771,8 @@ __device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
       Rot<R> jr;
       const int src = (lane & ~(NP - 1)) | (P & (NP - 1));
       jr.cs = __shfl(jc.cs, src, 64);
-      jr.sn = __shfl(jc.sn, src, 64);
-      jr.er = __shfl(jc.er, src, 64);
-      jr.ei = __shfl(jc.ei, src, 64);
+      jr.sx = __shfl(jc.sx, src, 64);
+      jr.sy = __shfl(jc.sy, src, 64);
       if (mine) {
         rot_right<R>(jc, b[0], b[1]);
         rot_right<R>(jc, b[2], b[3]);
