@@ -678,10 +678,249 @@ __global__ __launch_bounds__(256) void jac_inner(
   if (total > 0) {
     c_t* q = Qout + ((int64_t)bz * p + pi) * (int64_t)(W * W);
     for (int idx = tid; idx < W * W; idx += 256) {
-      const int r = idx % W, c = idx / W;
+      const int r = idx / W, c = idx % W;
       q[idx] = qf[qpos<W / 2>(r, c)];
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// 2a. The inner solve of the cross rounds (every outer round of a sweep but
+// its first, W = 32): sums the partial Grams and rotates the 16 x 16 pairs
+// across the two column blocks once, in 16 rounds.
+//
+// Bound by the latency of its dependent rounds (one workgroup per block
+// pair, 80 to 320 of them), so everything that can stays in registers.
+// Slot pair P holds index P of the first block (side 0, for good) and index
+// 16 + (P + t) mod 16 of the second (side 1) in round t.  Thread (P, c) of
+// waves 0-3 holds the 2x2 block of G between the pairs P and c, thread
+// (R, c) of waves 4-7 the rows 2R, 2R + 1 of Q in the columns of pair c: 16
+// lanes of a row hold the 16 column pairs, so moving the side-1 columns on
+// is a lane rotation within the row (DPP), of G and of Q.  Only the side-1
+// rows of G change threads through LDS (two entries per thread and round),
+// and the round's rotations, which the 16 threads (c, c) derive from their
+// own registers: the next diagonal block is their own side-0 entry, their
+// own off-diagonal entry, and the neighbour pair's new side-1 entry, which
+// travels with its rotation.  One barrier per round.
+// A solve on its own takes 11.1 us (630 x 100 and 100 x 550), 17.6 us with
+// every entry in LDS and three refined roots per round; the 40-qubit chi-256
+// circuit in FP64 393 -> 369 ms, 24 uneven circuits 370 -> 340 ms.
+constexpr int kCrossThreads = 512;
+
+// The value of the next lane of a row of 16 (cyclic): dst lane i <- i + 1.
+template <typename R>
+__device__ __forceinline__ R next_in_row(R x) {
+  constexpr int kRor15 = 0x12f;  // row_ror:15
+  if constexpr (sizeof(R) == 8) {
+    const int2 v = __builtin_bit_cast(int2, x);
+    const int2 r = make_int2(
+        __builtin_amdgcn_update_dpp(v.x, v.x, kRor15, 0xf, 0xf, false),
+        __builtin_amdgcn_update_dpp(v.y, v.y, kRor15, 0xf, 0xf, false));
+    return __builtin_bit_cast(R, r);
+  } else {
+    const int v = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(
+        R, __builtin_amdgcn_update_dpp(v, v, kRor15, 0xf, 0xf, false));
+  }
+}
+
+template <typename R>
+struct CrossShared {
+  typename JT<R>::c_t exch[2][2][256];  // side-1 rows on the move
+  R prm[2][4][16];                      // cs, sx, sy, dq per column pair
+  R dg[32];                             // diagonal of the summed Gram
+  int off, big, rot;
+};
+
+// The 16 rounds.  b: this thread's block of G (waves 0-3) or rows of Q
+// (waves 4-7), in the order (row side, column side); P, c its place.
+// Returns the rotations this thread derived.
+template <typename R>
+__device__ __forceinline__ int cross_rounds(CrossShared<R>& sh,
+                                            typename JT<R>::c_t (&b)[4],
+                                            bool is_g, int P, int c, R zt,
+                                            R tol2) {
+  const bool owner = is_g && P == c;
+  const int at = P * 16 + c, from = ((P + 1) & 15) * 16 + c;
+  R d = b[3].x;
+  int rot = 0;
+  for (int t = 0; t < 16; ++t) {
+    const int cur = t & 1;
+    Rot<R> o;
+    if (is_g) {
+      o = make_rot<R>(b[0].x, d, b[1], zt, tol2);
+      if (owner) {
+        sh.prm[cur][0][c] = o.cs;
+        sh.prm[cur][1][c] = o.sx;
+        sh.prm[cur][2][c] = o.sy;
+        sh.prm[cur][3][c] = o.dq;
+        rot += o.on ? 1 : 0;
+      }
+    }
+    __syncthreads();
+    const R cs = sh.prm[cur][0][c], sx = sh.prm[cur][1][c],
+            sy = sh.prm[cur][2][c];
+    if (is_g) {
+      const R rc = sh.prm[cur][0][P], rx = sh.prm[cur][1][P],
+              ry = sh.prm[cur][2][P];
+      d = sh.prm[cur][3][(c + 1) & 15];
+      if (t > 0) {
+        b[2] = sh.exch[cur ^ 1][0][from];
+        b[3] = sh.exch[cur ^ 1][1][from];
+      }
+      rot_right<R>(cs, sx, sy, b[0], b[1]);
+      rot_right<R>(cs, sx, sy, b[2], b[3]);
+      rot_right<R>(rc, rx, -ry, b[0], b[2]);
+      rot_right<R>(rc, rx, -ry, b[1], b[3]);
+      if (owner && o.on) {
+        b[0] = JT<R>::mk(o.ap, (R)0);
+        b[1] = JT<R>::mk((R)0, (R)0);
+        b[2] = JT<R>::mk((R)0, (R)0);
+        b[3] = JT<R>::mk(o.dq, (R)0);
+      }
+    } else {
+      rot_right<R>(cs, sx, sy, b[0], b[1]);
+      rot_right<R>(cs, sx, sy, b[2], b[3]);
+    }
+    // side-1 columns to the next round's pair
+    b[1] = JT<R>::mk(next_in_row(b[1].x), next_in_row(b[1].y));
+    b[3] = JT<R>::mk(next_in_row(b[3].x), next_in_row(b[3].y));
+    if (is_g) {
+      sh.exch[cur][0][at] = b[2];
+      sh.exch[cur][1][at] = b[3];
+    }
+  }
+  return rot;
+}
+
+// grid (p, batch), kCrossThreads threads; arguments as jac_inner's (Q leaves
+// row by row).
+template <typename R>
+__global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
+    const typename JT<R>::c_t* __restrict__ Gp, int nchunk, int p,
+    double tol, double conv2, const double* __restrict__ zthr, int n_inner,
+    typename JT<R>::c_t* __restrict__ Qout, int* __restrict__ flags,
+    int* __restrict__ counters, const int* __restrict__ active,
+    double* __restrict__ offmax, int* __restrict__ qpairs,
+    const int* __restrict__ want, int w_mode) {
+  using c_t = typename JT<R>::c_t;
+  constexpr int W = 32;
+  const int bz = blockIdx.y, pi = blockIdx.x;
+  if (!active[bz]) return;
+  __shared__ CrossShared<R> sh;
+  const int tid = threadIdx.x;
+  const bool is_g = tid < 256;
+  const int P = (tid & 255) >> 4, c = tid & 15;
+  const R zt = (R)zthr[bz];
+  const R tol2 = (R)(tol * tol);
+  c_t b[4];
+  if (is_g) {
+    // entries (P, c), (P, 16 + c), (16 + P, c), (16 + P, 16 + c): the
+    // partial Grams hold the first, the second and the last; all but the
+    // second are read as the adjoint, along consecutive rows
+    const c_t* src =
+        Gp + ((int64_t)bz * p + pi) * nchunk * (int64_t)(W * W);
+    const int a0 = c + W * P, a1 = P + W * (16 + c), a2 = c + W * (16 + P),
+              a3 = 16 + c + W * (16 + P);
+    R re[4] = {0, 0, 0, 0}, im[4] = {0, 0, 0, 0};
+#pragma unroll 8
+    for (int ch = 0; ch < nchunk; ++ch) {
+      const c_t* g = src + (int64_t)ch * (W * W);
+      const c_t v0 = g[a0], v1 = g[a1], v2 = g[a2], v3 = g[a3];
+      re[0] += v0.x;
+      im[0] -= v0.y;
+      re[1] += v1.x;
+      im[1] += v1.y;
+      re[2] += v2.x;
+      im[2] -= v2.y;
+      re[3] += v3.x;
+      im[3] -= v3.y;
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) b[u] = JT<R>::mk(re[u], im[u]);
+    if (P == c) {
+      sh.dg[c] = re[0];
+      sh.dg[16 + c] = re[3];
+    }
+  } else {
+    // Q = the identity
+    const int r = 2 * P;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      b[u] = JT<R>::mk(r + (u >> 1) == ((u & 1) ? 16 + c : c) ? (R)1 : (R)0,
+                       (R)0);
+  }
+  if (tid == 0) {
+    sh.off = 0;
+    sh.big = 0;
+    sh.rot = 0;
+  }
+  __syncthreads();
+  // Is there a cross pair to rotate (the sweep reduces no others), and does
+  // any pair lie above conv2 (the problem needs another sweep)?
+  if (is_g) {
+    const R a0 = sh.dg[P], a1 = sh.dg[c], d0 = sh.dg[16 + P],
+            d1 = sh.dg[16 + c];
+    const R n0 = b[0].x * b[0].x + b[0].y * b[0].y,
+            n1 = b[1].x * b[1].x + b[1].y * b[1].y,
+            n3 = b[3].x * b[3].x + b[3].y * b[3].y;
+    const R c2 = (R)conv2;
+    bool big = false, off = false;
+    if (pair_open<R>(a0, d1, zt)) {
+      const R sc = pair_scale<R>(a0, d1, zt);
+      off = n1 > tol2 * sc;
+      big = n1 > c2 * sc;
+    }
+    if (P != c) {
+      big = big || (pair_open<R>(a0, a1, zt) &&
+                    n0 > c2 * pair_scale<R>(a0, a1, zt));
+      big = big || (pair_open<R>(d0, d1, zt) &&
+                    n3 > c2 * pair_scale<R>(d0, d1, zt));
+    }
+    if (off) sh.off = 1;
+    if (big) sh.big = 1;
+  }
+  __syncthreads();
+  // the sweep's end only asks whether the maximum exceeds conv2
+  if (tid == 0 && sh.big)
+    atomicMax((unsigned long long*)&offmax[bz],
+              (unsigned long long)__double_as_longlong(1.0));
+  if (!sh.off) {
+    if (tid == 0) flags[bz * p + pi] = 0;
+    return;
+  }
+  int rot = 0;
+  for (int sweep = 0; sweep < n_inner; ++sweep) {
+    rot += cross_rounds<R>(sh, b, is_g, P, c, zt, tol2);
+    if (n_inner > 1) {
+      // the rows still on the move, for the next sweep
+      __syncthreads();
+      if (is_g) {
+        const int from = ((P + 1) & 15) * 16 + c;
+        b[2] = sh.exch[1][0][from];
+        b[3] = sh.exch[1][1][from];
+      }
+      __syncthreads();
+    }
+  }
+  if (rot) atomicAdd(&sh.rot, rot);
+  __syncthreads();
+  const int total = sh.rot;
+  if (tid == 0) {
+    flags[bz * p + pi] = total > 0 ? 1 : 0;
+    if (total > 0) {
+      atomicAdd(&counters[bz], total);
+      atomicAdd(qpairs, 1);
+      // rotated pairs whose W columns the update launch also rotates
+      if (w_mode == 1 || (w_mode == 2 && want[bz])) atomicAdd(qpairs + 1, 1);
+    }
+  }
+  if (total == 0 || is_g) return;
+  c_t* q = Qout + ((int64_t)bz * p + pi) * (int64_t)(W * W) + 2 * P * W;
+  q[c] = b[0];
+  q[16 + c] = b[1];
+  q[W + c] = b[2];
+  q[W + 16 + c] = b[3];
 }
 
 // ---------------------------------------------------------------------------
@@ -935,7 +1174,7 @@ __global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
     const int idx = tid + kWholeThreads * i;
-    const int r = idx % W, c = idx / W;
+    const int r = idx / W, c = idx % W;
     c_t v = JT<R>::mk(r == c ? (R)1 : (R)0, (R)0);
     if (r < 2 * np && c < 2 * np)
       v = Qp[narrow ? qpos_n<16>(r, c, np) : qpos_n<32>(r, c, np)];
@@ -991,8 +1230,8 @@ __global__ __launch_bounds__(256) void jac_update(
     Xi[c][r] = v.y;
   }
   for (int idx = tid; idx < W * W; idx += 256) {
-    const int r = idx % W, c = idx / W;
-    const c_t qv = Qp[idx];  // Q[r][c] col-major
+    const int r = idx / W, c = idx % W;
+    const c_t qv = Qp[idx];  // Q[r][c], row by row
     Qr[r][c] = qv.x;
     Qi[r][c] = qv.y;
   }
@@ -1980,7 +2219,8 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
 template <typename R, int WW>
 int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
                                    int64_t sX, void* Wv, int64_t sW, int r,
-                                   double tol, int n_inner, int nchunk_x,
+                                   double tol, double conv2, int n_inner,
+                                   int nchunk_x,
                                    int nchunk_w, bool per_problem_w) {
   using c_t = typename JT<R>::c_t;
   c_t* X = (c_t*)Xv;
@@ -2039,6 +2279,12 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
                        kWholeThreads, (const c_t*)G, npart, tol, tol, zthr,
                        n_inner, Qc, flags, counters, active, offmax, misc + 2,
                        (const int*)want_w, Wm ? (per_problem_w ? 2 : 1) : 0);
+  } else if (WW == 32 && cross_rounds && p > 1 && r > 0) {
+    QTN_TIMED_LAUNCH_N(ev[2], ev[3], (jac_inner_cross<R>), dim3(p, batch),
+                       kCrossThreads, (const c_t*)G, npart, p, tol, conv2,
+                       zthr, n_inner, Qc, flags, counters, active, offmax,
+                       misc + 2, (const int*)want_w,
+                       Wm ? (per_problem_w ? 2 : 1) : 0);
   } else
   QTN_TIMED_LAUNCH(ev[2], ev[3], (jac_inner<R, WW>), dim3(p, batch),
                    (const c_t*)G, npart, p, tol, zthr, n_inner, Qc, flags,
@@ -2252,11 +2498,11 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     for (int pass = 0; pass < passes; ++pass) {
       for (int r = 0; r < rounds; ++r) {
         if (this->W == 64)
-          QTN_TRY((launch_round<R, 64>(s, X, ldx, sX, Wm, sW, r, tol, n_inner,
+          QTN_TRY((launch_round<R, 64>(s, X, ldx, sX, Wm, sW, r, tol, conv2, n_inner,
                                        nchunk_x, nchunk_w,
                                        want_w_host != nullptr)));
         else
-          QTN_TRY((launch_round<R, 32>(s, X, ldx, sX, Wm, sW, r, tol, n_inner,
+          QTN_TRY((launch_round<R, 32>(s, X, ldx, sX, Wm, sW, r, tol, conv2, n_inner,
                                        nchunk_x, nchunk_w,
                                        want_w_host != nullptr)));
       }

@@ -82,8 +82,9 @@ struct JacobiEngine {
   // values.
   template <typename R, int WW>
   int32_t launch_round(hipStream_t s, void* X, int64_t ldx, int64_t sX,
-                       void* Wm, int64_t sW, int r, double tol, int n_inner,
-                       int nchunk_x, int nchunk_w, bool per_problem_w);
+                       void* Wm, int64_t sW, int r, double tol, double conv2,
+                       int n_inner, int nchunk_x, int nchunk_w,
+                       bool per_problem_w);
   template <typename R>
   int32_t run_t(qtn_ctx* ctx, typename CType<R>::type* X, int64_t ldx,
                 int64_t sX, typename CType<R>::type* Wm, int64_t sW,
