@@ -417,12 +417,12 @@ __global__ __launch_bounds__(256) void left_finish(
 //   E_ij = (S_ij + lambda_j R_ij) / (lambda_j - lambda_i),  E_jj = R_jj / 2,
 //   V_k <- V_k + V E_k.
 // Only the kept columns of S, R and E are formed.  Pairs too close for the
-// first order (|E_ij| above kRefineMax, where its square would outlast the
-// two Newton-Schulz steps that follow) only have their inner product removed,
-// E_ij = R_ij / 2.
+// first order (|E_ij| above kRefineMax) only have their inner product
+// removed, E_ij = R_ij / 2; Newton-Schulz steps then take the second order
+// out of V^H V.
 // Measured on the 40-qubit depth-20 chi-256 Haar circuit: amplitudes within
-// 7e-7 of FP64 against 6e-5 to 9e-5 without the step (chi 173: 9e-7), for six
-// products of two-site size per gate in place of a third Newton-Schulz step.
+// 7e-7 of FP64 against 6e-5 to 9e-5 without the step (chi 173: 9e-7), for five
+// products of two-site size per gate.
 constexpr double kRefineMax = 0.02;
 
 // One gate of the refinement.  theta is M x N, V (N x n, ld N) the FP32
@@ -1580,8 +1580,9 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
   for (int g = 0; g < ng; ++g) any_fp32 = any_fp32 || src[g] == 1;
   if (chosen || (learned && any_fp32)) {
     // First-order refinement of the FP32 vectors, then Newton-Schulz in
-    // FP64: V <- V (3 I - V^H V) / 2, two steps take the refinement's second
-    // order (at most kRefineMax^2) below FP64 rounding.
+    // FP64: V <- V (3 I - V^H V) / 2, three steps take the refinement's
+    // second order below FP64 rounding (two left 2e-12 where many kept
+    // values lie near the FP32 floor).
     if (any_fp32)
       QTN_TRY(refine_vk(ctx, ng, gd, src, kept, (const float2*)dX32, x_sz,
                         (const float2*)dW32, w_sz, cols_p, eng32, &refined));
@@ -1609,7 +1610,7 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
     QTN_CHECK_HIP(hipMemcpyAsync(d_gb, gb.data(),
                                  ng * sizeof(GemmDesc<double>),
                                  hipMemcpyHostToDevice, s));
-    for (int it = 0; it < 2; ++it) {
+    for (int it = 0; it < 3; ++it) {
       QTN_TRY(launch_zgemm_grouped(s, 2, 0, d_ga, ng, maxk, maxk));
       QTN_TRY(launch_zgemm_grouped(s, 0, 0, d_gb, ng, maxN, maxk));
       hipLaunchKernelGGL(ns_combine, dim3(grid_for(maxN * maxk), (unsigned)ng),
