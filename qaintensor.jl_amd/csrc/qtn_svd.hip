@@ -793,6 +793,67 @@ __device__ __forceinline__ int cross_rounds(CrossShared<R>& sh,
   return rot;
 }
 
+// Is there a cross pair to rotate (the sweep reduces no others)?  Also
+// records whether any pair lies above conv2 (the problem needs another
+// sweep).  Called by the whole workgroup with sh.dg set and visible.
+template <typename R>
+__device__ __forceinline__ bool cross_check(CrossShared<R>& sh,
+                                            const typename JT<R>::c_t (&b)[4],
+                                            bool is_g, int P, int c, R zt,
+                                            R tol2, R conv2,
+                                            double* offmax_bz) {
+  if (is_g) {
+    const R a0 = sh.dg[P], a1 = sh.dg[c], d0 = sh.dg[16 + P],
+            d1 = sh.dg[16 + c];
+    const R n0 = b[0].x * b[0].x + b[0].y * b[0].y,
+            n1 = b[1].x * b[1].x + b[1].y * b[1].y,
+            n3 = b[3].x * b[3].x + b[3].y * b[3].y;
+    bool big = false, off = false;
+    if (pair_open<R>(a0, d1, zt)) {
+      const R sc = pair_scale<R>(a0, d1, zt);
+      off = n1 > tol2 * sc;
+      big = n1 > conv2 * sc;
+    }
+    if (P != c) {
+      big = big || (pair_open<R>(a0, a1, zt) &&
+                    n0 > conv2 * pair_scale<R>(a0, a1, zt));
+      big = big || (pair_open<R>(d0, d1, zt) &&
+                    n3 > conv2 * pair_scale<R>(d0, d1, zt));
+    }
+    if (off) sh.off = 1;
+    if (big) sh.big = 1;
+  }
+  __syncthreads();
+  // the sweep's end only asks whether the maximum exceeds conv2
+  if (threadIdx.x == 0 && sh.big)
+    atomicMax((unsigned long long*)offmax_bz,
+              (unsigned long long)__double_as_longlong(1.0));
+  return sh.off != 0;
+}
+
+// n_inner sweeps of 16 rounds; returns the rotations this thread derived.
+template <typename R>
+__device__ __forceinline__ int cross_sweeps(CrossShared<R>& sh,
+                                            typename JT<R>::c_t (&b)[4],
+                                            bool is_g, int P, int c, R zt,
+                                            R tol2, int n_inner) {
+  int rot = 0;
+  for (int sweep = 0; sweep < n_inner; ++sweep) {
+    rot += cross_rounds<R>(sh, b, is_g, P, c, zt, tol2);
+    if (sweep + 1 < n_inner) {
+      // the rows still on the move, for the next sweep
+      __syncthreads();
+      if (is_g) {
+        const int from = ((P + 1) & 15) * 16 + c;
+        b[2] = sh.exch[1][0][from];
+        b[3] = sh.exch[1][1][from];
+      }
+      __syncthreads();
+    }
+  }
+  return rot;
+}
+
 // grid (p, batch), kCrossThreads threads; arguments as jac_inner's (Q leaves
 // row by row).
 template <typename R>
@@ -809,7 +870,7 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
   if (!active[bz]) return;
   __shared__ CrossShared<R> sh;
   const int tid = threadIdx.x;
-  const bool is_g = tid < 256;
+  const bool is_g = __builtin_amdgcn_readfirstlane(tid >> 6) < 4;
   const int P = (tid & 255) >> 4, c = tid & 15;
   const R zt = (R)zthr[bz];
   const R tol2 = (R)(tol * tol);
@@ -856,53 +917,11 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
     sh.rot = 0;
   }
   __syncthreads();
-  // Is there a cross pair to rotate (the sweep reduces no others), and does
-  // any pair lie above conv2 (the problem needs another sweep)?
-  if (is_g) {
-    const R a0 = sh.dg[P], a1 = sh.dg[c], d0 = sh.dg[16 + P],
-            d1 = sh.dg[16 + c];
-    const R n0 = b[0].x * b[0].x + b[0].y * b[0].y,
-            n1 = b[1].x * b[1].x + b[1].y * b[1].y,
-            n3 = b[3].x * b[3].x + b[3].y * b[3].y;
-    const R c2 = (R)conv2;
-    bool big = false, off = false;
-    if (pair_open<R>(a0, d1, zt)) {
-      const R sc = pair_scale<R>(a0, d1, zt);
-      off = n1 > tol2 * sc;
-      big = n1 > c2 * sc;
-    }
-    if (P != c) {
-      big = big || (pair_open<R>(a0, a1, zt) &&
-                    n0 > c2 * pair_scale<R>(a0, a1, zt));
-      big = big || (pair_open<R>(d0, d1, zt) &&
-                    n3 > c2 * pair_scale<R>(d0, d1, zt));
-    }
-    if (off) sh.off = 1;
-    if (big) sh.big = 1;
-  }
-  __syncthreads();
-  // the sweep's end only asks whether the maximum exceeds conv2
-  if (tid == 0 && sh.big)
-    atomicMax((unsigned long long*)&offmax[bz],
-              (unsigned long long)__double_as_longlong(1.0));
-  if (!sh.off) {
+  if (!cross_check<R>(sh, b, is_g, P, c, zt, tol2, (R)conv2, &offmax[bz])) {
     if (tid == 0) flags[bz * p + pi] = 0;
     return;
   }
-  int rot = 0;
-  for (int sweep = 0; sweep < n_inner; ++sweep) {
-    rot += cross_rounds<R>(sh, b, is_g, P, c, zt, tol2);
-    if (n_inner > 1) {
-      // the rows still on the move, for the next sweep
-      __syncthreads();
-      if (is_g) {
-        const int from = ((P + 1) & 15) * 16 + c;
-        b[2] = sh.exch[1][0][from];
-        b[3] = sh.exch[1][1][from];
-      }
-      __syncthreads();
-    }
-  }
+  const int rot = cross_sweeps<R>(sh, b, is_g, P, c, zt, tol2, n_inner);
   if (rot) atomicAdd(&sh.rot, rot);
   __syncthreads();
   const int total = sh.rot;
@@ -1795,6 +1814,271 @@ __global__ __launch_bounds__(256) void jac_round_res(
   }
 }
 
+// ---------------------------------------------------------------------------
+// The fused cross round with the block pair in registers (at most 512 rows,
+// W = 32): one workgroup of 512 threads per block pair streams X_IJ twice,
+// both times straight into MFMA operand registers -- once in the Gram's
+// layout (lane l: column l % 16, row 4 s + l / 16), once, behind the 16
+// inner rounds, in the update's (lane l: row l % 16, column 4 s + l / 16) --
+// so neither pass is staged through LDS, and Q X_IJ leaves from the
+// accumulators.  The 16-row tiles go to the eight waves in turn; the Gram's
+// partials meet in LDS.  The diagonal quadrants take three real products
+// (Im = M - M^T, M = Xr^T Xi), the update four.
+// Three launches per round cost a kernel boundary each (about 5 us with
+// several streams busy) and a pass over X more.
+// FP64 at 512 rows, six problems of 16 pairs on each of two streams: 43 us a
+// round against 15 + 20 + 20 us and two boundaries; the two passes of MFMAs
+// (160 and 256 of 64 cycles per wave, two waves a SIMD) are 22 us of it.
+//
+// NT: 16-row tiles per wave, for up to 128 NT rows.  A tile a wave does not
+// have is read as the last one and not used, so that the loads are a straight
+// run and the products wait for their own tile only.
+
+// Y = X Q for the tiles of this wave, in place: rows x 32 columns (blocks I
+// and J) of X; x holds the tiles' columns in the update's layout.
+template <typename R, int NT>
+__device__ __forceinline__ void reg_load(
+    const typename JT<R>::c_t* __restrict__ X, int64_t ldx, int ntiles, int I,
+    int J, int wave, typename JT<R>::c_t (&x)[NT][8]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    const int r0 = 16 * min(wave + 8 * i, ntiles - 1) + (lane & 15);
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      x[i][s] = X[r0 + pair_col<32>(4 * s + (lane >> 4), I, J) * ldx];
+  }
+}
+template <typename R, int NT>
+__device__ __forceinline__ void reg_update(
+    typename JT<R>::c_t* __restrict__ X, int64_t ldx, int ntiles, int I,
+    int J, int wave, const typename JT<R>::c_t (&x)[NT][8],
+    const R (*Qr)[33], const R (*Qi)[33]) {
+  using acc_t = typename JT<R>::acc_t;
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    if (wave + 8 * i >= ntiles) break;
+    acc_t yr[2], yi[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) yr[j][e] = yi[j][e] = (R)0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int k = 4 * s + (lane >> 4);
+      const R xr = x[i][s].x, xi = x[i][s].y;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const R qr = Qr[k][16 * j + (lane & 15)],
+                qi = Qi[k][16 * j + (lane & 15)];
+        yr[j] = JT<R>::mfma(qr, xr, yr[j]);
+        yr[j] = JT<R>::mfma(qi, -xi, yr[j]);
+        yi[j] = JT<R>::mfma(qi, xr, yi[j]);
+        yi[j] = JT<R>::mfma(qr, xi, yi[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        X[16 * (wave + 8 * i) + (lane & 15) +
+          pair_col<32>(16 * j + JT<R>::row(lane, e), I, J) * ldx] =
+            JT<R>::mk(yr[j][e], yi[j][e]);
+  }
+}
+
+template <typename R>
+struct RegShared {
+  CrossShared<R> cross;
+  union {
+    R part[4][24][64];  // partial Grams of four waves
+    struct {
+      R sum[24][64];    // their sum
+      R Qr[32][33], Qi[32][33];
+    } s;
+  };
+};
+
+template <typename R, int NT>
+__global__ __launch_bounds__(kCrossThreads)
+__attribute__((amdgpu_waves_per_eu(sizeof(R) * NT <= 8 ? 4 : 2)))
+void jac_round_reg(
+    typename JT<R>::c_t* __restrict__ X, int64_t ldx, int64_t sX,
+    int nchunk_x, typename JT<R>::c_t* __restrict__ Wm, int64_t ldw,
+    int64_t sW, int nchunk_w, const int* __restrict__ want, int p, int round,
+    double tol, double conv2, const double* __restrict__ zthr, int n_inner,
+    int* __restrict__ counters, const int* __restrict__ active,
+    double* __restrict__ offmax, int* __restrict__ qpairs) {
+  using c_t = typename JT<R>::c_t;
+  using acc_t = typename JT<R>::acc_t;
+  const int bz = blockIdx.y, pi = blockIdx.x;
+  if (!active[bz]) return;
+  const int nb = 2 * p;
+  const int b1 = rr_block(pi, round, nb);
+  const int b2 = rr_block(nb - 1 - pi, round, nb);
+  const int I = min(b1, b2), J = max(b1, b2);
+  X += (int64_t)bz * sX;
+  __shared__ RegShared<R> sh;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ntiles = 4 * nchunk_x;
+
+  // 1. Gram of the wave's tiles
+  {
+    c_t v[NT][4][2];
+    const c_t* c0 = X + pair_col<32>(lane & 15, I, J) * ldx + (lane >> 4);
+    const c_t* c1 = X + pair_col<32>(16 + (lane & 15), I, J) * ldx +
+                    (lane >> 4);
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int r0 = 16 * min(wave + 8 * i, ntiles - 1);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        v[i][s][0] = c0[r0 + 4 * s];
+        v[i][s][1] = c1[r0 + 4 * s];
+      }
+    }
+    acc_t g[3][2];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) g[q][0][e] = g[q][1][e] = (R)0;
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      if (wave + 8 * i >= ntiles) break;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const R xr = v[i][s][q].x, xi = v[i][s][q].y;
+          g[q][0] = JT<R>::mfma(xr, xr, g[q][0]);
+          g[q][0] = JT<R>::mfma(xi, xi, g[q][0]);
+          g[q][1] = JT<R>::mfma(xr, xi, g[q][1]);
+        }
+        const R ar = v[i][s][0].x, ai = v[i][s][0].y;
+        const R br = v[i][s][1].x, bi = v[i][s][1].y;
+        g[2][0] = JT<R>::mfma(ar, br, g[2][0]);
+        g[2][0] = JT<R>::mfma(ai, bi, g[2][0]);
+        g[2][1] = JT<R>::mfma(ar, bi, g[2][1]);
+        g[2][1] = JT<R>::mfma(-ai, br, g[2][1]);
+      }
+    }
+    // waves 4-7 hand theirs to waves 0-3
+    if (wave >= 4) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            sh.part[wave - 4][(q * 2 + h) * 4 + e][lane] = g[q][h][e];
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            R& at = sh.part[wave][(q * 2 + h) * 4 + e][lane];
+            at = g[q][h][e] + at;
+          }
+    }
+  }
+  __syncthreads();
+  // the four sums, added in order
+  R sum[3];
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    const int idx = tid + 512 * u;
+    sum[u] = sh.part[0][idx >> 6][idx & 63];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) sum[u] += sh.part[w][idx >> 6][idx & 63];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < 3; ++u) {
+    const int idx = tid + 512 * u;
+    sh.s.sum[idx >> 6][idx & 63] = sum[u];
+  }
+  if (tid == 0) {
+    sh.cross.off = 0;
+    sh.cross.big = 0;
+    sh.cross.rot = 0;
+  }
+  __syncthreads();
+
+  // 2. the inner rounds (jac_inner_cross)
+  const bool is_g = wave < 4;
+  const int P = (tid & 255) >> 4, c = tid & 15;
+  const R zt = (R)zthr[bz];
+  const R tol2 = (R)(tol * tol);
+  c_t b[4];
+  if (is_g) {
+    // entry (r, n) of quadrant q, half h: the lane and element holding it
+    auto at = [&](int q, int h, int r, int n) {
+      const int e = sizeof(R) == 8 ? r >> 2 : r & 3;
+      const int l = 16 * (sizeof(R) == 8 ? r & 3 : r >> 2) + n;
+      return sh.s.sum[(q * 2 + h) * 4 + e][l];
+    };
+    b[0] = JT<R>::mk(at(0, 0, P, c), at(0, 1, P, c) - at(0, 1, c, P));
+    b[1] = JT<R>::mk(at(2, 0, P, c), at(2, 1, P, c));
+    b[2] = JT<R>::mk(at(2, 0, c, P), -at(2, 1, c, P));
+    b[3] = JT<R>::mk(at(1, 0, P, c), at(1, 1, P, c) - at(1, 1, c, P));
+    if (P == c) {
+      sh.cross.dg[c] = b[0].x;
+      sh.cross.dg[16 + c] = b[3].x;
+    }
+  } else {
+    const int r = 2 * P;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      b[u] = JT<R>::mk(r + (u >> 1) == ((u & 1) ? 16 + c : c) ? (R)1 : (R)0,
+                       (R)0);
+  }
+  __syncthreads();
+  if (!cross_check<R>(sh.cross, b, is_g, P, c, zt, tol2, (R)conv2,
+                      &offmax[bz]))
+    return;
+  // X_IJ again, in the update's layout: behind the rounds where one
+  // workgroup fills the CU's registers, after them where two do (each hides
+  // the other's load)
+  constexpr bool kEarly = sizeof(R) * NT > 8;
+  c_t x[NT][8];
+  if constexpr (kEarly) reg_load<R, NT>(X, ldx, ntiles, I, J, wave, x);
+  const int rot = cross_sweeps<R>(sh.cross, b, is_g, P, c, zt, tol2, n_inner);
+  if (rot) atomicAdd(&sh.cross.rot, rot);
+  if (!is_g) {
+    const int r = 2 * P;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int col = (u & 1) ? 16 + c : c;
+      sh.s.Qr[r + (u >> 1)][col] = b[u].x;
+      sh.s.Qi[r + (u >> 1)][col] = b[u].y;
+    }
+  }
+  __syncthreads();
+  const int total = sh.cross.rot;
+  if (total == 0) return;
+  const bool do_w = Wm && (!want || want[bz]);
+  if (tid == 0) {
+    atomicAdd(&counters[bz], total);
+    atomicAdd(qpairs, 1);
+    if (do_w) atomicAdd(qpairs + 1, 1);
+  }
+  // 3. X_IJ <- X_IJ Q (and W_IJ <- W_IJ Q)
+  if constexpr (!kEarly) reg_load<R, NT>(X, ldx, ntiles, I, J, wave, x);
+  reg_update<R, NT>(X, ldx, ntiles, I, J, wave, x, sh.s.Qr, sh.s.Qi);
+  if (do_w) {
+    c_t* Wb = Wm + (int64_t)bz * sW;
+    reg_load<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x);
+    reg_update<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x, sh.s.Qr,
+                      sh.s.Qi);
+  }
+}
+
 // After a sweep: a problem stays active only if it rotated something and
 // the largest scaled off-diagonal |x_p^H x_q|^2 / (|x_p|^2 |x_q|^2) met in
 // the sweep was above conv2.  Below it the sweep's own rotations leave the
@@ -2140,7 +2424,17 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
     fused = it->second == QTN_TILING_W32_FUSED;
   }
   if (const char* e = getenv("QTN_JACOBI_W")) wdef = atoi(e) == 64 ? 64 : 32;
-  if (const char* e = getenv("QTN_JACOBI_FUSED")) fused = atoi(e) != 0;
+  // Cross rounds of at most 512 rows keep the block pair in registers unless
+  // a fused tiling was tuned in or QTN_JACOBI_FUSED forces either of the
+  // others.  Against three launches a round: the 40-qubit chi-256 circuit
+  // 370 -> 292 ms in FP64 and 253 -> 238 ms in the chosen form (its FP32
+  // rounds against jac_round_res), 24 uneven circuits 340 -> 302 ms, single
+  // problems of 256 rows even.
+  reg = it == ctx->jac_tiling.end() || !fused;
+  if (const char* e = getenv("QTN_JACOBI_FUSED")) {
+    fused = atoi(e) != 0;
+    reg = false;
+  }
   // Outer rounds 1.. of a sweep rotate only the cross pairs of their two
   // column blocks (16 inner rounds instead of 31 at W = 32); round 0, where
   // every block appears once, also rotates the pairs inside the blocks, so
@@ -2253,6 +2547,28 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
   } while (0)
 #define QTN_TIMED_LAUNCH(e0, e1, kern, grid, ...) \
   QTN_TIMED_LAUNCH_N(e0, e1, kern, grid, 256, __VA_ARGS__)
+  const bool one_launch = WW == 32 && reg_round(nchunk_x, Wm ? nchunk_w : 0, r);
+  if (ctx_ && ctx_->prof) prof_reg.push_back(one_launch ? 1 : 0);
+  if (one_launch) {
+    const int nt = (std::max(nchunk_x, Wm ? nchunk_w : 0) + 1) / 2;
+#define QTN_REG_ROUND(NT)                                                   \
+  QTN_TIMED_LAUNCH_N(ev[0], ev[1], (jac_round_reg<R, NT>), dim3(p, batch),  \
+                     kCrossThreads, X, ldx, sX, nchunk_x, Wm,               \
+                     ldw ? ldw : cols_p, sW, nchunk_w,                      \
+                     (const int*)(per_problem_w ? want_w : nullptr), p, r,  \
+                     tol, conv2, zthr, n_inner, counters, active, offmax,   \
+                     misc + 2)
+    if (nt <= 1)
+      QTN_REG_ROUND(1);
+    else if (nt == 2)
+      QTN_REG_ROUND(2);
+    else if (nt == 3)
+      QTN_REG_ROUND(3);
+    else
+      QTN_REG_ROUND(4);
+#undef QTN_REG_ROUND
+    return QTN_OK;
+  }
   if (fused && WW == 32) {
     if constexpr (std::is_same<R, float>::value) {
       if (res_round(nchunk_x, Wm ? nchunk_w : 0)) {
@@ -2313,39 +2629,11 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
 int32_t JacobiEngine::account_sweep(int n_active, int qpairs, int qpairs_w,
                                     int nchunk, int nchunk_w) {
   qtn_ctx* ctx = ctx_;
-  if (fused && W == 32) {
-    // jac_round (id 3 FP64, 7 FP32): the Gram of every active pair plus
-    // X_IJ <- X_IJ Q for every rotated pair; bytes: X_IJ read once for the
-    // Gram, read and written once more for the update.  jac_round_res reads X_IJ once and
-    // writes it once, and reads and writes W_IJ once for the pairs that
-    // rotate W.
-    const double Wd = W, c16 = single ? 8.0 : 16.0;
-    const double rows = (double)nchunk * 64.0;
-    const bool res = res_round(nchunk, nchunk_w);
-    const int kr = single ? 7 : 3;
-    for (size_t i = 0; i + 5 < prof_events.size(); i += 6) {
-      float t01;
-      QTN_CHECK_HIP(hipEventElapsedTime(&t01, prof_events[i],
-                                        prof_events[i + 1]));
-      ctx->prof_count[kr] += 1;
-      ctx->prof_ms[kr] += t01;
-      ctx->prof_flops[kr] += (double)n_active * p * 0.75 * 8.0 * rows * Wd * Wd;
-      ctx->prof_bytes[kr] += (double)n_active * p * rows * Wd * c16;
-    }
-    ctx->prof_flops[kr] += (double)qpairs * 8.0 * rows * Wd * Wd;
-    ctx->prof_bytes[kr] += (double)qpairs * (res ? 1.0 : 2.0) * rows * Wd * c16;
-    if (res) {
-      const double wrows = (double)nchunk_w * 64.0;
-      ctx->prof_flops[kr] += (double)qpairs_w * 8.0 * wrows * Wd * Wd;
-      ctx->prof_bytes[kr] += (double)qpairs_w * 2.0 * wrows * Wd * c16;
-    }
-    for (auto e : prof_events) ctx->ev_pool.push_back(e);
-    prof_events.clear();
-    return QTN_OK;
-  }
   const double Wd = W, c16 = single ? 8.0 : 16.0;
-  const double rounds = 2.0 * p - 1.0;
-  const int ki = single ? 4 : 0, kg = single ? 5 : 1, ku = single ? 6 : 2;
+  const double rows = (double)nchunk * 64.0, wrows = (double)nchunk_w * 64.0;
+  const int ki = single ? 4 : 0, kg = single ? 5 : 1, ku = single ? 6 : 2,
+            kr = single ? 7 : 3;
+  const bool res = res_round(nchunk, nchunk_w);
   // jac_gram reads each 64-row chunk of X_IJ and writes one partial Gram
   // per workgroup (npart of them); jac_inner reads those partials
   const double npart = gram_parts(nchunk);
@@ -2355,32 +2643,54 @@ int32_t JacobiEngine::account_sweep(int n_active, int qpairs, int qpairs_w,
   const double inner_b = (npart * 0.75 * Wd * Wd + Wd * Wd) * c16;
   const double upd_f = 8.0 * 64.0 * Wd * Wd;
   const double upd_b = (2.0 * 64.0 * Wd + Wd * Wd) * c16;
-  const double pairs_per_launch = (double)n_active * p;
-  // per round: (start, stop) of jac_gram, jac_inner and the update (X and,
-  // when there is one, W in the same launch)
-  for (size_t i = 0; i + 5 < prof_events.size(); i += 6) {
-    float t01, t12, t23;
-    QTN_CHECK_HIP(hipEventElapsedTime(&t01, prof_events[i], prof_events[i + 1]));
-    QTN_CHECK_HIP(hipEventElapsedTime(&t12, prof_events[i + 2], prof_events[i + 3]));
-    QTN_CHECK_HIP(hipEventElapsedTime(&t23, prof_events[i + 4], prof_events[i + 5]));
+  const double pairs = (double)n_active * p;  // per round
+  const size_t nrounds = prof_events.size() / 6;
+  size_t n_one = 0;  // rounds of one launch (jac_round_reg, _res, jac_round)
+  for (size_t i = 0; i < nrounds; ++i) {
+    const hipEvent_t* ev = &prof_events[6 * i];
+    float t;
+    if (prof_reg[i] || (fused && W == 32)) {
+      // the Gram of every active pair; X_IJ read once
+      QTN_CHECK_HIP(hipEventElapsedTime(&t, ev[0], ev[1]));
+      ctx->prof_count[kr] += 1;
+      ctx->prof_ms[kr] += t;
+      ctx->prof_flops[kr] += pairs * 0.75 * 8.0 * rows * Wd * Wd;
+      ctx->prof_bytes[kr] += pairs * rows * Wd * c16;
+      ++n_one;
+      continue;
+    }
+    // (start, stop) of jac_gram, jac_inner and the update (X and, when there
+    // is one, W in the same launch)
+    QTN_CHECK_HIP(hipEventElapsedTime(&t, ev[0], ev[1]));
     ctx->prof_count[kg] += 1;
-    ctx->prof_ms[kg] += t01;
-    ctx->prof_flops[kg] += pairs_per_launch * nchunk * gram_f;
-    ctx->prof_bytes[kg] += pairs_per_launch * nchunk * gram_b;
+    ctx->prof_ms[kg] += t;
+    ctx->prof_flops[kg] += pairs * nchunk * gram_f;
+    ctx->prof_bytes[kg] += pairs * nchunk * gram_b;
+    QTN_CHECK_HIP(hipEventElapsedTime(&t, ev[2], ev[3]));
     ctx->prof_count[ki] += 1;
-    ctx->prof_ms[ki] += t12;
-    ctx->prof_bytes[ki] += pairs_per_launch * inner_b;
+    ctx->prof_ms[ki] += t;
+    ctx->prof_bytes[ki] += pairs * inner_b;
+    QTN_CHECK_HIP(hipEventElapsedTime(&t, ev[4], ev[5]));
     ctx->prof_count[ku] += 1;
-    ctx->prof_ms[ku] += t23;
+    ctx->prof_ms[ku] += t;
   }
-  // rotated pairs are only known per sweep: spread over its launches
-  ctx->prof_flops[ku] += ((double)qpairs * nchunk +
-                          (double)qpairs_w * nchunk_w) * upd_f;
-  ctx->prof_bytes[ku] += ((double)qpairs * nchunk +
-                          (double)qpairs_w * nchunk_w) * upd_b;
-  (void)rounds;
+  // Rotated pairs are only known per sweep: spread over its rounds.  A
+  // one-launch round writes X_IJ once (the FP64 streaming jac_round reads it
+  // again too) and reads and writes W_IJ.
+  const double f1 = nrounds ? (double)n_one / (double)nrounds : 0.0;
+  const bool streams = fused && W == 32 && !res && !reg;
+  ctx->prof_flops[kr] +=
+      f1 * 8.0 * Wd * Wd * (qpairs * rows + qpairs_w * wrows);
+  ctx->prof_bytes[kr] += f1 * Wd * c16 *
+                         (qpairs * (streams ? 2.0 : 1.0) * rows +
+                          qpairs_w * 2.0 * wrows);
+  ctx->prof_flops[ku] += (1.0 - f1) * upd_f *
+                         ((double)qpairs * nchunk + (double)qpairs_w * nchunk_w);
+  ctx->prof_bytes[ku] += (1.0 - f1) * upd_b *
+                         ((double)qpairs * nchunk + (double)qpairs_w * nchunk_w);
   for (auto e : prof_events) ctx->ev_pool.push_back(e);
   prof_events.clear();
+  prof_reg.clear();
   return QTN_OK;
 }
 
@@ -2459,6 +2769,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   QTN_CHECK_HIP(hipMemsetAsync(misc, 0, 4 * sizeof(int), s));
   ctx_ = ctx;
   prof_events.clear();
+  prof_reg.clear();
   int n_act = batch;
   if (mask_host) {
     n_act = 0;
@@ -2523,7 +2834,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     std::memset(&key, 0, sizeof(key));
     key.dbl = dbl ? 1 : 0;
     key.w = this->W;
-    key.fused = fused ? 1 : 0;
+    key.fused = (fused ? 1 : 0) + (reg ? 2 : 0);
     key.cross = cross_rounds ? 1 : 0;
     key.batch = batch;
     key.p = p;

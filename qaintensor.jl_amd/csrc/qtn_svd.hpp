@@ -30,6 +30,13 @@ struct JacobiEngine {
   bool res_round(int nchunk_x, int nchunk_w) const {
     return single && nchunk_x * 64 <= 512 && nchunk_w * 64 <= 512;
   }
+  // Cross rounds of problems of at most 512 rows run as one launch with the
+  // block pair in registers (jac_round_reg)
+  bool reg_round(int nchunk_x, int nchunk_w, int r) const {
+    return reg && cross_rounds && p > 1 && r > 0 && nchunk_x * 64 <= 512 &&
+           nchunk_w * 64 <= 512;
+  }
+  bool reg = false;
   // the inner sweeps of outer rounds 1.. rotate only the cross pairs of
   // their two column blocks (round 0 of every outer sweep rotates all)
   bool cross_rounds = false;
@@ -65,6 +72,7 @@ struct JacobiEngine {
   double* sig = nullptr;  // [batch][cols_p], sorted descending after run
   qtn_ctx* ctx_ = nullptr;
   std::vector<hipEvent_t> prof_events;  // 6 per round while profiling
+  std::vector<char> prof_reg;           // rounds that were one jac_round_reg
   int32_t account_sweep(int n_active, int qpairs, int qpairs_w, int nchunk,
                         int nchunk_w);
   int* perm = nullptr;    // [batch][cols_p], column of X for each sigma
