@@ -156,23 +156,95 @@ __device__ __forceinline__ void block_sum_fast(double2 (&part)[N],
   __syncthreads();
 }
 
-// Factor panel k of every active problem (one workgroup of NT threads per
-// problem).  Writes the reflectors below the diagonal of A, R on and above
-// it, the explicit V (rows x NB, unit diagonal, zeros above) into Vb, V T^H
-// into VTh and V T into VTn (both rows x NB), all with ld = lda.
-// kLds: the panel (rows - r0 <= kLdsRows rows x NB) is held in LDS;
-// otherwise it is updated in place in A (the workgroup's own stores are
-// visible to it after each barrier).  Per column one norm reduction and one
-// 16-wide reduction that yields both w_c = v_j^H x_c (c > j, for the
-// reflector application) and Gv[i][j] = v_i^H v_j (i < j, for T).
+// Sum of 32 values per lane over a wave, scattered: lane l returns the sum
+// of value l / 2.  Each step halves the values a lane still carries (swaps
+// of half-waves and of rows of 16, then DPP within the rows), 32 additions
+// where 32 butterflies take 192.
+__device__ __forceinline__ double dpp_move(double x, int ctrl_id) {
+  const int2 v = __builtin_bit_cast(int2, x);
+  int2 r;
+  switch (ctrl_id) {
+    case 0:  // row_ror:8
+      r = make_int2(
+          __builtin_amdgcn_update_dpp(v.x, v.x, 0x128, 0xf, 0xf, false),
+          __builtin_amdgcn_update_dpp(v.y, v.y, 0x128, 0xf, 0xf, false));
+      break;
+    case 1:  // row_half_mirror
+      r = make_int2(
+          __builtin_amdgcn_update_dpp(v.x, v.x, 0x141, 0xf, 0xf, false),
+          __builtin_amdgcn_update_dpp(v.y, v.y, 0x141, 0xf, 0xf, false));
+      break;
+    case 2:  // quad_perm [2,3,0,1]
+      r = make_int2(
+          __builtin_amdgcn_update_dpp(v.x, v.x, 0x4e, 0xf, 0xf, false),
+          __builtin_amdgcn_update_dpp(v.y, v.y, 0x4e, 0xf, 0xf, false));
+      break;
+    default:  // quad_perm [1,0,3,2]
+      r = make_int2(
+          __builtin_amdgcn_update_dpp(v.x, v.x, 0xb1, 0xf, 0xf, false),
+          __builtin_amdgcn_update_dpp(v.y, v.y, 0xb1, 0xf, 0xf, false));
+  }
+  return __builtin_bit_cast(double, r);
+}
+template <bool k32>
+__device__ __forceinline__ double swap_add(double a, double b) {
+  const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+  uint2 p, q;
+  if constexpr (k32) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+    p = make_uint2(lo[0], hi[0]);
+    q = make_uint2(lo[1], hi[1]);
+  } else {
+    const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+    p = make_uint2(lo[0], hi[0]);
+    q = make_uint2(lo[1], hi[1]);
+  }
+  return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
+}
+__device__ __forceinline__ double wave_sum32(double (&v)[32]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int k = 0; k < 16; ++k) v[k] = swap_add<true>(v[k], v[k + 16]);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v[k] = swap_add<false>(v[k], v[k + 8]);
+  const bool b3 = lane & 8, b2 = lane & 4, b1 = lane & 2;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    v[k] = (b3 ? v[k + 4] : v[k]) + dpp_move(b3 ? v[k] : v[k + 4], 0);
+#pragma unroll
+  for (int k = 0; k < 2; ++k)
+    v[k] = (b2 ? v[k + 2] : v[k]) + dpp_move(b2 ? v[k] : v[k + 2], 1);
+  const double t = (b1 ? v[1] : v[0]) + dpp_move(b1 ? v[0] : v[1], 2);
+  return t + dpp_move(t, 3);
+}
+
+// Factor panel k of every active problem (one workgroup of 256 threads per
+// problem; at most 256 NR rows).  Writes the reflectors below the diagonal
+// of A, R on and above it, the explicit V (rows x NB, unit diagonal, zeros
+// above) into Vb, V T^H into VTh and V T into VTn (both rows x NB), all with
+// ld = lda.
+//
+// Bound by the chain of its NB columns.  Thread t keeps rows t and t + 256 of
+// the panel in registers, the current column first (the columns move down one
+// place per step).  With v = [1; scl x], one reduction gives x^H x_c for the
+// column's norm and every later column at once, w_c = x_c[j] + conj(scl)
+// x^H x_c, so a column costs one barrier.  V waits in LDS for V^H V (MFMA),
+// from which T follows a row per thread (zlarft), and V T.
+// A panel of 257 to 512 rows takes 49 us, one of up to 256 rows 38 us (189 us
+// with the panel in LDS, a norm reduction and a 16-wide butterfly reduction
+// per column).
 constexpr int kLdsRows = 512;
-template <bool kLds, int NT>
-__global__ __launch_bounds__(NT) void qr_panel_t(
+typedef double qr_d4 __attribute__((ext_vector_type(4)));
+
+template <int NR>
+__global__ __launch_bounds__(256) void qr_panel_reg(
     double2* __restrict__ A, int64_t lda, int64_t sA, int k,
     const QrDims* __restrict__ dims, double2* __restrict__ Vb,
     double2* __restrict__ VTh, double2* __restrict__ VTn, int64_t sV,
     int64_t sVh, int write_vtn) {
-  constexpr int NW = NT / 64;
+  constexpr int ROWS = 256 * NR;
   const int bz = blockIdx.x;
   const QrDims d = dims[bz];
   const int64_t r0 = (int64_t)k * NB;
@@ -183,41 +255,59 @@ __global__ __launch_bounds__(NT) void qr_panel_t(
   Vb += (int64_t)bz * sV;
   VTh += (int64_t)bz * sVh;
   VTn += (int64_t)bz * sV;
-  const int tid = threadIdx.x;
-  __shared__ double2 P[kLds ? NB : 1][kLds ? kLdsRows + 1 : 1];
-  __shared__ double2 scratch[NW * NB];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  __shared__ double2 P[NB][ROWS + 1];  // explicit V
+  __shared__ double2 red[2][4][NB];    // the waves' sums of x^H x_c
+  __shared__ double2 diag[2][NB];      // row j of the remaining columns
+  __shared__ double2 fb[4][NB];        // conj(tau) w_c, per wave
   __shared__ double2 tau_s[NB];
-  __shared__ double2 T[NB][NB + 1];
-  __shared__ double2 Gv[NB][NB + 1];
-  // panel entry (column c, panel row r)
-  auto at = [&](int c, int r) -> double2& {
-    if constexpr (kLds)
-      return P[c][r];
-    else
-      return A[r + (int64_t)c * lda];
-  };
-  if constexpr (kLds) {
-    for (int idx = tid; idx < NB * rows; idx += NT) {
-      const int r = idx % rows, c = idx / rows;
-      P[c][r] = c < ncp ? A[r + (int64_t)c * lda] : make_double2(0.0, 0.0);
+  __shared__ double2 Gv[NB][NB];
+  __shared__ double2 T[NB][NB];
+  __shared__ double2 gp[4][256];
+  double2 x[NR][NB];
+#pragma unroll
+  for (int c = 0; c < NB; ++c)
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int r = tid + 256 * i;
+      x[i][c] = (c < ncp && r < rows) ? A[r + (int64_t)c * lda]
+                                      : make_double2(0.0, 0.0);
     }
-  }
-  if (tid < NB)
-    for (int c = 0; c < NB; ++c) {
-      Gv[tid][c] = make_double2(0.0, 0.0);
-      T[tid][c] = make_double2(0.0, 0.0);
-    }
-  __syncthreads();
   for (int j = 0; j < ncp; ++j) {
-    double2 part[1] = {make_double2(0.0, 0.0)};
-    for (int r = j + 1 + tid; r < rows; r += NT) {
-      const double2 v = at(j, r);
-      part[0].x += v.x * v.x + v.y * v.y;
+    const int par = j & 1;
+    double v[32];
+#pragma unroll
+    for (int c = 0; c < 32; ++c) v[c] = 0.0;
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      double2 y = x[i][0];
+      if (i == 0 && tid <= j) y = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int c = 0; c < NB; ++c) {
+        v[2 * c] = fma(y.x, x[i][c].x, v[2 * c]);
+        v[2 * c] = fma(y.y, x[i][c].y, v[2 * c]);
+        v[2 * c + 1] = fma(y.x, x[i][c].y, v[2 * c + 1]);
+        v[2 * c + 1] = fma(-y.y, x[i][c].x, v[2 * c + 1]);
+      }
     }
-    double2 tot[1];
-    block_sum_fast<1, NW>(part, tot, scratch);
-    const double xn2 = tot[0].x;
-    const double2 alpha = at(j, j);
+    const double sum = wave_sum32(v);
+    if ((lane & 1) == 0)
+      reinterpret_cast<double*>(&red[par][wave][0])[lane >> 1] = sum;
+    if (tid == j) {
+#pragma unroll
+      for (int c = 0; c < NB; ++c) diag[par][c] = x[0][c];
+    }
+    __syncthreads();
+    const int cl = lane & (NB - 1);
+    double2 sc = red[par][0][cl];
+    double xn2 = red[par][0][0].x;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      sc.x += red[par][w][cl].x;
+      sc.y += red[par][w][cl].y;
+      xn2 += red[par][w][0].x;
+    }
+    const double2 alpha = diag[par][0];
     double2 tau, scl;
     double beta;
     if (xn2 == 0.0 && alpha.y == 0.0) {
@@ -233,115 +323,144 @@ __global__ __launch_bounds__(NT) void qr_panel_t(
       scl = make_double2(den.x / dd, -den.y / dd);
     }
     if (tid == 0) tau_s[j] = tau;
-    for (int r = j + 1 + tid; r < rows; r += NT) at(j, r) = cmul(at(j, r), scl);
-    __syncthreads();
-    if (tid == 0) at(j, j) = make_double2(beta, 0.0);
-    // c > j: w_c = v_j^H x_c ; c < j: g_c = v_c^H v_j (v_c lives in column
-    // c below its diagonal, and v_j is zero above row j)
-    double2 wp[NB], w[NB];
+    {
+      const double2 xc = diag[par][cl];
+      const double2 t = cmulc(scl, sc);
+      const double2 w = make_double2(xc.x + t.x, xc.y + t.y);
+      if (lane < NB) fb[wave][lane] = cmulc(tau, w);
+    }
+    __builtin_amdgcn_wave_barrier();
+    double2 vr[NR];
 #pragma unroll
-    for (int c = 0; c < NB; ++c) wp[c] = make_double2(0.0, 0.0);
-    for (int r = j + tid; r < rows; r += NT) {
-      const double2 v = (r == j) ? make_double2(1.0, 0.0) : at(j, r);
+    for (int i = 0; i < NR; ++i) {
+      const int r = tid + 256 * i;
+      vr[i] = r > j ? cmul(x[i][0], scl)
+                    : make_double2(r == j ? 1.0 : 0.0, 0.0);
+      P[j][r] = vr[i];
+      if (r > j && r < rows) A[r + (int64_t)j * lda] = vr[i];
+      if (r == j && r < rows)
+        A[j + (int64_t)j * lda] = make_double2(beta, 0.0);
+    }
 #pragma unroll
-      for (int c = 0; c < NB; ++c) {
-        if (c > j && c < ncp) {
-          const double2 pr = cmulc(v, at(c, r));
-          wp[c].x += pr.x;
-          wp[c].y += pr.y;
-        } else if (c < j) {
-          const double2 pr = cmulc(at(c, r), v);
-          wp[c].x += pr.x;
-          wp[c].y += pr.y;
-        }
+    for (int c = 1; c < NB; ++c) {
+      const double2 f = fb[wave][c];
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const double2 u = cmul(vr[i], f);
+        x[i][c - 1] = make_double2(x[i][c].x - u.x, x[i][c].y - u.y);
       }
     }
-    block_sum_fast<NB, NW>(wp, w, scratch);
-    if (tid < j) {
-      double2 g = make_double2(0.0, 0.0);
+    if (tid == j && j < rows) {
+      // row j of R (the columns have moved down one place)
 #pragma unroll
-      for (int c = 0; c < NB; ++c)
-        if (c == tid) g = w[c];
-      Gv[tid][j] = g;
+      for (int c = 1; c < NB; ++c)
+        if (j + c < ncp) A[j + (int64_t)(j + c) * lda] = x[0][c - 1];
     }
-    if (tau.x != 0.0 || tau.y != 0.0) {
-      for (int r = j + tid; r < rows; r += NT) {
-        const double2 v = (r == j) ? make_double2(1.0, 0.0) : at(j, r);
 #pragma unroll
-        for (int c = 0; c < NB; ++c)
-          if (c > j && c < ncp) {
-            const double2 u = cmul(v, cmulc(tau, w[c]));
-            double2& x = at(c, r);
-            x.x -= u.x;
-            x.y -= u.y;
-          }
-      }
-    }
-    __syncthreads();
+    for (int i = 0; i < NR; ++i) x[i][NB - 1] = make_double2(0.0, 0.0);
   }
-  if constexpr (kLds) {
-    // write R / reflectors back
-    for (int idx = tid; idx < NB * rows; idx += NT) {
-      const int r = idx % rows, c = idx / rows;
-      if (c < ncp) A[r + (int64_t)c * lda] = P[c][r];
-    }
-  }
-  // T (zlarft): column j = -tau_j T[0:j,0:j] Gv[0:j, j], T[j][j] = tau_j.
-  // Row tid of column j only needs T[tid][l] for tid <= l < j.  Barriers
-  // are unconditional: every thread takes both of them each step.
-  for (int j = 0; j < ncp; ++j) {
-    double2 q = make_double2(0.0, 0.0);
-    const double2 tj = tau_s[j];
-    if (tid < j) {
-      double2 acc = make_double2(0.0, 0.0);
+  for (int j = ncp; j < NB; ++j) {
 #pragma unroll
-      for (int l = 0; l < NB; ++l)
-        if (l >= tid && l < j) {
-          const double2 pr = cmul(T[tid][l], Gv[l][j]);
-          acc.x += pr.x;
-          acc.y += pr.y;
-        }
-      q = cmul(tj, acc);
-    }
-    __syncthreads();
-    if (tid < j) T[tid][j] = make_double2(-q.x, -q.y);
-    if (tid == j) T[j][j] = tj;
-    __syncthreads();
+    for (int i = 0; i < NR; ++i)
+      P[j][tid + 256 * i] = make_double2(0.0, 0.0);
+    if (tid == 0) tau_s[j] = make_double2(0.0, 0.0);
   }
-  // explicit V, V T^H and V T for every row of the problem (zero above r0).
-  // Thread (j = tid % NB, part = tid / NB) owns output column j and keeps
-  // column j of T and row j of T in registers.
+  __syncthreads();
+  // Gv = V^H V, the rows split over the waves
   {
-    const int j = tid % NB, part = tid / NB;
-    double2 tcol[NB], trow[NB];
+    qr_d4 gr, gi;
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      tcol[i] = T[i][j];
-      const double2 t = T[j][i];
-      trow[i] = make_double2(t.x, -t.y);  // conj(T[j][i])
+    for (int e = 0; e < 4; ++e) gr[e] = gi[e] = 0.0;
+    for (int q = 0; q < 16 * NR; ++q) {
+      const double2 a = P[lane & 15][64 * NR * wave + 4 * q + (lane >> 4)];
+      gr = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, a.x, gr, 0, 0, 0);
+      gr = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, a.y, gr, 0, 0, 0);
+      gi = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, a.y, gi, 0, 0, 0);
+      gi = __builtin_amdgcn_mfma_f64_16x16x4f64(-a.y, a.x, gi, 0, 0, 0);
     }
-    for (int64_t r = part; r < d.rows; r += NT / NB) {
-      const int64_t rl = r - r0;
-      double2 ah = make_double2(0.0, 0.0), an = make_double2(0.0, 0.0);
-      double2 vj = make_double2(0.0, 0.0);
-      if (rl >= 0) {
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          double2 v = make_double2(0.0, 0.0);
-          if (i < ncp && rl >= i)
-            v = (rl == i) ? make_double2(1.0, 0.0) : at(i, (int)rl);
-          if (i == j) vj = v;
-          const double2 h = cmul(v, trow[i]);
-          const double2 n = cmul(v, tcol[i]);
-          ah.x += h.x;
-          ah.y += h.y;
-          an.x += n.x;
-          an.y += n.y;
+    for (int e = 0; e < 4; ++e)
+      gp[wave][64 * e + lane] = make_double2(gr[e], gi[e]);
+  }
+  __syncthreads();
+  {
+    // result element e of lane l: row 4 e + l / 16, column l % 16
+    double2 t = gp[0][tid];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      t.x += gp[w][tid].x;
+      t.y += gp[w][tid].y;
+    }
+    Gv[tid >> 4][tid & 15] = t;
+  }
+  __syncthreads();
+  // T (zlarft): column j = -tau_j T[0:j,0:j] Gv[0:j, j], T[j][j] = tau_j;
+  // row i of T needs only its own entries
+  if (tid < NB) {
+    double2 t[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      double2 q = make_double2(0.0, 0.0);
+#pragma unroll
+      for (int l = 0; l < j; ++l) {
+        const double2 pr = cmul(t[l], Gv[l][j]);
+        q.x += pr.x;
+        q.y += pr.y;
+      }
+      const double2 tj = tau_s[j];
+      const double2 m = cmul(tj, q);
+      t[j] = j > tid ? make_double2(-m.x, -m.y)
+                     : j == tid ? tj : make_double2(0.0, 0.0);
+      T[tid][j] = t[j];
+    }
+  }
+  // explicit V, V T^H and V T; zero above the panel
+  for (int64_t r = tid; r < r0; r += 256)
+    for (int c = 0; c < NB; ++c) {
+      Vb[r + c * lda] = make_double2(0.0, 0.0);
+      VTh[r + c * lda] = make_double2(0.0, 0.0);
+      if (write_vtn) VTn[r + c * lda] = make_double2(0.0, 0.0);
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NR; ++i)
+#pragma unroll
+    for (int c = 0; c < NB; ++c) x[i][c] = P[c][tid + 256 * i];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    double2 ah[NR], an[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      ah[i] = an[i] = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int l = j; l < NB; ++l) {
+      const double2 t = T[j][l];
+#pragma unroll
+      for (int i = 0; i < NR; ++i) {
+        const double2 u = cmulc(t, x[i][l]);  // conj(T[j][l]) V[r][l]
+        ah[i].x += u.x;
+        ah[i].y += u.y;
+      }
+    }
+    if (write_vtn) {
+#pragma unroll
+      for (int l = 0; l <= j; ++l) {
+        const double2 t = T[l][j];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+          const double2 u = cmul(t, x[i][l]);
+          an[i].x += u.x;
+          an[i].y += u.y;
         }
       }
-      Vb[r + j * lda] = vj;
-      VTh[r + j * lda] = ah;
-      if (write_vtn) VTn[r + j * lda] = an;
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const int64_t r = r0 + tid + 256 * i;
+      if (r >= d.rows) continue;
+      Vb[r + j * lda] = x[i][j];
+      VTh[r + j * lda] = ah[i];
+      if (write_vtn) VTn[r + j * lda] = an[i];
     }
   }
 }
@@ -811,10 +930,12 @@ int32_t BatchedQR::factor(qtn_ctx* ctx, double2* A, int64_t lda, int64_t sA,
     double2* Vk = V + (int64_t)vslot(k) * vs;
     double2* VThk = VTh + (int64_t)(k & 1) * vs;
     double2* VTnk = VTn + (keep_q ? (int64_t)k * vs : 0);
-    if (maxr - (int64_t)k * NB <= kLdsRows)
-      hipLaunchKernelGGL((qr_panel_t<true, 256>), dim3(batch), dim3(256), 0,
-                         s, A, lda, sA, k, (const QrDims*)ddims, Vk, VThk,
-                         VTnk, vstride, 2 * vs, keep_q ? 1 : 0);
+    const int64_t left = maxr - (int64_t)k * NB;
+    if (left <= kLdsRows)
+      hipLaunchKernelGGL((left <= 256 ? qr_panel_reg<1> : qr_panel_reg<2>),
+                         dim3(batch), dim3(256), 0, s, A, lda, sA, k,
+                         (const QrDims*)ddims, Vk, VThk, VTnk, vstride, 2 * vs,
+                         keep_q ? 1 : 0);
     else
       hipLaunchKernelGGL((qr_panel_left<512>), dim3(batch), dim3(512), 0, s,
                          A, lda, sA, k, (const QrDims*)ddims, Vk, VThk, VTnk,
