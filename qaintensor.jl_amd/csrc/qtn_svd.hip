@@ -1823,12 +1823,16 @@ __global__ __launch_bounds__(256) void jac_round_res(
 // so neither pass is staged through LDS, and Q X_IJ leaves from the
 // accumulators.  The 16-row tiles go to the eight waves in turn; the Gram's
 // partials meet in LDS.  The diagonal quadrants take three real products
-// (Im = M - M^T, M = Xr^T Xi), the update four.
+// (Im = M - M^T, M = Xr^T Xi), and so does the update (Gauss, as in
+// res_update): matrix cores bound both passes.  Its error bound per column
+// has the same form as four products', and the error of the 40-qubit FP64
+// circuit against LAPACK in 64 bits did not move (3.8e-13 with four, 3.5e-13
+// with three; 290 -> 274 ms).
 // Three launches per round cost a kernel boundary each (about 5 us with
 // several streams busy) and a pass over X more.
 // FP64 at 512 rows, six problems of 16 pairs on each of two streams: 43 us a
 // round against 15 + 20 + 20 us and two boundaries; the two passes of MFMAs
-// (160 and 256 of 64 cycles per wave, two waves a SIMD) are 22 us of it.
+// (160 and 192 of 64 cycles per wave, two waves a SIMD) are 19 us of it.
 //
 // NT: 16-row tiles per wave, for up to 128 NT rows.  A tile a wave does not
 // have is read as the last one and not used, so that the loads are a straight
@@ -1853,30 +1857,30 @@ template <typename R, int NT>
 __device__ __forceinline__ void reg_update(
     typename JT<R>::c_t* __restrict__ X, int64_t ldx, int ntiles, int I,
     int J, int wave, const typename JT<R>::c_t (&x)[NT][8],
-    const R (*Qr)[33], const R (*Qi)[33]) {
+    const R (*Q0)[33], const R (*Q1)[33], const R (*Q2)[33]) {
   using acc_t = typename JT<R>::acc_t;
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     if (wave + 8 * i >= ntiles) break;
-    acc_t yr[2], yi[2];
+    acc_t k1[2], k2[2], k3[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) yr[j][e] = yi[j][e] = (R)0;
+      for (int e = 0; e < 4; ++e) k1[j][e] = k2[j][e] = k3[j][e] = (R)0;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int k = 4 * s + (lane >> 4);
-      const R xr = x[i][s].x, xi = x[i][s].y;
+      const R xr = x[i][s].x, xi = x[i][s].y, xs = xr + xi;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
-        const R qr = Qr[k][16 * j + (lane & 15)],
-                qi = Qi[k][16 * j + (lane & 15)];
-        yr[j] = JT<R>::mfma(qr, xr, yr[j]);
-        yr[j] = JT<R>::mfma(qi, -xi, yr[j]);
-        yi[j] = JT<R>::mfma(qi, xr, yi[j]);
-        yi[j] = JT<R>::mfma(qr, xi, yi[j]);
+        const int n = 16 * j + (lane & 15);
+        k1[j] = JT<R>::mfma(Q0[k][n], xs, k1[j]);
+        k2[j] = JT<R>::mfma(Q1[k][n], xr, k2[j]);
+        k3[j] = JT<R>::mfma(Q2[k][n], xi, k3[j]);
       }
+      // keep the compiler from reading every Q ahead (registers are full)
+      if (sizeof(R) == 8 && (s & 1)) __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
@@ -1884,7 +1888,7 @@ __device__ __forceinline__ void reg_update(
       for (int e = 0; e < 4; ++e)
         X[16 * (wave + 8 * i) + (lane & 15) +
           pair_col<32>(16 * j + JT<R>::row(lane, e), I, J) * ldx] =
-            JT<R>::mk(yr[j][e], yi[j][e]);
+            JT<R>::mk(k1[j][e] - k3[j][e], k1[j][e] + k2[j][e]);
   }
 }
 
@@ -1895,7 +1899,8 @@ struct RegShared {
     R part[4][24][64];  // partial Grams of four waves
     struct {
       R sum[24][64];    // their sum
-      R Qr[32][33], Qi[32][33];
+      // c, d - c and c + d of Q = c + i d
+      R Q0[32][33], Q1[32][33], Q2[32][33];
     } s;
   };
 };
@@ -2055,8 +2060,9 @@ void jac_round_reg(
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int col = (u & 1) ? 16 + c : c;
-      sh.s.Qr[r + (u >> 1)][col] = b[u].x;
-      sh.s.Qi[r + (u >> 1)][col] = b[u].y;
+      sh.s.Q0[r + (u >> 1)][col] = b[u].x;
+      sh.s.Q1[r + (u >> 1)][col] = b[u].y - b[u].x;
+      sh.s.Q2[r + (u >> 1)][col] = b[u].x + b[u].y;
     }
   }
   __syncthreads();
@@ -2070,12 +2076,12 @@ void jac_round_reg(
   }
   // 3. X_IJ <- X_IJ Q (and W_IJ <- W_IJ Q)
   if constexpr (!kEarly) reg_load<R, NT>(X, ldx, ntiles, I, J, wave, x);
-  reg_update<R, NT>(X, ldx, ntiles, I, J, wave, x, sh.s.Qr, sh.s.Qi);
+  reg_update<R, NT>(X, ldx, ntiles, I, J, wave, x, sh.s.Q0, sh.s.Q1, sh.s.Q2);
   if (do_w) {
     c_t* Wb = Wm + (int64_t)bz * sW;
     reg_load<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x);
-    reg_update<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x, sh.s.Qr,
-                      sh.s.Qi);
+    reg_update<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x, sh.s.Q0,
+                      sh.s.Q1, sh.s.Q2);
   }
 }
 
