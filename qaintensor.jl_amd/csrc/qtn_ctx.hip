@@ -74,6 +74,22 @@ int32_t qtn_ctx::pinned_buffer(size_t bytes, void** out) {
   return QTN_OK;
 }
 
+int32_t qtn_ctx::pinned_area(int area, size_t bytes, void** out) {
+  if (pin_bytes[area] < bytes) {
+    if (pin_area[area]) {
+      QTN_CHECK_HIP(hipStreamSynchronize(stream));
+      QTN_CHECK_HIP(hipHostFree(pin_area[area]));
+      pin_area[area] = nullptr;
+      pin_bytes[area] = 0;
+    }
+    const size_t want = bytes < 4096 ? 4096 : bytes;
+    QTN_CHECK_HIP(hipHostMalloc(&pin_area[area], want, hipHostMallocDefault));
+    pin_bytes[area] = want;
+  }
+  *out = pin_area[area];
+  return QTN_OK;
+}
+
 int32_t qtn_ctx::side_stream(hipStream_t* out) {
   if (!side) {
     QTN_CHECK_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
@@ -180,6 +196,8 @@ int32_t qtn_ctx_destroy(qtn_ctx* ctx) try {
   for (auto& b : ctx->bufs)
     if (b.ptr) QTN_CHECK_HIP(hipFree(b.ptr));
   if (ctx->pinned) QTN_CHECK_HIP(hipHostFree(ctx->pinned));
+  for (void* a : ctx->pin_area)
+    if (a) QTN_CHECK_HIP(hipHostFree(a));
   for (auto e : ctx->ev_pool) QTN_CHECK_HIP(hipEventDestroy(e));
   for (auto& g : ctx->sweep_graphs) {
     QTN_CHECK_HIP(hipGraphExecDestroy(g.exec));

@@ -168,6 +168,17 @@ struct qtn_ctx {
   // Returns a device buffer of at least `bytes` for slot `slot`.
   int32_t buffer(int slot, size_t bytes, void** out);
   int32_t pinned_buffer(size_t bytes, void** out);
+  // Small pinned areas with one purpose each, grown on demand: the sweep
+  // flags (fixed size, its address is part of cached graphs), the results a
+  // solve writes for the host, the inputs of a solve on their way to the
+  // device, and a batch's gate descriptors on theirs.  Kernels write the
+  // first two directly (host memory is mapped), so a read-back is the wait
+  // for the stream and nothing else.  An area may be reused once the stream
+  // has been waited for.
+  enum { kPinFlags = 0, kPinResults, kPinInputs, kPinGates, kPinAreas };
+  void* pin_area[kPinAreas] = {};
+  size_t pin_bytes[kPinAreas] = {};
+  int32_t pinned_area(int area, size_t bytes, void** out);
   // Worker contexts (same device, own stream and scratch) that run
   // independent batches concurrently with this one; created on first use,
   // destroyed with it.  parent is set on workers.

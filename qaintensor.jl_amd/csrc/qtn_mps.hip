@@ -32,7 +32,7 @@ namespace {
 
 constexpr int kSlot1q = 47;
 constexpr int kSlotPhi = 30, kSlotXm = 31, kSlotVk = 32, kSlotDesc = 33,
-              kSlotGates = 34, kSlotEnv = 35, kSlotT1 = 36, kSlotT2 = 37,
+              kSlotEnv = 35, kSlotT1 = 36, kSlotT2 = 37,
               kSlotRed = 38, kSlotBits = 39, kSlotAmp = 40, kSlotW2 = 41,
               kSlotA1 = 42, kSlotA2 = 43, kSlotQd = 44, kSlotNrm = 45,
               kSlotPerm2 = 46, kSlotX32 = 70, kSlotW32 = 71, kSlotNsG = 72,
@@ -1255,10 +1255,19 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
   QTN_TRY(ctx->buffer(kSlotVk, (size_t)ng * maxN * std::max(maxM, maxN) *
                                    sizeof(double2),
                       &dVk));
-  const size_t desc_bytes = (size_t)ng * (sizeof(GateDesc) +
-                                          4 * sizeof(GemmDesc<double>));
+  // gates, gate descriptors and the first products' descriptors go to the
+  // device together, through pinned memory; later ones behind them
+  const size_t gate_bytes = (size_t)ng * 16 * sizeof(double2);
+  const size_t first_bytes =
+      gate_bytes + (size_t)ng * (sizeof(GateDesc) + sizeof(GemmDesc<double>));
+  const size_t desc_bytes =
+      first_bytes + (size_t)ng * 3 * sizeof(GemmDesc<double>);
+  static_assert(sizeof(GateDesc) % 16 == 0 && sizeof(GemmDesc<double>) % 16 == 0,
+                "descriptors follow each other 16-byte aligned");
+  void* pin;
   QTN_TRY(ctx->buffer(kSlotDesc, desc_bytes, &ddesc));
-  QTN_TRY(ctx->buffer(kSlotGates, (size_t)ng * 16 * sizeof(double2), &dg));
+  QTN_TRY(ctx->pinned_area(qtn_ctx::kPinGates, desc_bytes, &pin));
+  dg = ddesc;
   std::vector<GateDesc> gd(ng);
   std::vector<GemmDesc<double>> g1(ng);
   std::vector<int64_t> nsv(ng);
@@ -1297,15 +1306,18 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
     e.C = d.phi;
     e.ldc = M;
   }
-  GateDesc* d_gd = (GateDesc*)ddesc;
+  GateDesc* d_gd = (GateDesc*)((char*)ddesc + gate_bytes);
   GemmDesc<double>* d_g1 = (GemmDesc<double>*)(d_gd + ng);
   GemmDesc<double>* d_g2 = d_g1 + ng;
-  QTN_CHECK_HIP(hipMemcpyAsync(dg, gates, (size_t)ng * 16 * sizeof(double2),
-                               hipMemcpyHostToDevice, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(d_gd, gd.data(), ng * sizeof(GateDesc),
-                               hipMemcpyHostToDevice, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(d_g1, g1.data(), ng * sizeof(GemmDesc<double>),
-                               hipMemcpyHostToDevice, s));
+  {
+    char* c = (char*)pin;
+    std::memcpy(c, gates, gate_bytes);
+    std::memcpy(c + gate_bytes, gd.data(), ng * sizeof(GateDesc));
+    std::memcpy(c + gate_bytes + ng * sizeof(GateDesc), g1.data(),
+                ng * sizeof(GemmDesc<double>));
+  }
+  QTN_CHECK_HIP(
+      hipMemcpyAsync(ddesc, pin, first_bytes, hipMemcpyHostToDevice, s));
   // 1. theta0 = B_i B_{i+1}
   QTN_TRY(launch_zgemm_grouped(s, 0, 0, d_g1, ng, maxM, maxN));
   // 2. gate, lambda scaling, X = theta^H (zero padded)
@@ -1376,17 +1388,12 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
                           std::vector<int>& t, std::vector<double>& d,
                           std::vector<double>& tt,
                           std::vector<double>& kw) -> int32_t {
-    QTN_CHECK_HIP(hipMemcpyAsync(k.data(), e.kept, ng * sizeof(int64_t),
-                                 hipMemcpyDeviceToHost, s));
-    QTN_CHECK_HIP(hipMemcpyAsync(t.data(), e.status, ng * sizeof(int),
-                                 hipMemcpyDeviceToHost, s));
-    QTN_CHECK_HIP(hipMemcpyAsync(d.data(), e.disc, ng * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
-    QTN_CHECK_HIP(hipMemcpyAsync(tt.data(), e.total, ng * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
-    QTN_CHECK_HIP(hipMemcpyAsync(kw.data(), e.keptw, ng * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
     QTN_CHECK_HIP(hipStreamSynchronize(s));
+    k.assign(e.h_kept, e.h_kept + ng);
+    t.assign(e.h_status, e.h_status + ng);
+    d.assign(e.h_disc, e.h_disc + ng);
+    tt.assign(e.h_total, e.h_total + ng);
+    kw.assign(e.h_keptw, e.h_keptw + ng);
     return QTN_OK;
   };
   // The learned form is the chosen form plus the range finder: gates whose
@@ -1662,8 +1669,12 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
     e.C = d.Bl;
     e.ldc = 2 * d.chiL;
   }
-  QTN_CHECK_HIP(hipMemcpyAsync(d_g2, g2.data(), ng * sizeof(GemmDesc<double>),
-                               hipMemcpyHostToDevice, s));
+  {
+    char* c = (char*)pin + first_bytes;
+    std::memcpy(c, g2.data(), ng * sizeof(GemmDesc<double>));
+    QTN_CHECK_HIP(hipMemcpyAsync(d_g2, c, ng * sizeof(GemmDesc<double>),
+                                 hipMemcpyHostToDevice, s));
+  }
   QTN_TRY(launch_zgemm_grouped(s, 0, 0, d_g2, ng, maxM, maxk));
   if (chosen || learned) {
     // S_k = column norms of diag(lambda_{i-1}) Phi V_k in FP64; B_i and

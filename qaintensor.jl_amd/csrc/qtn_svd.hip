@@ -43,7 +43,7 @@ struct SweepKey {
       per_problem_w;
   int64_t ldx, sx, sw, ldw;
   double tol, conv2;
-  const void* ptr[11];
+  const void* ptr[12];
 };
 
 // QTN_SWEEP_GRAPHS=0 launches every sweep directly (read at every call).
@@ -2091,13 +2091,14 @@ void jac_round_reg(
 // columns orthogonal to O(conv2) (cyclic Jacobi converges quadratically),
 // so the confirming sweep is skipped.
 // misc: [0] problems still active, [1] non-finite input seen, [2] / [3]
-// the sweep's rotated pairs (of X / of X and W); [4..7] receive a snapshot
-// of [0..3] for the host, and [2], [3] restart at zero, so the sweep needs
-// no memset (and can be replayed from a graph).
+// the sweep's rotated pairs (of X / of X and W); host (pinned) receives a
+// snapshot of the four, and [2], [3] restart at zero, so the sweep needs no
+// memset and no copy (and can be replayed from a graph).
 __global__ void jac_sweep_end(int* __restrict__ active,
                               int* __restrict__ counters,
                               double* __restrict__ offmax, double conv2,
-                              int batch, int* __restrict__ misc) {
+                              int batch, int* __restrict__ misc,
+                              int* __restrict__ host) {
   __shared__ int cnt;
   if (threadIdx.x == 0) cnt = 0;
   __syncthreads();
@@ -2111,10 +2112,10 @@ __global__ void jac_sweep_end(int* __restrict__ active,
   __syncthreads();
   if (threadIdx.x == 0) {
     misc[0] = cnt;
-    misc[4] = cnt;
-    misc[5] = misc[1];
-    misc[6] = misc[2];
-    misc[7] = misc[3];
+    host[0] = cnt;
+    host[1] = misc[1];
+    host[2] = misc[2];
+    host[3] = misc[3];
     misc[2] = 0;
     misc[3] = 0;
   }
@@ -2158,9 +2159,10 @@ __global__ __launch_bounds__(256) void jac_prep_partial(
     const typename JT<R>::c_t* __restrict__ X, int64_t rows, int64_t ldx,
     int64_t cols, int64_t sX, const int* __restrict__ mask,
     double* __restrict__ part_scale, double* __restrict__ part_ssq,
-    int* __restrict__ part_bad) {
+    int* __restrict__ part_bad, int* __restrict__ misc) {
   const int bz = blockIdx.y;
   const int slot = bz * kPrepBlocks + blockIdx.x;
+  if (slot == 0 && threadIdx.x < 4) misc[threadIdx.x] = 0;
   if (mask && !mask[bz]) {
     if (threadIdx.x == 0) {
       part_scale[slot] = 0.0;
@@ -2221,7 +2223,8 @@ __global__ void jac_prep_final(int batch, double zrel,
                                int* __restrict__ active,
                                int* __restrict__ counters,
                                int* __restrict__ bad,
-                               int* __restrict__ scale_e) {
+                               int* __restrict__ scale_e,
+                               double* __restrict__ offmax) {
   const int bz = blockIdx.x * blockDim.x + threadIdx.x;
   if (bz >= batch) return;
   double scale = 0.0, ssq = 0.0;
@@ -2241,6 +2244,7 @@ __global__ void jac_prep_final(int batch, double zrel,
   zthr[bz] = zrel * zrel * f2s;
   active[bz] = (on && f2s > 0.0 && !nf) ? 1 : 0;
   counters[bz] = 0;
+  offmax[bz] = 0.0;
   if (on && nf) atomicOr(bad, 1);
 }
 
@@ -2302,7 +2306,9 @@ __global__ __launch_bounds__(1024) void jac_sort_trunc(
     int64_t chimax, int64_t* __restrict__ kept, double* __restrict__ disc,
     double* __restrict__ total, double* __restrict__ keptw,
     int* __restrict__ status, const int* __restrict__ scale_e,
-    const int64_t* __restrict__ chimax_arr) {
+    const int64_t* __restrict__ chimax_arr, int64_t* __restrict__ h_kept,
+    double* __restrict__ h_disc, double* __restrict__ h_total,
+    double* __restrict__ h_keptw, int* __restrict__ h_status) {
   const int bz = blockIdx.x;
   __shared__ double sv[kSortMax];
   __shared__ int si[kSortMax];
@@ -2386,11 +2392,12 @@ __global__ __launch_bounds__(1024) void jac_sort_trunc(
       const double v = ldexp(sv[j], -e);
       kw += v * v;
     }
-    kept[bz] = k;
-    disc[bz] = ldexp(disc_w, 2 * e);
-    total[bz] = ldexp(tot, 2 * e);
-    keptw[bz] = ldexp(kw, 2 * e);
-    status[bz] = st;
+    // for the kernels that follow, and for the host (pinned)
+    h_kept[bz] = kept[bz] = k;
+    h_disc[bz] = disc[bz] = ldexp(disc_w, 2 * e);
+    h_total[bz] = total[bz] = ldexp(tot, 2 * e);
+    h_keptw[bz] = keptw[bz] = ldexp(kw, 2 * e);
+    h_status[bz] = status[bz] = st;
   }
 }
 
@@ -2484,10 +2491,15 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
   c += (size_t)batch * kPrepBlocks * sizeof(double);
   kept = (int64_t*)c;
   c += batch * sizeof(int64_t);
+  // the inputs of a run, one copy: caps, column counts, W wishes, mask
   chimax_dev = (int64_t*)c;
   c += batch * sizeof(int64_t);
   nsv = (int64_t*)c;
   c += batch * sizeof(int64_t);
+  want_w = (int*)c;
+  c += batch * sizeof(int);
+  mask = (int*)c;
+  c += batch * sizeof(int);
   flags = (int*)c;
   c += (size_t)batch * p * sizeof(int);
   counters = (int*)c;
@@ -2495,10 +2507,6 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
   active = (int*)c;
   c += batch * sizeof(int);
   status = (int*)c;
-  c += batch * sizeof(int);
-  want_w = (int*)c;
-  c += batch * sizeof(int);
-  mask = (int*)c;
   c += batch * sizeof(int);
   scale_e = (int*)c;
   c += batch * sizeof(int);
@@ -2760,19 +2768,38 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   const int nchunk_x = (int)(rows_p / 64);
   const int nchunk_w = (int)(cols_p / 64);
 
-  QTN_CHECK_HIP(hipMemcpyAsync(nsv, nsv_host, batch * sizeof(int64_t),
-                               hipMemcpyHostToDevice, s));
-  if (want_w_host)
-    QTN_CHECK_HIP(hipMemcpyAsync(want_w, want_w_host, batch * sizeof(int),
+  // Inputs through pinned memory in one copy (laid out as reserve() does),
+  // results and flags straight into it.
+  {
+    void* pin;
+    const size_t bytes =
+        (size_t)batch * (2 * sizeof(int64_t) + 2 * sizeof(int));
+    QTN_TRY(ctx->pinned_area(qtn_ctx::kPinInputs, bytes, &pin));
+    int64_t* pc = (int64_t*)pin;
+    int64_t* pn = pc + batch;
+    int* pw = (int*)(pn + batch);
+    int* pm = pw + batch;
+    for (int b = 0; b < batch; ++b) {
+      pc[b] = chimax_per ? chimax_per[b] : 0;
+      pn[b] = nsv_host[b];
+      pw[b] = want_w_host ? want_w_host[b] : 1;
+      pm[b] = mask_host ? mask_host[b] : 1;
+    }
+    QTN_CHECK_HIP(hipMemcpyAsync(chimax_dev, pin, bytes,
                                  hipMemcpyHostToDevice, s));
-  if (mask_host)
-    QTN_CHECK_HIP(hipMemcpyAsync(mask, mask_host, batch * sizeof(int),
-                                 hipMemcpyHostToDevice, s));
-  if (chimax_per)
-    QTN_CHECK_HIP(hipMemcpyAsync(chimax_dev, chimax_per,
-                                 batch * sizeof(int64_t),
-                                 hipMemcpyHostToDevice, s));
-  QTN_CHECK_HIP(hipMemsetAsync(misc, 0, 4 * sizeof(int), s));
+    QTN_TRY(ctx->pinned_area(
+        qtn_ctx::kPinResults,
+        (size_t)batch * (sizeof(int64_t) + 3 * sizeof(double) + sizeof(int)),
+        &pin));
+    h_kept = (int64_t*)pin;
+    h_disc = (double*)(h_kept + batch);
+    h_total = h_disc + batch;
+    h_keptw = h_total + batch;
+    h_status = (int*)(h_keptw + batch);
+  }
+  int* host_flags = nullptr;
+  QTN_TRY(ctx->pinned_area(qtn_ctx::kPinFlags, 4 * sizeof(int),
+                           (void**)&host_flags));
   ctx_ = ctx;
   prof_events.clear();
   prof_reg.clear();
@@ -2782,16 +2809,15 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     for (int b = 0; b < batch; ++b) n_act += mask_host[b] ? 1 : 0;
   }
   const int n_solved = n_act;
-  QTN_CHECK_HIP(hipMemsetAsync(offmax, 0, batch * sizeof(double), s));
   hipLaunchKernelGGL(jac_prep_partial<R>, dim3(kPrepBlocks, batch),
                      dim3(256), 0, s, (const c_t*)X, rows_p, ldx, cols_p, sX,
                      (const int*)(mask_host ? mask : nullptr), prep_scale,
-                     prep_ssq, prep_bad);
+                     prep_ssq, prep_bad, misc);
   hipLaunchKernelGGL(jac_prep_final, dim3((batch + 63) / 64), dim3(64), 0, s,
                      batch, zrel, (const double*)prep_scale,
                      (const double*)prep_ssq, (const int*)prep_bad,
                      (const int*)(mask_host ? mask : nullptr), normF2, zthr,
-                     active, counters, misc + 1, scale_e);
+                     active, counters, misc + 1, scale_e, offmax);
   QTN_CHECK_HIP(hipGetLastError());
   const unsigned sgrid = (unsigned)std::max<int64_t>(
       1, std::min<int64_t>((rows_p * cols_p + 255) / 256, 2048));
@@ -2803,8 +2829,6 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     QTN_TRY(launch_identity_t<R>(s, Wm, cols_p, ldw ? ldw : cols_p, sW,
                                  batch));
   }
-  int* host_flags = nullptr;
-  QTN_TRY(ctx->pinned_buffer(4 * sizeof(int), (void**)&host_flags));
   // A problem of one block pair is solved whole by its first pass and
   // checked on a fresh Gram by the second, so the two go out together (a
   // read-back less per solve; a problem done after the first skips the
@@ -2825,7 +2849,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
       }
       QTN_CHECK_HIP(hipGetLastError());
       hipLaunchKernelGGL(jac_sweep_end, dim3(1), dim3(256), 0, s, active,
-                         counters, offmax, conv2, batch, misc);
+                         counters, offmax, conv2, batch, misc, host_flags);
       QTN_CHECK_HIP(hipGetLastError());
     }
     return QTN_OK;
@@ -2855,7 +2879,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     key.tol = tol;
     key.conv2 = conv2;
     const void* ptrs[] = {X, Wm, want_w, zthr, counters, active, offmax,
-                          misc, Gp, Q, flags};
+                          misc, Gp, Q, flags, host_flags};
     static_assert(sizeof(ptrs) == sizeof(key.ptr), "SweepKey pointers");
     std::memcpy(key.ptr, ptrs, sizeof(ptrs));
     QTN_TRY(ctx->sweep_graph(&key, sizeof(key), s, enqueue_sweep, &exec));
@@ -2867,8 +2891,6 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
       QTN_CHECK_HIP(hipGraphLaunch(exec, s));
     else
       QTN_TRY(enqueue_sweep());
-    QTN_CHECK_HIP(hipMemcpyAsync(host_flags, misc + 4, 4 * sizeof(int),
-                                 hipMemcpyDeviceToHost, s));
     QTN_CHECK_HIP(hipStreamSynchronize(s));
     if (ctx->prof)
       QTN_TRY(account_sweep(n_act, host_flags[2], host_flags[3], nchunk_x,
@@ -2908,7 +2930,8 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   hipLaunchKernelGGL(jac_sort_trunc, dim3(batch), dim3(1024), 0, s, sig, perm,
                      cols_p, (const int64_t*)nsv, cutoff, relative, chimax,
                      kept, disc, total, keptw, status, (const int*)scale_e,
-                     (const int64_t*)(chimax_per ? chimax_dev : nullptr));
+                     (const int64_t*)(chimax_per ? chimax_dev : nullptr),
+                     h_kept, h_disc, h_total, h_keptw, h_status);
   QTN_CHECK_HIP(hipGetLastError());
   return QTN_OK;
 }

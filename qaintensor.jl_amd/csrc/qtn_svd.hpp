@@ -58,6 +58,12 @@ struct JacobiEngine {
   double* offmax = nullptr; // largest scaled off-diagonal of the sweep
   int64_t* kept = nullptr;
   int64_t* nsv = nullptr;
+  // The results of a run per problem in pinned host memory, written by the
+  // run's last kernel: valid once the stream has been waited for, until the
+  // next run on the context.
+  int64_t* h_kept = nullptr;
+  double *h_disc = nullptr, *h_total = nullptr, *h_keptw = nullptr;
+  int* h_status = nullptr;
   int* flags = nullptr;
   int* counters = nullptr;
   int* active = nullptr;

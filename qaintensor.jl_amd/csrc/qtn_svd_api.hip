@@ -272,16 +272,10 @@ bool precond_enabled(bool dflt) {
 int32_t read_trunc(qtn_ctx* ctx, const JacobiEngine& eng, bool truncate,
                    int64_t* k, double* disc) {
   if (!truncate) return QTN_OK;
-  hipStream_t s = ctx->stream;
-  int st = 0;
-  QTN_CHECK_HIP(hipMemcpyAsync(k, eng.kept, sizeof(int64_t),
-                               hipMemcpyDeviceToHost, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(&st, eng.status, sizeof(int),
-                               hipMemcpyDeviceToHost, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(disc, eng.disc, sizeof(double),
-                               hipMemcpyDeviceToHost, s));
-  QTN_CHECK_HIP(hipStreamSynchronize(s));
-  if (st != 0) {
+  QTN_CHECK_HIP(hipStreamSynchronize(ctx->stream));
+  *k = eng.h_kept[0];
+  *disc = eng.h_disc[0];
+  if (eng.h_status[0] != 0) {
     set_error("svd: every singular value is within the truncation error");
     return QTN_ERR_TRUNC;
   }
@@ -676,16 +670,10 @@ int32_t svd_device_chosen(qtn_ctx* ctx, const double2* dA, int64_t m,
   QTN_TRY(eng.run32(ctx, (float2*)dX, rows_p, rows_p * cols_p, (float2*)dW,
                     cols_p * cols_p, nullptr, &nsv, cutoff, relative, chimax,
                     60, &sweeps));
-  int64_t k = 0;
-  int st = 0;
-  double disc = 0.0;
-  QTN_CHECK_HIP(hipMemcpyAsync(&k, eng.kept, sizeof(int64_t),
-                               hipMemcpyDeviceToHost, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(&st, eng.status, sizeof(int),
-                               hipMemcpyDeviceToHost, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(&disc, eng.disc, sizeof(double),
-                               hipMemcpyDeviceToHost, s));
   QTN_CHECK_HIP(hipStreamSynchronize(s));
+  const int64_t k = eng.h_kept[0];
+  const int st = eng.h_status[0];
+  double disc = eng.h_disc[0];
   if (st != 0 || k != chimax) {
     ctx->n_rr_redone += 1;
     return fp64_fallback(fallback);
