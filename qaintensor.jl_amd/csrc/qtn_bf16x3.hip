@@ -10,10 +10,11 @@
 // x = x0 + x1 + x2 with x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 -
 // x1) (24 significand bits, the FP32 input's), and whose product keeps the
 // six terms a_i b_j with i + j <= 2 (the dropped ones are below 2^-24
-// relative), accumulated in FP32 by v_mfma_f32_16x16x32_bf16.  The result
-// carries FP32-level error (about 1e-7 relative to |opA| |B| per entry,
-// growing like sqrt(K)); it replaces FP64 only where that is the stated
-// precision (the large contractions of the MPO expectation sweep).
+// relative), accumulated by v_mfma_f32_16x16x32_bf16 in FP32 over 64 inner
+// indices and in FP64 over those.  The result carries FP32-level error (about
+// 1e-7 relative to |opA| |B| per entry, at any K); it replaces FP64 only where
+// that is the stated precision (the large contractions of the MPO expectation
+// sweep).
 #include <algorithm>
 #include <cstdint>
 
@@ -104,55 +105,96 @@ __global__ void split_b(const double2* __restrict__ B, int64_t ldb, int64_t K,
   }
 }
 
-// One 128 x 128 tile of the embedded product per workgroup (4 waves, each
-// 64 x 64 = 4 x 4 MFMA tiles of 16 x 16), K in steps of 32 staged through
-// LDS (three planes of A and of B, rows padded to 40 bf16).  MFMA operand
-// layout (16x16x32): lane l holds row (A) / column (B) l % 16 and the 8
-// consecutive k of group l / 16; the accumulator holds rows 4 (l / 16) + e,
-// column l % 16.  Output: rows r < M go to C[r, n].x, rows M <= r < 2M to
-// C[r - M, n].y.
-__global__ __launch_bounds__(256) void gemm_bf16x3(
+// One 128 x 128 tile of the embedded product per workgroup (8 waves, each
+// 32 x 64 = 2 x 4 MFMA tiles of 16 x 16), K in steps of 32 staged through two
+// LDS buffers (three planes of A and of B, rows padded to 40 bf16): the next
+// step's tiles are loaded before the products of the current one and written
+// to the other buffer after them, one barrier a step.  MFMA operand layout
+// (16x16x32): lane l holds row (A) / column (B) l % 16 and the 8 consecutive
+// k of group l / 16; the accumulator holds rows 4 (l / 16) + e, column l %
+// 16.  Output: rows r < M go to C[r, n].x, rows M <= r < 2M to C[r - M, n].y.
+//
+// The FP32 accumulators are added to FP64 ones every kFlush steps: over 2048
+// embedded inner indices the 384 FP32 additions per entry cost far more
+// accuracy than the operands' 24 bits.  The conversions run on the vector
+// units beside the other wave's MFMAs and cost what the prefetch gains.  Bound
+// by the matrix cores and the LDS reads that feed them (18 KB per wave and
+// step).  <psi|H|psi> of 24 sites at chi 1024 (the largest products 6144 x
+// 2048 x 2048): 298 us per product, about 1000 TF of bf16, and a relative
+// error of 2e-8..1e-7; one buffer, no prefetch and FP32 accumulation: 293 us
+// and 3e-7..7e-6.  128 x 64 tiles with three workgroups per CU: 339 us.
+constexpr int kFlush = 2;
+constexpr int kGemmThreads = 512;
+
+__global__ __launch_bounds__(kGemmThreads) void gemm_bf16x3(
     const uint16_t* __restrict__ Ap, const uint16_t* __restrict__ Bp,
     int64_t M, int64_t N, int64_t Mp, int64_t Np, int64_t Kp,
     double2* __restrict__ C, int64_t ldc) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[3][kBM][kLdsK];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[3][kBN][kLdsK];
+  __shared__ __attribute__((aligned(16))) uint16_t As[2][3][kBM][kLdsK];
+  __shared__ __attribute__((aligned(16))) uint16_t Bs[2][3][kBN][kLdsK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t m0 = (int64_t)blockIdx.x * kBM, n0 = (int64_t)blockIdx.y * kBN;
-  const int wm = (wave & 1) * 64, wn = (wave >> 1) * 64;
+  // consecutive workgroups go to the 8 XCDs in turn: each takes a contiguous
+  // run of tiles
+  const uint32_t nt = gridDim.x * gridDim.y;
+  uint32_t t = blockIdx.x + gridDim.x * blockIdx.y;
+  t = (t % 8) * (nt / 8) + min(t % 8, nt % 8) + t / 8;
+  const int64_t m0 = (int64_t)(t % gridDim.x) * kBM;
+  const int64_t n0 = (int64_t)(t / gridDim.x) * kBN;
+  const int wm = (wave & 3) * 32, wn = (wave >> 2) * 64;
   const int64_t planeA = Mp * Kp, planeB = Np * Kp;
-  f32x4 acc[4][4];
+  f32x4 acc[2][4];
+  double sum[2][4][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < 4; ++j) {
+      acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum[i][j][e] = 0.0;
+    }
+  // per plane 128 rows x 32 k = 512 chunks of 8 bf16 (16 B), one per thread
+  const int srow = tid >> 2, skq = (tid & 3) * 8;
+  const uint16_t* pa = Ap + (m0 + srow) * Kp + skq;
+  const uint16_t* pb = Bp + (n0 + srow) * Kp + skq;
+  uint4 a0 = *(const uint4*)pa, a1 = *(const uint4*)(pa + planeA),
+        a2 = *(const uint4*)(pa + 2 * planeA);
+  uint4 b0 = *(const uint4*)pb, b1 = *(const uint4*)(pb + planeB),
+        b2 = *(const uint4*)(pb + 2 * planeB);
+  *(uint4*)&As[0][0][srow][skq] = a0;
+  *(uint4*)&As[0][1][srow][skq] = a1;
+  *(uint4*)&As[0][2][srow][skq] = a2;
+  *(uint4*)&Bs[0][0][srow][skq] = b0;
+  *(uint4*)&Bs[0][1][srow][skq] = b1;
+  *(uint4*)&Bs[0][2][srow][skq] = b2;
+  __syncthreads();
+  int buf = 0, step = 0;
   for (int64_t k0 = 0; k0 < Kp; k0 += kBK) {
-    // stage: per plane 128 rows x 32 k = 512 chunks of 8 bf16 (16 B)
-#pragma unroll
-    for (int pl = 0; pl < 3; ++pl)
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int c = tid + 256 * u;
-        const int row = c >> 2, kq = (c & 3) * 8;
-        const uint4 va = *(const uint4*)(Ap + pl * planeA +
-                                         (m0 + row) * Kp + k0 + kq);
-        const uint4 vb = *(const uint4*)(Bp + pl * planeB +
-                                         (n0 + row) * Kp + k0 + kq);
-        *(uint4*)&As[pl][row][kq] = va;
-        *(uint4*)&Bs[pl][row][kq] = vb;
-      }
-    __syncthreads();
+    const bool more = k0 + kBK < Kp;
+    if (more) {
+      pa += kBK;
+      pb += kBK;
+      a0 = *(const uint4*)pa;
+      a1 = *(const uint4*)(pa + planeA);
+      a2 = *(const uint4*)(pa + 2 * planeA);
+      b0 = *(const uint4*)pb;
+      b1 = *(const uint4*)(pb + planeB);
+      b2 = *(const uint4*)(pb + 2 * planeB);
+    }
     const int kg = (lane >> 4) * 8;
-    bf16x8 a[3][4], b[3][4];
+    bf16x8 a[3][2], b[3][4];
 #pragma unroll
-    for (int pl = 0; pl < 3; ++pl)
+    for (int pl = 0; pl < 3; ++pl) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[pl][i] = *(const bf16x8*)&As[pl][wm + i * 16 + (lane & 15)][kg];
-        b[pl][i] = *(const bf16x8*)&Bs[pl][wn + i * 16 + (lane & 15)][kg];
-      }
+      for (int i = 0; i < 2; ++i)
+        a[pl][i] =
+            *(const bf16x8*)&As[buf][pl][wm + i * 16 + (lane & 15)][kg];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int j = 0; j < 4; ++j)
+        b[pl][j] =
+            *(const bf16x8*)&Bs[buf][pl][wn + j * 16 + (lane & 15)][kg];
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         // smallest terms first
@@ -169,10 +211,30 @@ __global__ __launch_bounds__(256) void gemm_bf16x3(
         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
             a[0][i], b[0][j], acc[i][j], 0, 0, 0);
       }
+    if (++step == kFlush || !more) {
+      step = 0;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[i][j][e] += (double)acc[i][j][e];
+          acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    if (more) {
+      *(uint4*)&As[buf ^ 1][0][srow][skq] = a0;
+      *(uint4*)&As[buf ^ 1][1][srow][skq] = a1;
+      *(uint4*)&As[buf ^ 1][2][srow][skq] = a2;
+      *(uint4*)&Bs[buf ^ 1][0][srow][skq] = b0;
+      *(uint4*)&Bs[buf ^ 1][1][srow][skq] = b1;
+      *(uint4*)&Bs[buf ^ 1][2][srow][skq] = b2;
+    }
     __syncthreads();
+    buf ^= 1;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int64_t n = n0 + wn + j * 16 + (lane & 15);
@@ -181,10 +243,9 @@ __global__ __launch_bounds__(256) void gemm_bf16x3(
       for (int e = 0; e < 4; ++e) {
         const int64_t r = m0 + wm + i * 16 + 4 * (lane >> 4) + e;
         if (r < M)
-          reinterpret_cast<double*>(C + r + n * ldc)[0] = (double)acc[i][j][e];
+          reinterpret_cast<double*>(C + r + n * ldc)[0] = sum[i][j][e];
         else if (r < 2 * M)
-          reinterpret_cast<double*>(C + (r - M) + n * ldc)[1] =
-              (double)acc[i][j][e];
+          reinterpret_cast<double*>(C + (r - M) + n * ldc)[1] = sum[i][j][e];
       }
     }
 }
@@ -226,7 +287,7 @@ int32_t launch_zgemm_bf16x3(qtn_ctx* ctx, int opA, int64_t m, int64_t n,
                      ldb, k, n, Np, Kp, (uint16_t*)pb);
   hipLaunchKernelGGL(gemm_bf16x3, dim3((unsigned)(Mp / kBM),
                                        (unsigned)(Np / kBN)),
-                     dim3(256), 0, s, (const uint16_t*)pa,
+                     dim3(kGemmThreads), 0, s, (const uint16_t*)pa,
                      (const uint16_t*)pb, m, n, Mp, Np, Kp, C, ldc);
   QTN_CHECK_HIP(hipGetLastError());
   return QTN_OK;
