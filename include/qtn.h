@@ -50,9 +50,11 @@ extern "C" {
 #define QTN_ERR_NOTFINITE  -6  /* NaN/Inf met in the input of an SVD         */
 
 /* Jacobi block-pair tilings (qtn_tune_jacobi, qtn_set_jacobi_tiling) */
-#define QTN_TILING_W32       0  /* 32x32 Gram blocks, three launches a round */
+#define QTN_TILING_W32       0  /* 32x32 Gram blocks, three launches a round;
+                                 * up to 512 rows one launch in every round
+                                 * of a sweep but the first                   */
 #define QTN_TILING_W32_FUSED 1  /* 32x32 Gram blocks, one fused launch        */
-#define QTN_TILING_W64       2  /* 64x64 Gram blocks, three launches a round */
+#define QTN_TILING_W64       2  /* 64x64 Gram blocks, three launches a round  */
 
 /* precision forms of the two-site update */
 #define QTN_FORM_PLAIN      0  /* ComplexF64 end to end                       */
@@ -84,10 +86,11 @@ int32_t qtn_ctx_stream(qtn_ctx* ctx, void** stream);
 int32_t qtn_ctx_counters(qtn_ctx* ctx, int64_t* out, int32_t n,
                          int32_t reset);
 /* Per-kernel timing with HIP events on the context stream (off by default).
- * Kernel ids: 0 jac_inner, 1 jac_gram, 2 jac_update (the three-launch
- * block Jacobi round, FP64 sweeps), 3 jac_round (the opt-in fused round),
- * 4 jac_inner, 5 jac_gram, 6 jac_update, 7 jac_round (FP32 sweeps of the
- * chosen form; the fused round is their default from 320 to 512 rows).
+ * Kernel ids: 0 the inner solves, 1 jac_gram, 2 jac_update (the three-launch
+ * block Jacobi round, FP64 sweeps), 3 the rounds in one launch (up to 512
+ * rows all but a sweep's first), 4 the inner solves, 5 jac_gram, 6
+ * jac_update, 7 the rounds in one launch (FP32 sweeps of the chosen form;
+ * from 320 to 512 rows all of them).
  * Times come from start / stop events stamped by each dispatch.  qtn_ctx_profile(ctx, 1) enables and clears the accumulators.
  * qtn_ctx_profile_read returns, for one kernel id, the launch count, the
  * summed launch durations (ms), and the algorithmic HBM bytes and flops of
@@ -374,8 +377,9 @@ int32_t qtn_mps_expect_mpo(const qtn_mps* mps, const qtn_mpo* mpo,
 /* The same sweep in a precision form: QTN_FORM_PLAIN (= qtn_mps_expect_mpo,
  * complex FP64 throughout) or QTN_FORM_CHOSEN, where each site's two
  * bond-sized contractions run as BF16x3 split-precision GEMMs (three bf16
- * terms per operand, six products, FP32 accumulation on the bf16 matrix
- * cores) once all of their dimensions reach 512; smaller ones stay FP64.  */
+ * terms per operand, six products on the bf16 matrix cores, accumulated in
+ * FP32 over 64 inner indices and in FP64 over those) once all of their
+ * dimensions reach 512; smaller ones stay FP64.                           */
 int32_t qtn_mps_expect_mpo_form(const qtn_mps* mps, const qtn_mpo* mpo,
                                 int32_t form, double* out);
 /* C (m x n) = op(A) B in BF16x3 split precision (as above) on host

@@ -104,58 +104,6 @@ __global__ void qr_gather_cols(const double2* __restrict__ src,
   }
 }
 
-// Wave-shuffle then LDS sum of N complex partials per thread; every thread
-// gets the totals in out[].  scratch: NW waves x N double2 in LDS.
-template <int N, int NW = 4>
-__device__ __forceinline__ void block_sum_fast(double2 (&part)[N],
-                                               double2 (&out)[N],
-                                               double2* scratch) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // one butterfly step for all N values at a time, so the 2N shuffles of a
-  // step are independent and their latencies overlap
-  double x[N], y[N];
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    x[i] = part[i].x;
-    y[i] = part[i].y;
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    double sx[N], sy[N];
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      sx[i] = __shfl_xor(x[i], off, 64);
-      sy[i] = __shfl_xor(y[i], off, 64);
-    }
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-      x[i] += sx[i];
-      y[i] += sy[i];
-    }
-  }
-  if (lane < N) {
-    double vx = 0.0, vy = 0.0;
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-      if (i == lane) {
-        vx = x[i];
-        vy = y[i];
-      }
-    scratch[wave * N + lane] = make_double2(vx, vy);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < N; ++i) {
-    double2 t = scratch[i];
-    for (int w = 1; w < NW; ++w) {
-      t.x += scratch[w * N + i].x;
-      t.y += scratch[w * N + i].y;
-    }
-    out[i] = t;
-  }
-  __syncthreads();
-}
-
 // Sum of 32 values per lane over a wave, scattered: lane l returns the sum
 // of value l / 2.  Each step halves the values a lane still carries (swaps
 // of half-waves and of rows of 16, then DPP within the rows), 32 additions

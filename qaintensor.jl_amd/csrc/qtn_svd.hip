@@ -8,15 +8,20 @@
 //   X (rows x cols, zero padded to multiples of 64) is orthogonalised by
 //   right-multiplication with unitary rotations until every pair of columns
 //   satisfies |x_i^H x_j| <= tol * |x_i| |x_j|.  Columns are grouped into
-//   2p blocks of 32; a sweep is 2p-1 rounds of the round-robin tournament,
-//   each round handling p disjoint block pairs.  For a block pair (64
+//   2p blocks of 16; a sweep is 2p-1 rounds of the round-robin tournament,
+//   each round handling p disjoint block pairs.  For a block pair (32
 //   columns):
-//     1. jac_gram   : G = X_IJ^H X_IJ (64x64) on MFMA, split over row chunks
-//     2. jac_inner  : one cyclic two-sided Jacobi sweep on G in LDS (Hermitian
-//                     2x2 rotations, Golub & Van Loan 8.5), accumulating Q
+//     1. jac_gram   : G = X_IJ^H X_IJ (32x32) on MFMA, split over row chunks
+//     2. the inner sweep on G (Hermitian 2x2 rotations, Golub & Van Loan
+//                     8.5), accumulating Q: jac_inner in a sweep's first
+//                     round, where every pair of columns is rotated, and
+//                     jac_inner_cross in the others, where only the pairs
+//                     across the two blocks are
 //     3. jac_update : X_IJ <- X_IJ Q on MFMA (and W_IJ <- W_IJ Q if vectors
 //                     of the other side are needed)
-//   The pair is skipped when G already meets the tolerance, so convergence
+//   Problems of at most 512 rows run the three as one launch in the cross
+//   rounds (jac_round_reg), and problems of at most 64 columns are one block
+//   of 64 whose Gram is solved whole (jac_inner_whole).  The pair is skipped when G already meets the tolerance, so convergence
 //   is always decided on a Gram matrix freshly computed from the columns.
 // At convergence sigma_j = |x_j|; X W = U_X diag(sigma) with W unitary.
 // All updates are unitary rotations applied to X, so the singular values are
@@ -73,12 +78,7 @@ struct JT<double> {
   static __device__ __forceinline__ c_t mk(double re, double im) {
     return make_double2(re, im);
   }
-  static __device__ __forceinline__ double rsq(double x) { return rsqrt(x); }
-  static __device__ __forceinline__ double sq(double x) { return sqrt(x); }
   static __device__ __forceinline__ double ab(double x) { return fabs(x); }
-  static __device__ __forceinline__ double dv(double a, double b) {
-    return a / b;
-  }
   // 1 / sqrt(x) for the rotation parameters (make_rot): the hardware
   // v_rsq_f64 estimate (relative error e about 2^-26) and one third-order
   // step, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2, whose error e^3 is
@@ -106,20 +106,13 @@ struct JT<float> {
   }
   // The FP32 sweeps only produce candidates that are re-orthogonalised and
   // re-measured in FP64, so the rotation parameters use the one-instruction
-  // hardware forms (v_rsq_f32, v_sqrt_f32, v_rcp_f32, about 1 ulp) instead
-  // of the correctly rounded library sequences: the inner sweep is bound by
+  // hardware form (v_rsq_f32, about 1 ulp) instead of the correctly rounded
+  // library sequence: the inner sweep is bound by
   // its per-round instruction count.
-  static __device__ __forceinline__ float rsq(float x) {
+  static __device__ __forceinline__ float ab(float x) { return fabsf(x); }
+  static __device__ __forceinline__ float rsq_r(float x) {
     return __builtin_amdgcn_rsqf(x);
   }
-  static __device__ __forceinline__ float sq(float x) {
-    return __builtin_amdgcn_sqrtf(x);
-  }
-  static __device__ __forceinline__ float ab(float x) { return fabsf(x); }
-  static __device__ __forceinline__ float dv(float a, float b) {
-    return a * __builtin_amdgcn_rcpf(b);
-  }
-  static __device__ __forceinline__ float rsq_r(float x) { return rsq(x); }
 };
 
 // Round-robin (circle method) position -> block for 2p blocks.
@@ -567,11 +560,7 @@ __device__ __forceinline__ int inner_solve(
 // ---------------------------------------------------------------------------
 // 2. Sum the partial Grams, run inner cyclic Jacobi sweep(s), emit Q.
 // grid (p, batch), 256 threads.  flags[bz*p + pi] = 1 if Q must be applied.
-// Each of the W/2 rotation pairs of a round is owned by 512/W threads, which
-// all derive the rotation from G_pp, G_qq, G_pq themselves; thread t of a
-// pair updates rows / columns t, t+TP, ...  Two barriers per round: after
-// the column update (G J, Q J) and after the row update (J^H G).  Operands
-// are loaded into registers before any store so LDS latencies overlap.
+// The sweep itself is inner_solve, on planes in LDS, one barrier per round.
 template <typename R, int W>
 __global__ __launch_bounds__(256) void jac_inner(
     const typename JT<R>::c_t* __restrict__ Gp, int nchunk, int p,
@@ -581,9 +570,6 @@ __global__ __launch_bounds__(256) void jac_inner(
     double* __restrict__ offmax, int* __restrict__ qpairs, int cross,
     const int* __restrict__ want, int w_mode) {
   using c_t = typename JT<R>::c_t;
-  constexpr int NP = W / 2;       // rotation pairs per round
-  constexpr int TP = 256 / NP;    // threads per pair
-  constexpr int RPT = W / TP;     // rows (columns) per thread
   const int bz = blockIdx.y;
   const int pi = blockIdx.x;
   if (!active[bz]) return;
@@ -2408,16 +2394,17 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
                               int64_t cols_p_, bool single_, int n_active) {
   batch = batch_;
   single = single_;
-  // The fused round (one workgroup per block pair) leaves each 64-row
-  // chunk's load latency exposed with only 1-2 workgroups per CU; the
-  // three-launch round overlaps them across all chunks and is faster at
-  // chi = 256 in FP64.  FP32 problems of 320 to 512 rows fuse by default:
-  // their round keeps the whole block pair in LDS (jac_round_res), so only
-  // the tile load and store wait on memory.  The tile's LDS allows one
-  // workgroup per CU, which costs throughput on large batches of smaller
-  // problems (a 256-circuit batch of chi <= 128 ran 8% slower fused), so
-  // those keep the three launches.  QTN_JACOBI_FUSED=1 / 0 forces fused /
-  // three-launch rounds everywhere.
+  // A sweep's first round (and every round above 512 rows) runs as three
+  // launches: the fused jac_round (one workgroup per block pair) leaves each
+  // 64-row chunk's load latency exposed with only 1-2 workgroups per CU,
+  // while the three launches overlap them across all chunks.  FP32 problems
+  // of 320 to 512 rows fuse their first round by default: it keeps the whole
+  // block pair in LDS (jac_round_res), so only the tile load and store wait
+  // on memory.  The tile's LDS allows one workgroup per CU, which costs
+  // throughput on large batches of smaller problems (a 256-circuit batch of
+  // chi <= 128 ran 8% slower with every round fused), so those keep the
+  // three launches.  QTN_JACOBI_FUSED=1 / 0 forces fused / three-launch
+  // rounds everywhere.
   const size_t csz = single ? sizeof(float2) : sizeof(double2);
   rows_p = rows_p_;
   cols_p = cols_p_;

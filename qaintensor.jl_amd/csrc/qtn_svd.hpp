@@ -24,7 +24,7 @@ struct JacobiEngine {
   int p = 0;           // block pairs per round (= cols_p / W)
   bool single = false; // FP32 sweeps (complex float X, Gram and rotations)
   int slot_base = kSlotGram;  // first of the 5 context slots it uses
-  bool fused = false;  // W = 32 rounds as one jac_round launch
+  bool fused = false;  // W = 32 rounds as one jac_round / jac_round_res
   // FP32 fused rounds whose X (and W) tiles fit the LDS-resident kernel
   // (at most 512 rows) run jac_round_res; the other fused rounds jac_round
   bool res_round(int nchunk_x, int nchunk_w) const {
