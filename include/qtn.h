@@ -51,8 +51,9 @@ extern "C" {
 
 /* Jacobi block-pair tilings (qtn_tune_jacobi, qtn_set_jacobi_tiling) */
 #define QTN_TILING_W32       0  /* 32x32 Gram blocks, three launches a round;
-                                 * up to 512 rows one launch in every round
-                                 * of a sweep but the first                   */
+                                 * FP64 up to 512 rows outside the chosen and
+                                 * learned forms: one launch in every round of
+                                 * a sweep but the first                      */
 #define QTN_TILING_W32_FUSED 1  /* 32x32 Gram blocks, one fused launch        */
 #define QTN_TILING_W64       2  /* 64x64 Gram blocks, three launches a round  */
 
@@ -87,8 +88,8 @@ int32_t qtn_ctx_counters(qtn_ctx* ctx, int64_t* out, int32_t n,
                          int32_t reset);
 /* Per-kernel timing with HIP events on the context stream (off by default).
  * Kernel ids: 0 the inner solves, 1 jac_gram, 2 jac_update (the three-launch
- * block Jacobi round, FP64 sweeps), 3 the rounds in one launch (up to 512
- * rows all but a sweep's first), 4 the inner solves, 5 jac_gram, 6
+ * block Jacobi round, FP64 sweeps), 3 the rounds in one launch (plain form
+ * up to 512 rows: all but a sweep's first), 4 the inner solves, 5 jac_gram, 6
  * jac_update, 7 the rounds in one launch (FP32 sweeps of the chosen form;
  * from 320 to 512 rows all of them).
  * Times come from start / stop events stamped by each dispatch.  qtn_ctx_profile(ctx, 1) enables and clears the accumulators.

@@ -36,9 +36,7 @@ constexpr int kSlotPhi = 30, kSlotXm = 31, kSlotVk = 32, kSlotDesc = 33,
               kSlotRed = 38, kSlotBits = 39, kSlotAmp = 40, kSlotW2 = 41,
               kSlotA1 = 42, kSlotA2 = 43, kSlotQd = 44, kSlotNrm = 45,
               kSlotPerm2 = 46, kSlotX32 = 70, kSlotW32 = 71, kSlotNsG = 72,
-              kSlotNsT = 73, kSlotS64 = 74, kSlotMix = 75, kSlotEng32 = 80,
-              kSlotRef = 230, kSlotRefV = 231, kSlotRefP = 232,
-              kSlotRefS = 233, kSlotRefR = 234, kSlotRefLam = 235;
+              kSlotNsT = 73, kSlotS64 = 74, kSlotMix = 75, kSlotEng32 = 80;
 
 unsigned grid_for(int64_t n) {
   return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256,
@@ -404,142 +402,6 @@ __global__ __launch_bounds__(256) void left_finish(
   if (blockIdx.x == 0)
     for (int64_t j = threadIdx.x; j < k; j += blockDim.x)
       d.lamM[j] = s[j] * inv;
-}
-
-// ---- chosen form: first-order refinement of the FP32 vectors -------------
-// The FP32 sweeps leave V = V_true (I + dV) with |dV_ij| about
-// 1e-6 sigma^2 / (sigma_j^2 - sigma_i^2): the pairs next to the cap mix kept
-// and discarded directions by 1e-4 and more, and those few pairs carry the
-// form's error.  One step of Ogita and Aishima's iteration (Japan J. Indust.
-// Appl. Math. 35 (2018) 1007) in FP64 on the whole FP32 basis removes the
-// first order: with S = V^H theta^H theta V, R = I - V^H V and
-// lambda_i = S_ii / (1 - R_ii),
-//   E_ij = (S_ij + lambda_j R_ij) / (lambda_j - lambda_i),  E_jj = R_jj / 2,
-//   V_k <- V_k + V E_k.
-// Only the kept columns of S, R and E are formed.  Pairs too close for the
-// first order (|E_ij| above kRefineMax) only have their inner product
-// removed, E_ij = R_ij / 2; Newton-Schulz steps then take the second order
-// out of V^H V.
-// Measured on the 40-qubit depth-20 chi-256 Haar circuit: amplitudes within
-// 7e-7 of FP64 against 6e-5 to 9e-5 without the step (chi 173: 9e-7), for five
-// products of two-site size per gate.
-constexpr double kRefineMax = 0.02;
-
-// One gate of the refinement.  theta is M x N, V (N x n, ld N) the FP32
-// basis in FP64 (columns in descending order of the FP32 values; n = min(M,
-// N)), P = theta V (M x n, ld M), S and R n x k.
-struct RefineDesc {
-  int gate;
-  int trans;       // X = theta^H
-  int64_t M, N, n, k, ldx;
-  const double2* X;
-  double2 *V, *P, *S, *R, *Vk;
-  double* lam;     // n values lambda_i
-  double* nrm;     // 3 n squared column norms: V, P, X
-  double* w;       // |theta|^2, kept weight
-};
-
-// V from the FP32 result: X32[:, perm[j]] / sig[j] (trans) or
-// W32[:, perm[j]].  grid (tiles, count).
-__global__ void refine_basis(const RefineDesc* __restrict__ rd,
-                             const float2* __restrict__ X32, int64_t x_sz,
-                             const float2* __restrict__ W32, int64_t w_sz,
-                             int64_t cols_p, const double* __restrict__ sig32,
-                             const int* __restrict__ perm32, int64_t cols32) {
-  const RefineDesc d = rd[blockIdx.y];
-  const double* s = sig32 + (int64_t)d.gate * cols32;
-  const int* pm = perm32 + (int64_t)d.gate * cols32;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-       idx < d.N * d.n; idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t c = idx % d.N, j = idx / d.N;
-    const int64_t col = pm[j];
-    float2 v;
-    double f = 1.0;
-    if (d.trans) {
-      v = X32[d.gate * x_sz + c + d.ldx * col];
-      f = s[j] > 0.0 ? 1.0 / s[j] : 0.0;
-    } else {
-      v = W32[d.gate * w_sz + c + cols_p * col];
-    }
-    d.V[idx] = make_double2(v.x * f, v.y * f);
-  }
-}
-
-// Squared column norms of V, P and X.  One wave per column; grid
-// (ceil(n / 4), 3, count).
-__global__ __launch_bounds__(256) void refine_norms(
-    const RefineDesc* __restrict__ rd) {
-  const RefineDesc d = rd[blockIdx.z];
-  const int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (j >= d.n) return;
-  const int which = blockIdx.y;
-  const int64_t rows = which == 0 ? d.N : which == 1 ? d.M
-                                                     : d.trans ? d.N : d.M;
-  const double2* c = which == 0   ? d.V + d.N * j
-                     : which == 1 ? d.P + d.M * j
-                                  : d.X + d.ldx * j;
-  double acc = 0.0;
-  for (int64_t r = lane; r < rows; r += 64) {
-    const double2 v = c[r];
-    acc += v.x * v.x + v.y * v.y;
-  }
-  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-  if (lane == 0) d.nrm[which * d.n + j] = acc;
-}
-
-// lambda and the weights (kept values smallest first).  grid (count).
-__global__ __launch_bounds__(256) void refine_lambda(
-    const RefineDesc* __restrict__ rd) {
-  const RefineDesc d = rd[blockIdx.x];
-  for (int64_t j = threadIdx.x; j < d.n; j += 256) {
-    const double v = d.nrm[j];
-    d.lam[j] = v > 0.0 ? d.nrm[d.n + j] / v : 0.0;
-  }
-  __shared__ double part[2][4];
-  double tot = 0.0, kw = 0.0;
-  for (int64_t j = threadIdx.x; j < d.n; j += 256) {
-    tot += d.nrm[2 * d.n + j];
-    if (j < d.k) kw += d.lam[j];
-  }
-  for (int off = 32; off > 0; off >>= 1) {
-    tot += __shfl_xor(tot, off, 64);
-    kw += __shfl_xor(kw, off, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    part[0][threadIdx.x >> 6] = tot;
-    part[1][threadIdx.x >> 6] = kw;
-  }
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    const double* q = part[threadIdx.x];
-    d.w[threadIdx.x] = (q[0] + q[1]) + (q[2] + q[3]);
-  }
-}
-
-// S <- E + I.  grid (tiles, count).
-__global__ void refine_rotation(const RefineDesc* __restrict__ rd) {
-  const RefineDesc d = rd[blockIdx.y];
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-       idx < d.n * d.k; idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = idx % d.n, j = idx / d.n;
-    const double lj = d.lam[j];
-    double2 e;
-    if (i == j) {
-      e = make_double2(1.0 + 0.5 * (1.0 - d.R[idx].x), 0.0);
-    } else {
-      const double gap = lj - d.lam[i];
-      const double2 s = d.S[idx];
-      const double2 r = make_double2(-d.R[idx].x, -d.R[idx].y);
-      const double2 num = make_double2(s.x + lj * r.x, s.y + lj * r.y);
-      if (num.x * num.x + num.y * num.y <=
-          kRefineMax * kRefineMax * gap * gap && gap != 0.0)
-        e = make_double2(num.x / gap, num.y / gap);
-      else
-        e = make_double2(0.5 * r.x, 0.5 * r.y);
-    }
-    d.S[idx] = e;
-  }
 }
 
 // ---- learned form: randomized range finder ------------------------------
@@ -1072,128 +934,6 @@ int32_t rand_range_finder(qtn_ctx* ctx, int ng,
   return QTN_OK;
 }
 
-// Host side of a refinement in flight: the descriptors its copies read and
-// the weights (|theta|^2, kept) it returns; valid until the next wait.
-struct RefineHost {
-  std::vector<RefineDesc> rd;
-  std::vector<GemmDesc<double>> products;
-  std::vector<double> w;
-};
-
-// Refines V_k of the gates the FP32 engine decided (src 1; see the
-// refinement's kernels) and queues the read-back of their weights in FP64.
-// X is the batch's FP64 copy of theta^H / theta.
-int32_t refine_vk(qtn_ctx* ctx, int ng, const std::vector<GateDesc>& gd,
-                  const std::vector<int>& src,
-                  const std::vector<int64_t>& kept, const float2* X32,
-                  int64_t x_sz, const float2* W32, int64_t w_sz,
-                  int64_t cols_p, const JacobiEngine& eng32,
-                  RefineHost* host) {
-  hipStream_t s = ctx->stream;
-  std::vector<RefineDesc>& rd = host->rd;
-  int64_t maxM = 0, maxN = 0, maxn = 0, maxk = 0;
-  for (int g = 0; g < ng; ++g) {
-    if (src[g] != 1) continue;
-    RefineDesc d;
-    d.gate = g;
-    d.trans = gd[g].trans;
-    d.M = 2 * gd[g].chiL;
-    d.N = 2 * gd[g].chiR;
-    d.n = std::min(d.M, d.N);
-    d.k = kept[g];
-    d.ldx = gd[g].ldx;
-    d.X = gd[g].X;
-    d.Vk = gd[g].Vk;
-    maxM = std::max(maxM, d.M);
-    maxN = std::max(maxN, d.N);
-    maxn = std::max(maxn, d.n);
-    maxk = std::max(maxk, d.k);
-    rd.push_back(d);
-  }
-  const int cnt = (int)rd.size();
-  if (cnt == 0) return QTN_OK;
-  const int64_t v_sz = maxN * maxn;
-  void *dV, *dP, *dS, *dR, *dl, *dd;
-  QTN_TRY(ctx->buffer(kSlotRefV, (size_t)cnt * v_sz * sizeof(double2), &dV));
-  QTN_TRY(ctx->buffer(kSlotRefP, (size_t)cnt * maxM * maxn * sizeof(double2),
-                      &dP));
-  QTN_TRY(ctx->buffer(kSlotRefS, (size_t)cnt * maxn * maxk * sizeof(double2),
-                      &dS));
-  QTN_TRY(ctx->buffer(kSlotRefR, (size_t)cnt * maxn * maxk * sizeof(double2),
-                      &dR));
-  QTN_TRY(ctx->buffer(kSlotRefLam,
-                      (size_t)cnt * (4 * maxn + 2) * sizeof(double), &dl));
-  QTN_TRY(ctx->buffer(kSlotRef,
-                      (size_t)cnt * (sizeof(RefineDesc) +
-                                     4 * sizeof(GemmDesc<double>)),
-                      &dd));
-  for (int i = 0; i < cnt; ++i) {
-    RefineDesc& d = rd[i];
-    d.V = (double2*)dV + i * v_sz;
-    d.P = (double2*)dP + i * maxM * maxn;
-    d.S = (double2*)dS + i * maxn * maxk;
-    d.R = (double2*)dR + i * maxn * maxk;
-    d.w = (double*)dl + 2 * i;
-    d.lam = (double*)dl + 2 * cnt + i * 4 * maxn;
-    d.nrm = d.lam + maxn;
-  }
-  const double2 one = make_double2(1.0, 0.0), zero = make_double2(0.0, 0.0);
-  auto mm = [&](int64_t m, int64_t n, int64_t k, const double2* A,
-                int64_t lda, const double2* B, int64_t ldb, double2* C,
-                int64_t ldc) {
-    return GemmDesc<double>{m, n, k, one, zero, A, lda, B, ldb, C, ldc};
-  };
-  // the products in the order they run: P (of the transposed X, of the
-  // others), S, R, V_k
-  std::vector<GemmDesc<double>> pt, pn, sd, rr, vk;
-  for (const RefineDesc& d : rd) {
-    if (d.trans)
-      pt.push_back(mm(d.M, d.n, d.N, d.X, d.ldx, d.V, d.N, d.P, d.M));
-    else
-      pn.push_back(mm(d.M, d.n, d.N, d.X, d.ldx, d.V, d.N, d.P, d.M));
-    sd.push_back(mm(d.n, d.k, d.M, d.P, d.M, d.P, d.M, d.S, d.n));
-    rr.push_back(mm(d.n, d.k, d.N, d.V, d.N, d.V, d.N, d.R, d.n));
-    vk.push_back(mm(d.N, d.k, d.n, d.V, d.N, d.S, d.n, d.Vk, d.N));
-  }
-  std::vector<GemmDesc<double>>& all = host->products;
-  for (const auto* v : {&pt, &pn, &sd, &rr, &vk})
-    all.insert(all.end(), v->begin(), v->end());
-  RefineDesc* d_rd = (RefineDesc*)dd;
-  GemmDesc<double>* d_g = (GemmDesc<double>*)(d_rd + cnt);
-  QTN_CHECK_HIP(hipMemcpyAsync(d_rd, rd.data(), cnt * sizeof(RefineDesc),
-                               hipMemcpyHostToDevice, s));
-  QTN_CHECK_HIP(hipMemcpyAsync(d_g, all.data(),
-                               all.size() * sizeof(GemmDesc<double>),
-                               hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(refine_basis, dim3(grid_for(maxN * maxn), (unsigned)cnt),
-                     dim3(256), 0, s, (const RefineDesc*)d_rd, X32, x_sz, W32,
-                     w_sz, cols_p, (const double*)eng32.sig,
-                     (const int*)eng32.perm, eng32.cols_p);
-  QTN_CHECK_HIP(hipGetLastError());
-  QTN_TRY(launch_zgemm_grouped(s, 2, 0, d_g, (int)pt.size(), maxM, maxn));
-  d_g += pt.size();
-  QTN_TRY(launch_zgemm_grouped(s, 0, 0, d_g, (int)pn.size(), maxM, maxn));
-  d_g += pn.size();
-  hipLaunchKernelGGL(refine_norms,
-                     dim3((unsigned)((maxn + 3) / 4), 3, (unsigned)cnt),
-                     dim3(256), 0, s, (const RefineDesc*)d_rd);
-  hipLaunchKernelGGL(refine_lambda, dim3((unsigned)cnt), dim3(256), 0, s,
-                     (const RefineDesc*)d_rd);
-  QTN_CHECK_HIP(hipGetLastError());
-  // S and R of every gate in one launch
-  QTN_TRY(launch_zgemm_grouped(s, 2, 0, d_g, 2 * cnt, maxn, maxk));
-  d_g += 2 * cnt;
-  hipLaunchKernelGGL(refine_rotation,
-                     dim3(grid_for(maxn * maxk), (unsigned)cnt), dim3(256), 0,
-                     s, (const RefineDesc*)d_rd);
-  QTN_CHECK_HIP(hipGetLastError());
-  QTN_TRY(launch_zgemm_grouped(s, 0, 0, d_g, cnt, maxN, maxk));
-  host->w.resize(2 * cnt);
-  QTN_CHECK_HIP(hipMemcpyAsync(host->w.data(), dl, 2 * cnt * sizeof(double),
-                               hipMemcpyDeviceToHost, s));
-  return QTN_OK;
-}
-
 // Gate g acts on sites (sites[g], sites[g] + 1) of state ms[g] with the
 // bond cap chis[g]; the states may differ (one batch over many circuits)
 // but share ctx.
@@ -1469,12 +1209,6 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
       for (int g = 0; g < ng; ++g) n32 += cand[g];
       QTN_TRY(eng32.reserve(ctx, ng, rows_p, cols_p, true, n32));
       eng32.chimax_per = chis;
-      // The FP32 vectors are refined to first order in FP64 below, so the
-      // sweeps may stop at scaled off-diagonals of 1e-2 (the 40-qubit chi-256
-      // circuit: 7.6 sweeps per solve instead of 8.5, 290 -> 263 ms, its
-      // amplitudes' error unchanged at 7e-7; 3e-2 would save another 0.3
-      // sweeps, but a chi-173 circuit loses a factor of ten).
-      eng32.conv2_refined = 1e-4;
       QTN_TRY(eng32.run32(ctx, (float2*)dX32, rows_p, x_sz, (float2*)dW32,
                           w_sz, any_w ? wantw.data() : nullptr, nsv.data(),
                           cutoff, 1, 0, 60, &sweeps, cand.data()));
@@ -1515,6 +1249,9 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
       cols_eng = round_up64(c64);
     }
     eng.ldw = cols_p;  // W keeps the batch layout
+    // next to FP32 sweeps, whose rounding every change of a bit before them
+    // draws anew: the rounds that keep those circuits' amplitudes
+    eng.general = chosen || learned;
     int n64 = 0;
     for (int g = 0; g < ng; ++g) n64 += need64[g];
     QTN_TRY(eng.reserve(ctx, ng, rows_eng, cols_eng, false, n64));
@@ -1583,16 +1320,11 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
     QTN_CHECK_HIP(hipGetLastError());
   }
   bool any_fp32 = false;
-  RefineHost refined;
   for (int g = 0; g < ng; ++g) any_fp32 = any_fp32 || src[g] == 1;
   if (chosen || (learned && any_fp32)) {
-    // First-order refinement of the FP32 vectors, then Newton-Schulz in
-    // FP64: V <- V (3 I - V^H V) / 2, three steps take the refinement's
-    // second order below FP64 rounding (two left 2e-12 where many kept
-    // values lie near the FP32 floor).
-    if (any_fp32)
-      QTN_TRY(refine_vk(ctx, ng, gd, src, kept, (const float2*)dX32, x_sz,
-                        (const float2*)dW32, w_sz, cols_p, eng32, &refined));
+    // Newton-Schulz in FP64: V <- V (3 I - V^H V) / 2, three steps take the
+    // FP32 orthogonality error (<~1e-3 on the smallest kept columns) below
+    // FP64 rounding.
     void *dG, *dT;
     const int64_t t_sz = maxN * maxk;
     QTN_TRY(ctx->buffer(kSlotNsG, (size_t)ng * maxk * maxk * sizeof(double2),
@@ -1692,18 +1424,12 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
                        (const int64_t*)d_kept, (const double*)dS64, cols_p);
     QTN_CHECK_HIP(hipGetLastError());
   }
-  QTN_CHECK_HIP(hipStreamSynchronize(s));
-  // discarded weights of the refined gates from the FP64 sums
-  for (size_t i = 0; i < refined.rd.size(); ++i) {
-    const int g = refined.rd[i].gate;
-    total[g] = refined.w[2 * i];
-    disc[g] = std::max(0.0, refined.w[2 * i] - refined.w[2 * i + 1]);
-  }
   for (int g = 0; g < ng; ++g) {
     ms[g]->dims[sites[g]] = kept[g];
     if (kept_out) kept_out[g] = kept[g];
     if (disc_out) disc_out[g] = total[g] > 0 ? disc[g] / total[g] : 0.0;
   }
+  QTN_CHECK_HIP(hipStreamSynchronize(s));
   return QTN_OK;
 }
 

@@ -13,15 +13,17 @@
 //   columns):
 //     1. jac_gram   : G = X_IJ^H X_IJ (32x32) on MFMA, split over row chunks
 //     2. the inner sweep on G (Hermitian 2x2 rotations, Golub & Van Loan
-//                     8.5), accumulating Q: jac_inner in a sweep's first
-//                     round, where every pair of columns is rotated, and
-//                     jac_inner_cross in the others, where only the pairs
-//                     across the two blocks are
+//                     8.5), accumulating Q (jac_inner); a sweep's first
+//                     round rotates every pair of columns, the others only
+//                     the pairs across the two blocks
 //     3. jac_update : X_IJ <- X_IJ Q on MFMA (and W_IJ <- W_IJ Q if vectors
 //                     of the other side are needed)
-//   Problems of at most 512 rows run the three as one launch in the cross
-//   rounds (jac_round_reg), and problems of at most 64 columns are one block
-//   of 64 whose Gram is solved whole (jac_inner_whole).  The pair is skipped when G already meets the tolerance, so convergence
+//   In FP64 the cross rounds take jac_inner_cross instead, or, up to 512
+//   rows, run the three as one launch (jac_round_reg), and problems of at
+//   most 64 columns are one block of 64 whose Gram is solved whole
+//   (jac_inner_whole).  A form that also runs FP32 sweeps keeps the general
+//   kernels in both precisions (JacobiEngine::general).
+//   The pair is skipped when G already meets the tolerance, so convergence
 //   is always decided on a Gram matrix freshly computed from the columns.
 // At convergence sigma_j = |x_j|; X W = U_X diag(sigma) with W unitary.
 // All updates are unitary rotations applied to X, so the singular values are
@@ -79,16 +81,27 @@ struct JT<double> {
     return make_double2(re, im);
   }
   static __device__ __forceinline__ double ab(double x) { return fabs(x); }
-  // 1 / sqrt(x) for the rotation parameters (make_rot): the hardware
-  // v_rsq_f64 estimate (relative error e about 2^-26) and one third-order
-  // step, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2, whose error e^3 is
-  // below FP64 rounding: a shorter dependent chain than the correctly
-  // rounded library sequence or two Newton steps, and the inner sweep is
-  // bound by that chain.  x is positive and normal (the rotation guards it).
+  // Rotation parameters (make_rot): the hardware v_rsq_f64 / v_rcp_f64
+  // estimates refined by two Newton steps each (quadratic convergence from
+  // their ~2^-26 relative error to below FP64 rounding), which shortens the
+  // dependent chain of the inner sweep's rounds against the correctly
+  // rounded library sequences.  Arguments are positive and normal (the
+  // rotation guards them).
   static __device__ __forceinline__ double rsq_r(double x) {
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-x * y, y, 1.0);
-    return fma(y * e, fma(e, 0.375, 0.5), y);
+    double y = __builtin_amdgcn_rsq(x);
+    const double hx = 0.5 * x;
+    y = y * fma(-hx * y, y, 1.5);
+    y = y * fma(-hx * y, y, 1.5);
+    return y;
+  }
+  static __device__ __forceinline__ double sq_r(double x) {
+    return x * rsq_r(x);
+  }
+  static __device__ __forceinline__ double dv_r(double a, double b) {
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(r, fma(-b, r, 1.0), r);
+    r = fma(r, fma(-b, r, 1.0), r);
+    return a * r;
   }
 };
 template <>
@@ -106,12 +119,23 @@ struct JT<float> {
   }
   // The FP32 sweeps only produce candidates that are re-orthogonalised and
   // re-measured in FP64, so the rotation parameters use the one-instruction
-  // hardware form (v_rsq_f32, about 1 ulp) instead of the correctly rounded
-  // library sequence: the inner sweep is bound by
+  // hardware forms (v_rsq_f32, v_sqrt_f32, v_rcp_f32, about 1 ulp) instead
+  // of the correctly rounded library sequences: the inner sweep is bound by
   // its per-round instruction count.
-  static __device__ __forceinline__ float ab(float x) { return fabsf(x); }
-  static __device__ __forceinline__ float rsq_r(float x) {
+  static __device__ __forceinline__ float rsq(float x) {
     return __builtin_amdgcn_rsqf(x);
+  }
+  static __device__ __forceinline__ float sq(float x) {
+    return __builtin_amdgcn_sqrtf(x);
+  }
+  static __device__ __forceinline__ float ab(float x) { return fabsf(x); }
+  static __device__ __forceinline__ float dv(float a, float b) {
+    return a * __builtin_amdgcn_rcpf(b);
+  }
+  static __device__ __forceinline__ float rsq_r(float x) { return rsq(x); }
+  static __device__ __forceinline__ float sq_r(float x) { return sq(x); }
+  static __device__ __forceinline__ float dv_r(float a, float b) {
+    return dv(a, b);
   }
 };
 
@@ -231,37 +255,18 @@ inline int gram_parts(int nchunk) {
 
 // Rotation of the pair (p, q) from the Gram entries a = G_pp, d = G_qq and
 // g = G_pq (Golub & Van Loan 8.5, complex Hermitian form):
-//   J = [[cs, conj(s)], [-s, cs]],  J^H [[a, g], [conj g, d]] J = diag(ap, dq)
-// with the smaller of the two angles.  With h = d - a and
-// r = sqrt(h^2 + 4 |g|^2): cos(2 theta) = |h| / r, so cs^2 = (1 + |h| / r) / 2
-// and s = sign(h) conj(g) / (r cs); t = |g| tan(theta) = |g|^2 / (r cs^2).
-// Two reciprocal square roots in sequence, no division and no |g|.  Computed
-// without branches; a pair that already meets the tolerance (or cannot be
-// rotated, pair_open) gets cs = 1, s = 0, which leaves every entry it
-// touches unchanged bit for bit.
+//   J = [[cs, sn], [-sn e, cs e]], e = e^{-i phi} = conj(g) / |g|,
+// J^H [[a, g], [conj g, d]] J = diag(ap, dq).  With zeta = (d - a) / (2|g|)
+// and tau = |zeta| + sqrt(1 + zeta^2) (so t = tan = sign(zeta) / tau):
+// cs = tau / sqrt(1 + tau^2), sn = sign(zeta) / sqrt(1 + tau^2).  Computed
+// without branches; a pair that already meets the tolerance (or has a
+// column below the zero threshold) gets cs = 1, sn = 0, e = 1, which
+// leaves every entry it touches unchanged bit for bit.
 template <typename R>
 struct Rot {
-  R cs, sx, sy, ap, dq;
+  R cs, sn, er, ei, ap, dq;
   bool on;
 };
-
-// Whether a pair can be rotated, and the product a d its off-diagonal is
-// scaled by.  FP64: both columns above the zero threshold zt.  FP32: one of
-// them, with the other's norm taken as the threshold at least: a column
-// below the FP32 floor has no direction of its own, but what it shares with
-// a large column is resolved, and left in place it would stay in the kept
-// vectors (up to the floor, 2e-5 |X|_F, per column).
-template <typename R>
-__device__ __forceinline__ bool pair_open(R a, R d, R zt) {
-  if (sizeof(R) == sizeof(float)) return a > zt || d > zt;
-  return a > zt && d > zt;
-}
-template <typename R>
-__device__ __forceinline__ R pair_scale(R a, R d, R zt) {
-  if (sizeof(R) == sizeof(float))
-    return (a > zt ? a : zt) * (d > zt ? d : zt);
-  return a * d;
-}
 
 template <typename R>
 __device__ __forceinline__ Rot<R> make_rot(R a, R d,
@@ -269,47 +274,48 @@ __device__ __forceinline__ Rot<R> make_rot(R a, R d,
                                            R tol2) {
   Rot<R> o;
   const R absc2 = g.x * g.x + g.y * g.y;
-  o.on = pair_open<R>(a, d, zt) && absc2 > tol2 * pair_scale<R>(a, d, zt);
-  const R h = d - a;
-  const R ir = JT<R>::rsq_r(o.on ? h * h + (R)4 * absc2 : (R)1);
-  const R c2 = o.on ? (R)0.5 + (R)0.5 * JT<R>::ab(h) * ir : (R)1;
-  const R ic = JT<R>::rsq_r(c2);
-  const R f = h >= (R)0 ? ir * ic : -(ir * ic);
-  const R t = absc2 * f * ic;
-  o.cs = o.on ? c2 * ic : (R)1;
-  o.sx = o.on ? g.x * f : (R)0;
-  o.sy = o.on ? -g.y * f : (R)0;
-  o.ap = o.on ? a - t : a;
-  o.dq = o.on ? d + t : d;
+  o.on = (a > zt && d > zt && absc2 > tol2 * a * d);
+  const R s2 = o.on ? absc2 : (R)1;
+  const R inv = JT<R>::rsq_r(s2);
+  const R absc = s2 * inv;
+  const R zeta = (R)0.5 * (d - a) * inv;
+  const R tau = JT<R>::ab(zeta) + JT<R>::sq_r((R)1 + zeta * zeta);
+  const R rr = JT<R>::rsq_r((R)1 + tau * tau);
+  const R sgn = zeta >= (R)0 ? (R)1 : (R)-1;
+  const R tt = JT<R>::dv_r(sgn, tau);
+  o.cs = o.on ? tau * rr : (R)1;
+  o.sn = o.on ? sgn * rr : (R)0;
+  o.er = o.on ? g.x * inv : (R)1;
+  o.ei = o.on ? -g.y * inv : (R)0;
+  o.ap = o.on ? a - tt * absc : a;
+  o.dq = o.on ? d + tt * absc : d;
   return o;
 }
 
 // [u v] <- [u v] J (a row of two entries in the columns p, q of the pair)
 template <typename R>
-__device__ __forceinline__ void rot_right(R cs, R sx, R sy,
-                                          typename JT<R>::c_t& u,
-                                          typename JT<R>::c_t& v) {
-  const typename JT<R>::c_t nu =
-      JT<R>::mk(cs * u.x - sx * v.x + sy * v.y,
-                cs * u.y - sx * v.y - sy * v.x);
-  v = JT<R>::mk(cs * v.x + sx * u.x + sy * u.y,
-                cs * v.y + sx * u.y - sy * u.x);
-  u = nu;
-}
-template <typename R>
 __device__ __forceinline__ void rot_right(const Rot<R>& j,
                                           typename JT<R>::c_t& u,
                                           typename JT<R>::c_t& v) {
-  rot_right<R>(j.cs, j.sx, j.sy, u, v);
+  const R yr = j.er * v.x - j.ei * v.y;
+  const R yi = j.er * v.y + j.ei * v.x;
+  const typename JT<R>::c_t nu =
+      JT<R>::mk(j.cs * u.x - j.sn * yr, j.cs * u.y - j.sn * yi);
+  v = JT<R>::mk(j.sn * u.x + j.cs * yr, j.sn * u.y + j.cs * yi);
+  u = nu;
 }
 
-// [u; v] <- J^H [u; v], J^H = [[cs, -conj(s)], [s, cs]]: the right rotation
-// with conj(s)
+// [u; v] <- J^H [u; v], J^H = [[cs, -sn conj(e)], [sn, cs conj(e)]]
 template <typename R>
 __device__ __forceinline__ void rot_left(const Rot<R>& j,
                                          typename JT<R>::c_t& u,
                                          typename JT<R>::c_t& v) {
-  rot_right<R>(j.cs, j.sx, -j.sy, u, v);
+  const R yr = j.er * v.x + j.ei * v.y;
+  const R yi = j.er * v.y - j.ei * v.x;
+  const typename JT<R>::c_t nu =
+      JT<R>::mk(j.cs * u.x - j.sn * yr, j.cs * u.y - j.sn * yi);
+  v = JT<R>::mk(j.sn * u.x + j.cs * yr, j.sn * u.y + j.cs * yi);
+  u = nu;
 }
 
 // Round-robin slots of the inner sweep.  The W indices of the block pair
@@ -413,9 +419,9 @@ __device__ __forceinline__ int inner_solve(
     const int r = idx % W, c = idx / W;
     if (r < c) {
       const R a = Gp[gpos<NP>(r, r)].x, d = Gp[gpos<NP>(c, c)].x;
-      if (pair_open<R>(a, d, zt)) {
+      if (a > zt && d > zt) {
         const c_t g = Gp[gpos<NP>(r, c)];
-        const R o2 = (g.x * g.x + g.y * g.y) / pair_scale<R>(a, d, zt);
+        const R o2 = (g.x * g.x + g.y * g.y) / (a * d);
         omax = fmax(omax, (double)o2);
         // the sweep can only reduce the pairs it rotates
         off = off || (o2 > tol2 && (!cross || (r < NP && c >= NP)));
@@ -502,8 +508,9 @@ __device__ __forceinline__ int inner_solve(
         // the lane of this wave whose column pair is this row pair
         const int src = (lane & ~(NP - 1)) | (pr0 + RS * k);
         jr[k].cs = __shfl(jc.cs, src, 64);
-        jr[k].sx = __shfl(jc.sx, src, 64);
-        jr[k].sy = __shfl(jc.sy, src, 64);
+        jr[k].sn = __shfl(jc.sn, src, 64);
+        jr[k].er = __shfl(jc.er, src, 64);
+        jr[k].ei = __shfl(jc.ei, src, 64);
       }
       // --- transform, then write each entry to its next-round slot
 #pragma unroll
@@ -671,7 +678,7 @@ __global__ __launch_bounds__(256) void jac_inner(
 }
 
 // ---------------------------------------------------------------------------
-// 2a. The inner solve of the cross rounds (every outer round of a sweep but
+// 2a. The FP64 inner solve of the cross rounds (every outer round of a sweep but
 // its first, W = 32): sums the partial Grams and rotates the 16 x 16 pairs
 // across the two column blocks once, in 16 rounds.
 //
@@ -694,47 +701,92 @@ __global__ __launch_bounds__(256) void jac_inner(
 constexpr int kCrossThreads = 512;
 
 // The value of the next lane of a row of 16 (cyclic): dst lane i <- i + 1.
-template <typename R>
-__device__ __forceinline__ R next_in_row(R x) {
+__device__ __forceinline__ double next_in_row(double x) {
   constexpr int kRor15 = 0x12f;  // row_ror:15
-  if constexpr (sizeof(R) == 8) {
-    const int2 v = __builtin_bit_cast(int2, x);
-    const int2 r = make_int2(
-        __builtin_amdgcn_update_dpp(v.x, v.x, kRor15, 0xf, 0xf, false),
-        __builtin_amdgcn_update_dpp(v.y, v.y, kRor15, 0xf, 0xf, false));
-    return __builtin_bit_cast(R, r);
-  } else {
-    const int v = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(
-        R, __builtin_amdgcn_update_dpp(v, v, kRor15, 0xf, 0xf, false));
-  }
+  const int2 v = __builtin_bit_cast(int2, x);
+  return __builtin_bit_cast(
+      double,
+      make_int2(__builtin_amdgcn_update_dpp(v.x, v.x, kRor15, 0xf, 0xf, false),
+                __builtin_amdgcn_update_dpp(v.y, v.y, kRor15, 0xf, 0xf,
+                                            false)));
 }
 
-template <typename R>
+// The rotation of the register-resident kernels (2a, 2b), for the same pair
+// as make_rot's in fewer dependent steps:
+//   J = [[cs, conj(s)], [-s, cs]],  J^H [[a, g], [conj g, d]] J = diag(ap, dq)
+// with the smaller of the two angles.  With h = d - a and
+// r = sqrt(h^2 + 4 |g|^2): cos(2 theta) = |h| / r, so cs^2 = (1 + |h| / r) / 2
+// and s = sign(h) conj(g) / (r cs); t = |g| tan(theta) = |g|^2 / (r cs^2).
+// Two reciprocal square roots in sequence, no division and no |g|.  Computed
+// without branches; a pair that already meets the tolerance (or has a column
+// below the zero threshold) gets cs = 1, s = 0, which leaves every entry it
+// touches unchanged bit for bit.
+struct CrossRot {
+  double cs, sx, sy, ap, dq;
+  bool on;
+};
+
+// 1 / sqrt(x): the hardware v_rsq_f64 estimate (relative error e about 2^-26)
+// and one third-order step, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - x y^2,
+// whose error e^3 is below FP64 rounding: a shorter dependent chain than two
+// Newton steps.  x is positive and normal (the rotation guards it).
+__device__ __forceinline__ double cross_rsq(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
+}
+
+__device__ __forceinline__ CrossRot cross_rot(double a, double d, double2 g,
+                                              double zt, double tol2) {
+  CrossRot o;
+  const double absc2 = g.x * g.x + g.y * g.y;
+  o.on = a > zt && d > zt && absc2 > tol2 * (a * d);
+  const double h = d - a;
+  const double ir = cross_rsq(o.on ? h * h + 4.0 * absc2 : 1.0);
+  const double c2 = o.on ? 0.5 + 0.5 * fabs(h) * ir : 1.0;
+  const double ic = cross_rsq(c2);
+  const double f = h >= 0.0 ? ir * ic : -(ir * ic);
+  const double t = absc2 * f * ic;
+  o.cs = o.on ? c2 * ic : 1.0;
+  o.sx = o.on ? g.x * f : 0.0;
+  o.sy = o.on ? -g.y * f : 0.0;
+  o.ap = o.on ? a - t : a;
+  o.dq = o.on ? d + t : d;
+  return o;
+}
+
+// [u v] <- [u v] J; J^H [u; v] is the same with conj(s) (sy negated).
+__device__ __forceinline__ void cross_apply(double cs, double sx, double sy,
+                                            double2& u, double2& v) {
+  const double2 nu = make_double2(cs * u.x - sx * v.x + sy * v.y,
+                                  cs * u.y - sx * v.y - sy * v.x);
+  v = make_double2(cs * v.x + sx * u.x + sy * u.y,
+                   cs * v.y + sx * u.y - sy * u.x);
+  u = nu;
+}
+
 struct CrossShared {
-  typename JT<R>::c_t exch[2][2][256];  // side-1 rows on the move
-  R prm[2][4][16];                      // cs, sx, sy, dq per column pair
-  R dg[32];                             // diagonal of the summed Gram
+  double2 exch[2][2][256];  // side-1 rows on the move
+  double prm[2][4][16];     // cs, sx, sy, dq per column pair
+  double dg[32];            // diagonal of the summed Gram
   int off, big, rot;
 };
 
 // The 16 rounds.  b: this thread's block of G (waves 0-3) or rows of Q
 // (waves 4-7), in the order (row side, column side); P, c its place.
 // Returns the rotations this thread derived.
-template <typename R>
-__device__ __forceinline__ int cross_rounds(CrossShared<R>& sh,
-                                            typename JT<R>::c_t (&b)[4],
-                                            bool is_g, int P, int c, R zt,
-                                            R tol2) {
+__device__ __forceinline__ int cross_rounds(CrossShared& sh, double2 (&b)[4],
+                                            bool is_g, int P, int c, double zt,
+                                            double tol2) {
   const bool owner = is_g && P == c;
   const int at = P * 16 + c, from = ((P + 1) & 15) * 16 + c;
-  R d = b[3].x;
+  double d = b[3].x;
   int rot = 0;
   for (int t = 0; t < 16; ++t) {
     const int cur = t & 1;
-    Rot<R> o;
+    CrossRot o;
     if (is_g) {
-      o = make_rot<R>(b[0].x, d, b[1], zt, tol2);
+      o = cross_rot(b[0].x, d, b[1], zt, tol2);
       if (owner) {
         sh.prm[cur][0][c] = o.cs;
         sh.prm[cur][1][c] = o.sx;
@@ -744,33 +796,33 @@ __device__ __forceinline__ int cross_rounds(CrossShared<R>& sh,
       }
     }
     __syncthreads();
-    const R cs = sh.prm[cur][0][c], sx = sh.prm[cur][1][c],
+    const double cs = sh.prm[cur][0][c], sx = sh.prm[cur][1][c],
             sy = sh.prm[cur][2][c];
     if (is_g) {
-      const R rc = sh.prm[cur][0][P], rx = sh.prm[cur][1][P],
+      const double rc = sh.prm[cur][0][P], rx = sh.prm[cur][1][P],
               ry = sh.prm[cur][2][P];
       d = sh.prm[cur][3][(c + 1) & 15];
       if (t > 0) {
         b[2] = sh.exch[cur ^ 1][0][from];
         b[3] = sh.exch[cur ^ 1][1][from];
       }
-      rot_right<R>(cs, sx, sy, b[0], b[1]);
-      rot_right<R>(cs, sx, sy, b[2], b[3]);
-      rot_right<R>(rc, rx, -ry, b[0], b[2]);
-      rot_right<R>(rc, rx, -ry, b[1], b[3]);
+      cross_apply(cs, sx, sy, b[0], b[1]);
+      cross_apply(cs, sx, sy, b[2], b[3]);
+      cross_apply(rc, rx, -ry, b[0], b[2]);
+      cross_apply(rc, rx, -ry, b[1], b[3]);
       if (owner && o.on) {
-        b[0] = JT<R>::mk(o.ap, (R)0);
-        b[1] = JT<R>::mk((R)0, (R)0);
-        b[2] = JT<R>::mk((R)0, (R)0);
-        b[3] = JT<R>::mk(o.dq, (R)0);
+        b[0] = make_double2(o.ap, 0.0);
+        b[1] = make_double2(0.0, 0.0);
+        b[2] = make_double2(0.0, 0.0);
+        b[3] = make_double2(o.dq, 0.0);
       }
     } else {
-      rot_right<R>(cs, sx, sy, b[0], b[1]);
-      rot_right<R>(cs, sx, sy, b[2], b[3]);
+      cross_apply(cs, sx, sy, b[0], b[1]);
+      cross_apply(cs, sx, sy, b[2], b[3]);
     }
     // side-1 columns to the next round's pair
-    b[1] = JT<R>::mk(next_in_row(b[1].x), next_in_row(b[1].y));
-    b[3] = JT<R>::mk(next_in_row(b[3].x), next_in_row(b[3].y));
+    b[1] = make_double2(next_in_row(b[1].x), next_in_row(b[1].y));
+    b[3] = make_double2(next_in_row(b[3].x), next_in_row(b[3].y));
     if (is_g) {
       sh.exch[cur][0][at] = b[2];
       sh.exch[cur][1][at] = b[3];
@@ -782,29 +834,26 @@ __device__ __forceinline__ int cross_rounds(CrossShared<R>& sh,
 // Is there a cross pair to rotate (the sweep reduces no others)?  Also
 // records whether any pair lies above conv2 (the problem needs another
 // sweep).  Called by the whole workgroup with sh.dg set and visible.
-template <typename R>
-__device__ __forceinline__ bool cross_check(CrossShared<R>& sh,
-                                            const typename JT<R>::c_t (&b)[4],
-                                            bool is_g, int P, int c, R zt,
-                                            R tol2, R conv2,
+__device__ __forceinline__ bool cross_check(CrossShared& sh,
+                                            const double2 (&b)[4], bool is_g,
+                                            int P, int c, double zt,
+                                            double tol2, double conv2,
                                             double* offmax_bz) {
   if (is_g) {
-    const R a0 = sh.dg[P], a1 = sh.dg[c], d0 = sh.dg[16 + P],
+    const double a0 = sh.dg[P], a1 = sh.dg[c], d0 = sh.dg[16 + P],
             d1 = sh.dg[16 + c];
-    const R n0 = b[0].x * b[0].x + b[0].y * b[0].y,
+    const double n0 = b[0].x * b[0].x + b[0].y * b[0].y,
             n1 = b[1].x * b[1].x + b[1].y * b[1].y,
             n3 = b[3].x * b[3].x + b[3].y * b[3].y;
     bool big = false, off = false;
-    if (pair_open<R>(a0, d1, zt)) {
-      const R sc = pair_scale<R>(a0, d1, zt);
+    if (a0 > zt && d1 > zt) {
+      const double sc = a0 * d1;
       off = n1 > tol2 * sc;
       big = n1 > conv2 * sc;
     }
     if (P != c) {
-      big = big || (pair_open<R>(a0, a1, zt) &&
-                    n0 > conv2 * pair_scale<R>(a0, a1, zt));
-      big = big || (pair_open<R>(d0, d1, zt) &&
-                    n3 > conv2 * pair_scale<R>(d0, d1, zt));
+      big = big || (a0 > zt && a1 > zt && n0 > conv2 * (a0 * a1)) ||
+            (d0 > zt && d1 > zt && n3 > conv2 * (d0 * d1));
     }
     if (off) sh.off = 1;
     if (big) sh.big = 1;
@@ -818,14 +867,12 @@ __device__ __forceinline__ bool cross_check(CrossShared<R>& sh,
 }
 
 // n_inner sweeps of 16 rounds; returns the rotations this thread derived.
-template <typename R>
-__device__ __forceinline__ int cross_sweeps(CrossShared<R>& sh,
-                                            typename JT<R>::c_t (&b)[4],
-                                            bool is_g, int P, int c, R zt,
-                                            R tol2, int n_inner) {
+__device__ __forceinline__ int cross_sweeps(CrossShared& sh, double2 (&b)[4],
+                                            bool is_g, int P, int c, double zt,
+                                            double tol2, int n_inner) {
   int rot = 0;
   for (int sweep = 0; sweep < n_inner; ++sweep) {
-    rot += cross_rounds<R>(sh, b, is_g, P, c, zt, tol2);
+    rot += cross_rounds(sh, b, is_g, P, c, zt, tol2);
     if (sweep + 1 < n_inner) {
       // the rows still on the move, for the next sweep
       __syncthreads();
@@ -842,38 +889,36 @@ __device__ __forceinline__ int cross_sweeps(CrossShared<R>& sh,
 
 // grid (p, batch), kCrossThreads threads; arguments as jac_inner's (Q leaves
 // row by row).
-template <typename R>
 __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
-    const typename JT<R>::c_t* __restrict__ Gp, int nchunk, int p,
+    const double2* __restrict__ Gp, int nchunk, int p,
     double tol, double conv2, const double* __restrict__ zthr, int n_inner,
-    typename JT<R>::c_t* __restrict__ Qout, int* __restrict__ flags,
+    double2* __restrict__ Qout, int* __restrict__ flags,
     int* __restrict__ counters, const int* __restrict__ active,
     double* __restrict__ offmax, int* __restrict__ qpairs,
     const int* __restrict__ want, int w_mode) {
-  using c_t = typename JT<R>::c_t;
   constexpr int W = 32;
   const int bz = blockIdx.y, pi = blockIdx.x;
   if (!active[bz]) return;
-  __shared__ CrossShared<R> sh;
+  __shared__ CrossShared sh;
   const int tid = threadIdx.x;
   const bool is_g = __builtin_amdgcn_readfirstlane(tid >> 6) < 4;
   const int P = (tid & 255) >> 4, c = tid & 15;
-  const R zt = (R)zthr[bz];
-  const R tol2 = (R)(tol * tol);
-  c_t b[4];
+  const double zt = zthr[bz];
+  const double tol2 = tol * tol;
+  double2 b[4];
   if (is_g) {
     // entries (P, c), (P, 16 + c), (16 + P, c), (16 + P, 16 + c): the
     // partial Grams hold the first, the second and the last; all but the
     // second are read as the adjoint, along consecutive rows
-    const c_t* src =
+    const double2* src =
         Gp + ((int64_t)bz * p + pi) * nchunk * (int64_t)(W * W);
     const int a0 = c + W * P, a1 = P + W * (16 + c), a2 = c + W * (16 + P),
               a3 = 16 + c + W * (16 + P);
-    R re[4] = {0, 0, 0, 0}, im[4] = {0, 0, 0, 0};
+    double re[4] = {0, 0, 0, 0}, im[4] = {0, 0, 0, 0};
 #pragma unroll 8
     for (int ch = 0; ch < nchunk; ++ch) {
-      const c_t* g = src + (int64_t)ch * (W * W);
-      const c_t v0 = g[a0], v1 = g[a1], v2 = g[a2], v3 = g[a3];
+      const double2* g = src + (int64_t)ch * (W * W);
+      const double2 v0 = g[a0], v1 = g[a1], v2 = g[a2], v3 = g[a3];
       re[0] += v0.x;
       im[0] -= v0.y;
       re[1] += v1.x;
@@ -884,7 +929,7 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
       im[3] -= v3.y;
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) b[u] = JT<R>::mk(re[u], im[u]);
+    for (int u = 0; u < 4; ++u) b[u] = make_double2(re[u], im[u]);
     if (P == c) {
       sh.dg[c] = re[0];
       sh.dg[16 + c] = re[3];
@@ -894,8 +939,8 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
     const int r = 2 * P;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      b[u] = JT<R>::mk(r + (u >> 1) == ((u & 1) ? 16 + c : c) ? (R)1 : (R)0,
-                       (R)0);
+      b[u] = make_double2(r + (u >> 1) == ((u & 1) ? 16 + c : c) ? 1.0 : 0.0,
+                          0.0);
   }
   if (tid == 0) {
     sh.off = 0;
@@ -903,11 +948,11 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
     sh.rot = 0;
   }
   __syncthreads();
-  if (!cross_check<R>(sh, b, is_g, P, c, zt, tol2, (R)conv2, &offmax[bz])) {
+  if (!cross_check(sh, b, is_g, P, c, zt, tol2, conv2, &offmax[bz])) {
     if (tid == 0) flags[bz * p + pi] = 0;
     return;
   }
-  const int rot = cross_sweeps<R>(sh, b, is_g, P, c, zt, tol2, n_inner);
+  const int rot = cross_sweeps(sh, b, is_g, P, c, zt, tol2, n_inner);
   if (rot) atomicAdd(&sh.rot, rot);
   __syncthreads();
   const int total = sh.rot;
@@ -921,7 +966,7 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
     }
   }
   if (total == 0 || is_g) return;
-  c_t* q = Qout + ((int64_t)bz * p + pi) * (int64_t)(W * W) + 2 * P * W;
+  double2* q = Qout + ((int64_t)bz * p + pi) * (int64_t)(W * W) + 2 * P * W;
   q[c] = b[0];
   q[16 + c] = b[1];
   q[W + c] = b[2];
@@ -929,7 +974,7 @@ __global__ __launch_bounds__(kCrossThreads) void jac_inner_cross(
 }
 
 // ---------------------------------------------------------------------------
-// 2b. The inner solve of a problem that is one block pair (at most 64
+// 2b. The FP64 inner solve of a problem that is one block pair (at most 64
 // columns): sweeps to convergence on the whole Gram.  The cyclic order runs
 // over the columns that are there: np = ceil(eff / 2) slot pairs for the
 // eff leading columns up to the last one that can be rotated (padding never
@@ -951,20 +996,18 @@ constexpr int kWholeThreads = 1024;
 // them at O(conv2): the fresh Gram of the next outer pass decides), or
 // max_sweeps.  Called by the whole workgroup; the first NP^2 threads own the
 // blocks.  Returns the rotations made; the final Q planes are Qc's.
-template <typename R, int NP>
-__device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
-                                            typename JT<R>::c_t* Gn,
-                                            typename JT<R>::c_t*& Qc, int np,
-                                            R zt, R tol2, R conv2,
+template <int NP>
+__device__ __forceinline__ int whole_sweeps(double2* Gc, double2* Gn,
+                                            double2*& Qc, int np, double zt,
+                                            double tol2, double conv2,
                                             int max_sweeps, int* big,
                                             int* nrot) {
-  using c_t = typename JT<R>::c_t;
   constexpr int NBLK = NP * NP;
   const int tid = threadIdx.x, lane = tid & 63;
   const int P = tid / NP, pc = tid % NP;
   const bool mine = tid < NBLK && P < np && pc < np;
   const int blk = P * NP + pc;
-  c_t* Qp = Qc;
+  double2* Qp = Qc;
   auto next = [&](int a, int side) {  // slot_next on np pairs
     if (np == 1) return side;
     if (side == 0)
@@ -984,7 +1027,7 @@ __device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
     for (int q = 0; q < 4; ++q) {
       const int idx = (q & 1) ? 2 * np - 1 - pc : pc;
       Qp[q * NBLK + blk] =
-          JT<R>::mk(2 * P + (q >> 1) == idx ? (R)1 : (R)0, (R)0);
+          make_double2(2 * P + (q >> 1) == idx ? 1.0 : 0.0, 0.0);
     }
   }
   if (tid == 0) *nrot = 0;
@@ -995,9 +1038,9 @@ __device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
     __syncthreads();
     bool any_big = false;
     for (int round = 0; round < 2 * np - 1; ++round) {
-      c_t b[4], q[4];
-      R ga = 0, gdd = 0;
-      c_t gg = JT<R>::mk((R)0, (R)0);
+      double2 b[4], q[4];
+      double ga = 0, gdd = 0;
+      double2 gg = make_double2(0.0, 0.0);
       if (mine) {
         const int dcol = pc * (NP + 1);
         ga = Gc[dcol].x;
@@ -1011,29 +1054,29 @@ __device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
       }
       if (!dbuf) __syncthreads();
       else __builtin_amdgcn_wave_barrier();
-      const Rot<R> jc = make_rot<R>(ga, gdd, gg, zt, tol2);
-      Rot<R> jr;
+      const CrossRot jc = cross_rot(ga, gdd, gg, zt, tol2);
+      CrossRot jr;
       const int src = (lane & ~(NP - 1)) | (P & (NP - 1));
       jr.cs = __shfl(jc.cs, src, 64);
       jr.sx = __shfl(jc.sx, src, 64);
       jr.sy = __shfl(jc.sy, src, 64);
       if (mine) {
-        rot_right<R>(jc, b[0], b[1]);
-        rot_right<R>(jc, b[2], b[3]);
-        rot_left<R>(jr, b[0], b[2]);
-        rot_left<R>(jr, b[1], b[3]);
+        cross_apply(jc.cs, jc.sx, jc.sy, b[0], b[1]);
+        cross_apply(jc.cs, jc.sx, jc.sy, b[2], b[3]);
+        cross_apply(jr.cs, jr.sx, -jr.sy, b[0], b[2]);
+        cross_apply(jr.cs, jr.sx, -jr.sy, b[1], b[3]);
         if (P == pc && jc.on) {
           any_big = any_big ||
                     gg.x * gg.x + gg.y * gg.y >
-                        conv2 * pair_scale<R>(ga, gdd, zt);
-          b[0] = JT<R>::mk(jc.ap, (R)0);
-          b[1] = JT<R>::mk((R)0, (R)0);
-          b[2] = JT<R>::mk((R)0, (R)0);
-          b[3] = JT<R>::mk(jc.dq, (R)0);
+                        conv2 * (ga * gdd);
+          b[0] = make_double2(jc.ap, 0.0);
+          b[1] = make_double2(0.0, 0.0);
+          b[2] = make_double2(0.0, 0.0);
+          b[3] = make_double2(jc.dq, 0.0);
           ++rot;
         }
-        rot_right<R>(jc, q[0], q[1]);
-        rot_right<R>(jc, q[2], q[3]);
+        cross_apply(jc.cs, jc.sx, jc.sy, q[0], q[1]);
+        cross_apply(jc.cs, jc.sx, jc.sy, q[2], q[3]);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           Gn[gd[u]] = b[u];
@@ -1041,7 +1084,7 @@ __device__ __forceinline__ int whole_sweeps(typename JT<R>::c_t* Gc,
         }
       }
       __syncthreads();
-      c_t* t = Gc;
+      double2* t = Gc;
       Gc = Gn;
       Gn = t;
     }
@@ -1071,42 +1114,40 @@ __device__ __forceinline__ int qpos_n(int r, int c, int np) {
 }
 
 // grid (1, batch), kWholeThreads threads; arguments as jac_inner's.
-template <typename R>
 __global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
-    const typename JT<R>::c_t* __restrict__ Gp, int nchunk, double tol,
+    const double2* __restrict__ Gp, int nchunk, double tol,
     double conv2, const double* __restrict__ zthr, int max_sweeps,
-    typename JT<R>::c_t* __restrict__ Qout, int* __restrict__ flags,
+    double2* __restrict__ Qout, int* __restrict__ flags,
     int* __restrict__ counters, const int* __restrict__ active,
     double* __restrict__ offmax, int* __restrict__ qpairs,
     const int* __restrict__ want, int w_mode) {
-  using c_t = typename JT<R>::c_t;
   constexpr int W = 64, IPT = W * W / kWholeThreads;
   const int bz = blockIdx.y;
   if (!active[bz]) return;
-  __shared__ c_t pool[2 * W * W];
-  __shared__ R dg[W];
+  __shared__ double2 pool[2 * W * W];
+  __shared__ double dg[W];
   __shared__ int s_eff, s_off, s_big, s_rot;
   __shared__ double wmax[kWholeThreads / 64];
   const int tid = threadIdx.x;
-  const R zt = (R)zthr[bz];
-  const R tol2 = (R)(tol * tol);
-  const c_t* src = Gp + (int64_t)bz * nchunk * (W * W);
+  const double zt = zthr[bz];
+  const double tol2 = tol * tol;
+  const double2* src = Gp + (int64_t)bz * nchunk * (W * W);
   // the lower-left quadrant of the partial Grams is not filled (jac_gram):
   // its entries are the adjoints of the upper-right one
-  c_t g[IPT];
+  double2 g[IPT];
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
     const int idx = tid + kWholeThreads * i;
     const int r = idx % W, c = idx / W;
     const bool ll = r >= W / 2 && c < W / 2;
     const int at = ll ? c + W * r : idx;
-    R re = 0, im = 0;
+    double re = 0, im = 0;
     for (int ch = 0; ch < nchunk; ++ch) {
-      const c_t v = src[(int64_t)ch * (W * W) + at];
+      const double2 v = src[(int64_t)ch * (W * W) + at];
       re += v.x;
       im += v.y;
     }
-    g[i] = JT<R>::mk(re, ll ? -im : im);
+    g[i] = make_double2(re, ll ? -im : im);
     if (r == c) dg[r] = re;
   }
   if (tid == 0) {
@@ -1114,8 +1155,7 @@ __global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
     s_off = 0;
   }
   __syncthreads();
-  if (tid < W && dg[tid] > (sizeof(R) == sizeof(float) ? (R)0 : zt))
-    atomicMax(&s_eff, tid + 1);
+  if (tid < W && dg[tid] > zt) atomicMax(&s_eff, tid + 1);
   // largest scaled off-diagonal, and whether any pair needs a rotation
   double omax = 0.0;
   bool off = false;
@@ -1123,9 +1163,9 @@ __global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
   for (int i = 0; i < IPT; ++i) {
     const int idx = tid + kWholeThreads * i;
     const int r = idx % W, c = idx / W;
-    if (r < c && pair_open<R>(dg[r], dg[c], zt)) {
-      const R o2 = (g[i].x * g[i].x + g[i].y * g[i].y) /
-                   pair_scale<R>(dg[r], dg[c], zt);
+    if (r < c && dg[r] > zt && dg[c] > zt) {
+      const double o2 = (g[i].x * g[i].x + g[i].y * g[i].y) /
+                        (dg[r] * dg[c]);
       omax = fmax(omax, (double)o2);
       off = off || o2 > tol2;
     }
@@ -1158,14 +1198,14 @@ __global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
     if (r < 2 * np && c < 2 * np)
       pool[narrow ? gpos_n<16>(r, c, np) : gpos_n<32>(r, c, np)] = g[i];
   }
-  c_t* Qp = narrow ? pool + 2048 : pool + W * W;
+  double2* Qp = narrow ? pool + 2048 : pool + W * W;
   int total;
   if (narrow)
-    total = whole_sweeps<R, 16>(pool, pool + 1024, Qp, np, zt, tol2,
-                                (R)conv2, max_sweeps, &s_big, &s_rot);
+    total = whole_sweeps<16>(pool, pool + 1024, Qp, np, zt, tol2, conv2,
+                             max_sweeps, &s_big, &s_rot);
   else
-    total = whole_sweeps<R, 32>(pool, pool, Qp, np, zt, tol2, (R)conv2,
-                                max_sweeps, &s_big, &s_rot);
+    total = whole_sweeps<32>(pool, pool, Qp, np, zt, tol2, conv2, max_sweeps,
+                             &s_big, &s_rot);
   if (tid == 0) {
     flags[bz] = total > 0 ? 1 : 0;
     if (total > 0) {
@@ -1175,12 +1215,12 @@ __global__ __launch_bounds__(kWholeThreads) void jac_inner_whole(
     }
   }
   if (total == 0) return;
-  c_t* q = Qout + (int64_t)bz * (W * W);
+  double2* q = Qout + (int64_t)bz * (W * W);
 #pragma unroll
   for (int i = 0; i < IPT; ++i) {
     const int idx = tid + kWholeThreads * i;
     const int r = idx / W, c = idx % W;
-    c_t v = JT<R>::mk(r == c ? (R)1 : (R)0, (R)0);
+    double2 v = make_double2(r == c ? 1.0 : 0.0, 0.0);
     if (r < 2 * np && c < 2 * np)
       v = Qp[narrow ? qpos_n<16>(r, c, np) : qpos_n<32>(r, c, np)];
     q[idx] = v;
@@ -1801,7 +1841,7 @@ __global__ __launch_bounds__(256) void jac_round_res(
 }
 
 // ---------------------------------------------------------------------------
-// The fused cross round with the block pair in registers (at most 512 rows,
+// The fused FP64 cross round, the block pair in registers (at most 512 rows,
 // W = 32): one workgroup of 512 threads per block pair streams X_IJ twice,
 // both times straight into MFMA operand registers -- once in the Gram's
 // layout (lane l: column l % 16, row 4 s + l / 16), once, behind the 16
@@ -1826,10 +1866,10 @@ __global__ __launch_bounds__(256) void jac_round_res(
 
 // Y = X Q for the tiles of this wave, in place: rows x 32 columns (blocks I
 // and J) of X; x holds the tiles' columns in the update's layout.
-template <typename R, int NT>
+template <int NT>
 __device__ __forceinline__ void reg_load(
-    const typename JT<R>::c_t* __restrict__ X, int64_t ldx, int ntiles, int I,
-    int J, int wave, typename JT<R>::c_t (&x)[NT][8]) {
+    const double2* __restrict__ X, int64_t ldx, int ntiles, int I,
+    int J, int wave, double2 (&x)[NT][8]) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
@@ -1839,70 +1879,66 @@ __device__ __forceinline__ void reg_load(
       x[i][s] = X[r0 + pair_col<32>(4 * s + (lane >> 4), I, J) * ldx];
   }
 }
-template <typename R, int NT>
+template <int NT>
 __device__ __forceinline__ void reg_update(
-    typename JT<R>::c_t* __restrict__ X, int64_t ldx, int ntiles, int I,
-    int J, int wave, const typename JT<R>::c_t (&x)[NT][8],
-    const R (*Q0)[33], const R (*Q1)[33], const R (*Q2)[33]) {
-  using acc_t = typename JT<R>::acc_t;
+    double2* __restrict__ X, int64_t ldx, int ntiles, int I,
+    int J, int wave, const double2 (&x)[NT][8],
+    const double (*Q0)[33], const double (*Q1)[33], const double (*Q2)[33]) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     if (wave + 8 * i >= ntiles) break;
-    acc_t k1[2], k2[2], k3[2];
+    d4_t k1[2], k2[2], k3[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) k1[j][e] = k2[j][e] = k3[j][e] = (R)0;
+      for (int e = 0; e < 4; ++e) k1[j][e] = k2[j][e] = k3[j][e] = 0.0;
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const int k = 4 * s + (lane >> 4);
-      const R xr = x[i][s].x, xi = x[i][s].y, xs = xr + xi;
+      const double xr = x[i][s].x, xi = x[i][s].y, xs = xr + xi;
 #pragma unroll
       for (int j = 0; j < 2; ++j) {
         const int n = 16 * j + (lane & 15);
-        k1[j] = JT<R>::mfma(Q0[k][n], xs, k1[j]);
-        k2[j] = JT<R>::mfma(Q1[k][n], xr, k2[j]);
-        k3[j] = JT<R>::mfma(Q2[k][n], xi, k3[j]);
+        k1[j] = JT<double>::mfma(Q0[k][n], xs, k1[j]);
+        k2[j] = JT<double>::mfma(Q1[k][n], xr, k2[j]);
+        k3[j] = JT<double>::mfma(Q2[k][n], xi, k3[j]);
       }
       // keep the compiler from reading every Q ahead (registers are full)
-      if (sizeof(R) == 8 && (s & 1)) __builtin_amdgcn_sched_barrier(0);
+      if (s & 1) __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int e = 0; e < 4; ++e)
         X[16 * (wave + 8 * i) + (lane & 15) +
-          pair_col<32>(16 * j + JT<R>::row(lane, e), I, J) * ldx] =
-            JT<R>::mk(k1[j][e] - k3[j][e], k1[j][e] + k2[j][e]);
+          pair_col<32>(16 * j + JT<double>::row(lane, e), I, J) * ldx] =
+            make_double2(k1[j][e] - k3[j][e], k1[j][e] + k2[j][e]);
   }
 }
 
-template <typename R>
 struct RegShared {
-  CrossShared<R> cross;
+  CrossShared cross;
   union {
-    R part[4][24][64];  // partial Grams of four waves
+    double part[4][24][64];  // partial Grams of four waves
     struct {
-      R sum[24][64];    // their sum
+      double sum[24][64];    // their sum
       // c, d - c and c + d of Q = c + i d
-      R Q0[32][33], Q1[32][33], Q2[32][33];
+      double Q0[32][33], Q1[32][33], Q2[32][33];
     } s;
   };
 };
 
-template <typename R, int NT>
+template <int NT>
 __global__ __launch_bounds__(kCrossThreads)
-__attribute__((amdgpu_waves_per_eu(sizeof(R) * NT <= 8 ? 4 : 2)))
+__attribute__((amdgpu_waves_per_eu(NT <= 1 ? 4 : 2)))
 void jac_round_reg(
-    typename JT<R>::c_t* __restrict__ X, int64_t ldx, int64_t sX,
-    int nchunk_x, typename JT<R>::c_t* __restrict__ Wm, int64_t ldw,
+    double2* __restrict__ X, int64_t ldx, int64_t sX,
+    int nchunk_x, double2* __restrict__ Wm, int64_t ldw,
     int64_t sW, int nchunk_w, const int* __restrict__ want, int p, int round,
     double tol, double conv2, const double* __restrict__ zthr, int n_inner,
     int* __restrict__ counters, const int* __restrict__ active,
     double* __restrict__ offmax, int* __restrict__ qpairs) {
-  using c_t = typename JT<R>::c_t;
-  using acc_t = typename JT<R>::acc_t;
   const int bz = blockIdx.y, pi = blockIdx.x;
   if (!active[bz]) return;
   const int nb = 2 * p;
@@ -1910,16 +1946,16 @@ void jac_round_reg(
   const int b2 = rr_block(nb - 1 - pi, round, nb);
   const int I = min(b1, b2), J = max(b1, b2);
   X += (int64_t)bz * sX;
-  __shared__ RegShared<R> sh;
+  __shared__ RegShared sh;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ntiles = 4 * nchunk_x;
 
   // 1. Gram of the wave's tiles
   {
-    c_t v[NT][4][2];
-    const c_t* c0 = X + pair_col<32>(lane & 15, I, J) * ldx + (lane >> 4);
-    const c_t* c1 = X + pair_col<32>(16 + (lane & 15), I, J) * ldx +
+    double2 v[NT][4][2];
+    const double2* c0 = X + pair_col<32>(lane & 15, I, J) * ldx + (lane >> 4);
+    const double2* c1 = X + pair_col<32>(16 + (lane & 15), I, J) * ldx +
                     (lane >> 4);
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -1930,11 +1966,11 @@ void jac_round_reg(
         v[i][s][1] = c1[r0 + 4 * s];
       }
     }
-    acc_t g[3][2];
+    d4_t g[3][2];
 #pragma unroll
     for (int q = 0; q < 3; ++q)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) g[q][0][e] = g[q][1][e] = (R)0;
+      for (int e = 0; e < 4; ++e) g[q][0][e] = g[q][1][e] = 0.0;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       if (wave + 8 * i >= ntiles) break;
@@ -1942,17 +1978,17 @@ void jac_round_reg(
       for (int s = 0; s < 4; ++s) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-          const R xr = v[i][s][q].x, xi = v[i][s][q].y;
-          g[q][0] = JT<R>::mfma(xr, xr, g[q][0]);
-          g[q][0] = JT<R>::mfma(xi, xi, g[q][0]);
-          g[q][1] = JT<R>::mfma(xr, xi, g[q][1]);
+          const double xr = v[i][s][q].x, xi = v[i][s][q].y;
+          g[q][0] = JT<double>::mfma(xr, xr, g[q][0]);
+          g[q][0] = JT<double>::mfma(xi, xi, g[q][0]);
+          g[q][1] = JT<double>::mfma(xr, xi, g[q][1]);
         }
-        const R ar = v[i][s][0].x, ai = v[i][s][0].y;
-        const R br = v[i][s][1].x, bi = v[i][s][1].y;
-        g[2][0] = JT<R>::mfma(ar, br, g[2][0]);
-        g[2][0] = JT<R>::mfma(ai, bi, g[2][0]);
-        g[2][1] = JT<R>::mfma(ar, bi, g[2][1]);
-        g[2][1] = JT<R>::mfma(-ai, br, g[2][1]);
+        const double ar = v[i][s][0].x, ai = v[i][s][0].y;
+        const double br = v[i][s][1].x, bi = v[i][s][1].y;
+        g[2][0] = JT<double>::mfma(ar, br, g[2][0]);
+        g[2][0] = JT<double>::mfma(ai, bi, g[2][0]);
+        g[2][1] = JT<double>::mfma(ar, bi, g[2][1]);
+        g[2][1] = JT<double>::mfma(-ai, br, g[2][1]);
       }
     }
     // waves 4-7 hand theirs to waves 0-3
@@ -1973,14 +2009,14 @@ void jac_round_reg(
         for (int h = 0; h < 2; ++h)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
-            R& at = sh.part[wave][(q * 2 + h) * 4 + e][lane];
+            double& at = sh.part[wave][(q * 2 + h) * 4 + e][lane];
             at = g[q][h][e] + at;
           }
     }
   }
   __syncthreads();
   // the four sums, added in order
-  R sum[3];
+  double sum[3];
 #pragma unroll
   for (int u = 0; u < 3; ++u) {
     const int idx = tid + 512 * u;
@@ -2004,20 +2040,18 @@ void jac_round_reg(
   // 2. the inner rounds (jac_inner_cross)
   const bool is_g = wave < 4;
   const int P = (tid & 255) >> 4, c = tid & 15;
-  const R zt = (R)zthr[bz];
-  const R tol2 = (R)(tol * tol);
-  c_t b[4];
+  const double zt = zthr[bz];
+  const double tol2 = tol * tol;
+  double2 b[4];
   if (is_g) {
     // entry (r, n) of quadrant q, half h: the lane and element holding it
     auto at = [&](int q, int h, int r, int n) {
-      const int e = sizeof(R) == 8 ? r >> 2 : r & 3;
-      const int l = 16 * (sizeof(R) == 8 ? r & 3 : r >> 2) + n;
-      return sh.s.sum[(q * 2 + h) * 4 + e][l];
+      return sh.s.sum[(q * 2 + h) * 4 + (r >> 2)][16 * (r & 3) + n];
     };
-    b[0] = JT<R>::mk(at(0, 0, P, c), at(0, 1, P, c) - at(0, 1, c, P));
-    b[1] = JT<R>::mk(at(2, 0, P, c), at(2, 1, P, c));
-    b[2] = JT<R>::mk(at(2, 0, c, P), -at(2, 1, c, P));
-    b[3] = JT<R>::mk(at(1, 0, P, c), at(1, 1, P, c) - at(1, 1, c, P));
+    b[0] = make_double2(at(0, 0, P, c), at(0, 1, P, c) - at(0, 1, c, P));
+    b[1] = make_double2(at(2, 0, P, c), at(2, 1, P, c));
+    b[2] = make_double2(at(2, 0, c, P), -at(2, 1, c, P));
+    b[3] = make_double2(at(1, 0, P, c), at(1, 1, P, c) - at(1, 1, c, P));
     if (P == c) {
       sh.cross.dg[c] = b[0].x;
       sh.cross.dg[16 + c] = b[3].x;
@@ -2026,20 +2060,20 @@ void jac_round_reg(
     const int r = 2 * P;
 #pragma unroll
     for (int u = 0; u < 4; ++u)
-      b[u] = JT<R>::mk(r + (u >> 1) == ((u & 1) ? 16 + c : c) ? (R)1 : (R)0,
-                       (R)0);
+      b[u] = make_double2(r + (u >> 1) == ((u & 1) ? 16 + c : c) ? 1.0 : 0.0,
+                          0.0);
   }
   __syncthreads();
-  if (!cross_check<R>(sh.cross, b, is_g, P, c, zt, tol2, (R)conv2,
+  if (!cross_check(sh.cross, b, is_g, P, c, zt, tol2, conv2,
                       &offmax[bz]))
     return;
   // X_IJ again, in the update's layout: behind the rounds where one
   // workgroup fills the CU's registers, after them where two do (each hides
   // the other's load)
-  constexpr bool kEarly = sizeof(R) * NT > 8;
-  c_t x[NT][8];
-  if constexpr (kEarly) reg_load<R, NT>(X, ldx, ntiles, I, J, wave, x);
-  const int rot = cross_sweeps<R>(sh.cross, b, is_g, P, c, zt, tol2, n_inner);
+  constexpr bool kEarly = NT > 1;
+  double2 x[NT][8];
+  if constexpr (kEarly) reg_load<NT>(X, ldx, ntiles, I, J, wave, x);
+  const int rot = cross_sweeps(sh.cross, b, is_g, P, c, zt, tol2, n_inner);
   if (rot) atomicAdd(&sh.cross.rot, rot);
   if (!is_g) {
     const int r = 2 * P;
@@ -2061,12 +2095,12 @@ void jac_round_reg(
     if (do_w) atomicAdd(qpairs + 1, 1);
   }
   // 3. X_IJ <- X_IJ Q (and W_IJ <- W_IJ Q)
-  if constexpr (!kEarly) reg_load<R, NT>(X, ldx, ntiles, I, J, wave, x);
-  reg_update<R, NT>(X, ldx, ntiles, I, J, wave, x, sh.s.Q0, sh.s.Q1, sh.s.Q2);
+  if constexpr (!kEarly) reg_load<NT>(X, ldx, ntiles, I, J, wave, x);
+  reg_update<NT>(X, ldx, ntiles, I, J, wave, x, sh.s.Q0, sh.s.Q1, sh.s.Q2);
   if (do_w) {
-    c_t* Wb = Wm + (int64_t)bz * sW;
-    reg_load<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x);
-    reg_update<R, NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x, sh.s.Q0,
+    double2* Wb = Wm + (int64_t)bz * sW;
+    reg_load<NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x);
+    reg_update<NT>(Wb, ldw, 4 * nchunk_w, I, J, wave, x, sh.s.Q0,
                       sh.s.Q1, sh.s.Q2);
   }
 }
@@ -2394,17 +2428,15 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
                               int64_t cols_p_, bool single_, int n_active) {
   batch = batch_;
   single = single_;
-  // A sweep's first round (and every round above 512 rows) runs as three
-  // launches: the fused jac_round (one workgroup per block pair) leaves each
-  // 64-row chunk's load latency exposed with only 1-2 workgroups per CU,
-  // while the three launches overlap them across all chunks.  FP32 problems
-  // of 320 to 512 rows fuse their first round by default: it keeps the whole
-  // block pair in LDS (jac_round_res), so only the tile load and store wait
-  // on memory.  The tile's LDS allows one workgroup per CU, which costs
-  // throughput on large batches of smaller problems (a 256-circuit batch of
-  // chi <= 128 ran 8% slower with every round fused), so those keep the
-  // three launches.  QTN_JACOBI_FUSED=1 / 0 forces fused / three-launch
-  // rounds everywhere.
+  // The fused round (one workgroup per block pair) leaves each 64-row
+  // chunk's load latency exposed with only 1-2 workgroups per CU; three
+  // launches overlap them across all chunks.  FP32 problems of 320 to 512
+  // rows fuse by default: their round keeps the whole block pair in LDS
+  // (jac_round_res), so only the tile load and store wait on memory.  The
+  // tile's LDS allows one workgroup per CU, which costs throughput on large
+  // batches of smaller problems (a 256-circuit batch of chi <= 128 ran 8%
+  // slower fused), so those keep the three launches.  QTN_JACOBI_FUSED=1 / 0
+  // forces fused / three-launch rounds everywhere.
   const size_t csz = single ? sizeof(float2) : sizeof(double2);
   rows_p = rows_p_;
   cols_p = cols_p_;
@@ -2424,13 +2456,12 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
     fused = it->second == QTN_TILING_W32_FUSED;
   }
   if (const char* e = getenv("QTN_JACOBI_W")) wdef = atoi(e) == 64 ? 64 : 32;
-  // Cross rounds of at most 512 rows keep the block pair in registers unless
-  // a fused tiling was tuned in or QTN_JACOBI_FUSED forces either of the
-  // others.  Against three launches a round: the 40-qubit chi-256 circuit
-  // 370 -> 292 ms in FP64 and 253 -> 238 ms in the chosen form (its FP32
-  // rounds against jac_round_res), 24 uneven circuits 340 -> 302 ms, single
-  // problems of 256 rows even.
-  reg = it == ctx->jac_tiling.end() || !fused;
+  // FP64 cross rounds of at most 512 rows keep the block pair in registers
+  // unless a fused tiling was tuned in or QTN_JACOBI_FUSED forces either of
+  // the others.  Against three launches a round: the 40-qubit chi-256 circuit
+  // 370 -> 292 ms, 24 uneven circuits 340 -> 302 ms, single problems of 256
+  // rows even.
+  reg = !single && !general && !fused;
   if (const char* e = getenv("QTN_JACOBI_FUSED")) {
     fused = atoi(e) != 0;
     reg = false;
@@ -2548,27 +2579,30 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
   } while (0)
 #define QTN_TIMED_LAUNCH(e0, e1, kern, grid, ...) \
   QTN_TIMED_LAUNCH_N(e0, e1, kern, grid, 256, __VA_ARGS__)
-  const bool one_launch = WW == 32 && reg_round(nchunk_x, Wm ? nchunk_w : 0, r);
+  const bool one_launch =
+      WW == 32 && reg_round(nchunk_x, Wm ? nchunk_w : 0, r);
   if (ctx_ && ctx_->prof) prof_reg.push_back(one_launch ? 1 : 0);
-  if (one_launch) {
-    const int nt = (std::max(nchunk_x, Wm ? nchunk_w : 0) + 1) / 2;
+  if constexpr (std::is_same<R, double>::value) {
+    if (one_launch) {
+      const int nt = (std::max(nchunk_x, Wm ? nchunk_w : 0) + 1) / 2;
 #define QTN_REG_ROUND(NT)                                                   \
-  QTN_TIMED_LAUNCH_N(ev[0], ev[1], (jac_round_reg<R, NT>), dim3(p, batch),  \
-                     kCrossThreads, X, ldx, sX, nchunk_x, Wm,               \
-                     ldw ? ldw : cols_p, sW, nchunk_w,                      \
-                     (const int*)(per_problem_w ? want_w : nullptr), p, r,  \
-                     tol, conv2, zthr, n_inner, counters, active, offmax,   \
-                     misc + 2)
-    if (nt <= 1)
-      QTN_REG_ROUND(1);
-    else if (nt == 2)
-      QTN_REG_ROUND(2);
-    else if (nt == 3)
-      QTN_REG_ROUND(3);
-    else
-      QTN_REG_ROUND(4);
+    QTN_TIMED_LAUNCH_N(ev[0], ev[1], (jac_round_reg<NT>), dim3(p, batch),  \
+                       kCrossThreads, X, ldx, sX, nchunk_x, Wm,               \
+                       ldw ? ldw : cols_p, sW, nchunk_w,                      \
+                       (const int*)(per_problem_w ? want_w : nullptr), p, r,  \
+                       tol, conv2, zthr, n_inner, counters, active, offmax,   \
+                       misc + 2)
+      if (nt <= 1)
+        QTN_REG_ROUND(1);
+      else if (nt == 2)
+        QTN_REG_ROUND(2);
+      else if (nt == 3)
+        QTN_REG_ROUND(3);
+      else
+        QTN_REG_ROUND(4);
 #undef QTN_REG_ROUND
-    return QTN_OK;
+      return QTN_OK;
+    }
   }
   if (fused && WW == 32) {
     if constexpr (std::is_same<R, float>::value) {
@@ -2591,23 +2625,29 @@ int32_t JacobiEngine::launch_round(hipStream_t s, void* Xv, int64_t ldx,
   QTN_TIMED_LAUNCH(ev[0], ev[1], (jac_gram<R, WW>), dim3(npart, p, batch),
                    (const c_t*)X, ldx, sX, p, r, nchunk_x, gram_cpw(nchunk_x),
                    G, active);
-  if (WW == 64 && p == 1) {
-    QTN_TIMED_LAUNCH_N(ev[2], ev[3], (jac_inner_whole<R>), dim3(1, batch),
-                       kWholeThreads, (const c_t*)G, npart, tol, tol, zthr,
-                       n_inner, Qc, flags, counters, active, offmax, misc + 2,
-                       (const int*)want_w, Wm ? (per_problem_w ? 2 : 1) : 0);
-  } else if (WW == 32 && cross_rounds && p > 1 && r > 0) {
-    QTN_TIMED_LAUNCH_N(ev[2], ev[3], (jac_inner_cross<R>), dim3(p, batch),
-                       kCrossThreads, (const c_t*)G, npart, p, tol, conv2,
-                       zthr, n_inner, Qc, flags, counters, active, offmax,
-                       misc + 2, (const int*)want_w,
-                       Wm ? (per_problem_w ? 2 : 1) : 0);
-  } else
-  QTN_TIMED_LAUNCH(ev[2], ev[3], (jac_inner<R, WW>), dim3(p, batch),
-                   (const c_t*)G, npart, p, tol, zthr, n_inner, Qc, flags,
-                   counters, active, offmax, misc + 2,
-                   (cross_rounds && p > 1 && r > 0) ? 1 : 0,
-                   (const int*)want_w, Wm ? (per_problem_w ? 2 : 1) : 0);
+  const int w_mode = Wm ? (per_problem_w ? 2 : 1) : 0;
+  bool inner_done = false;
+  if constexpr (std::is_same<R, double>::value) {
+    if (whole()) {
+      QTN_TIMED_LAUNCH_N(ev[2], ev[3], jac_inner_whole, dim3(1, batch),
+                         kWholeThreads, (const c_t*)G, npart, tol, tol, zthr,
+                         n_inner, Qc, flags, counters, active, offmax,
+                         misc + 2, (const int*)want_w, w_mode);
+      inner_done = true;
+    } else if (WW == 32 && cross_rounds && p > 1 && r > 0 && !general) {
+      QTN_TIMED_LAUNCH_N(ev[2], ev[3], jac_inner_cross, dim3(p, batch),
+                         kCrossThreads, (const c_t*)G, npart, p, tol, conv2,
+                         zthr, n_inner, Qc, flags, counters, active, offmax,
+                         misc + 2, (const int*)want_w, w_mode);
+      inner_done = true;
+    }
+  }
+  if (!inner_done)
+    QTN_TIMED_LAUNCH(ev[2], ev[3], (jac_inner<R, WW>), dim3(p, batch),
+                     (const c_t*)G, npart, p, tol, zthr, n_inner, Qc, flags,
+                     counters, active, offmax, misc + 2,
+                     (cross_rounds && p > 1 && r > 0) ? 1 : 0,
+                     (const int*)want_w, w_mode);
   QTN_TIMED_LAUNCH(ev[4], ev[5], (jac_update<R, WW>),
                    dim3(nchunk_x + (Wm ? nchunk_w : 0), p, batch), X, ldx,
                    sX, nchunk_x, Wm, ldw ? ldw : cols_p, sW, p, r,
@@ -2676,10 +2716,10 @@ int32_t JacobiEngine::account_sweep(int n_active, int qpairs, int qpairs_w,
     ctx->prof_ms[ku] += t;
   }
   // Rotated pairs are only known per sweep: spread over its rounds.  A
-  // one-launch round writes X_IJ once (the FP64 streaming jac_round reads it
+  // one-launch round writes X_IJ once (the streaming jac_round reads it
   // again too) and reads and writes W_IJ.
   const double f1 = nrounds ? (double)n_one / (double)nrounds : 0.0;
-  const bool streams = fused && W == 32 && !res && !reg;
+  const bool streams = fused && W == 32 && !res;
   ctx->prof_flops[kr] +=
       f1 * 8.0 * Wd * Wd * (qpairs * rows + qpairs_w * wrows);
   ctx->prof_bytes[kr] += f1 * Wd * c16 *
@@ -2723,9 +2763,9 @@ int32_t JacobiEngine::run32(qtn_ctx* ctx, float2* X, int64_t ldx, int64_t sX,
 
 // FP64: tol = sqrt(rows) eps / 2 and zero columns below rows eps |X|_F
 // (before the sweeps: never rotated; after them: exact zeros in sig).
-// FP32 (the chosen form's sweeps): tol = sqrt(rows) eps32, and columns below
+// FP32 (the chosen form's sweeps): tol = sqrt(rows) eps32 and columns below
 // 8 sqrt(rows) eps32 |X|_F (the rounding noise a column gathers over the
-// sweeps) are only rotated against larger ones (pair_open).
+// sweeps) are left alone.
 template <typename R>
 int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
                             int64_t ldx, int64_t sX,
@@ -2748,10 +2788,8 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   int n_inner_big = 1;
   if (const char* e = getenv("QTN_JACOBI_INNER")) n_inner_big = std::max(1, atoi(e));
   const int n_inner = (p == 1) ? 40 : n_inner_big;
-  // Stop once a sweep's largest scaled off-diagonal is below sqrt(conv2):
-  // sqrt(tol), so that the sweep's own rotations leave it converged, unless
-  // the caller refines the vectors (conv2_refined).
-  const double conv2 = conv2_refined > 0.0 ? conv2_refined : tol;
+  // stop once a sweep's largest scaled off-diagonal is below sqrt(tol)
+  const double conv2 = tol;
   const int nchunk_x = (int)(rows_p / 64);
   const int nchunk_w = (int)(cols_p / 64);
 
@@ -2820,18 +2858,18 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
   // checked on a fresh Gram by the second, so the two go out together (a
   // read-back less per solve; a problem done after the first skips the
   // second on the device).  Counted per pass while profiling.
-  const int passes = (p == 1 && !ctx->prof) ? 2 : 1;
+  const int passes = (whole() && !ctx->prof) ? 2 : 1;
   // One sweep: every round, then the convergence bookkeeping.
   auto enqueue_sweep = [&]() -> int32_t {
     for (int pass = 0; pass < passes; ++pass) {
       for (int r = 0; r < rounds; ++r) {
         if (this->W == 64)
-          QTN_TRY((launch_round<R, 64>(s, X, ldx, sX, Wm, sW, r, tol, conv2, n_inner,
-                                       nchunk_x, nchunk_w,
+          QTN_TRY((launch_round<R, 64>(s, X, ldx, sX, Wm, sW, r, tol, conv2,
+                                       n_inner, nchunk_x, nchunk_w,
                                        want_w_host != nullptr)));
         else
-          QTN_TRY((launch_round<R, 32>(s, X, ldx, sX, Wm, sW, r, tol, conv2, n_inner,
-                                       nchunk_x, nchunk_w,
+          QTN_TRY((launch_round<R, 32>(s, X, ldx, sX, Wm, sW, r, tol, conv2,
+                                       n_inner, nchunk_x, nchunk_w,
                                        want_w_host != nullptr)));
       }
       QTN_CHECK_HIP(hipGetLastError());
@@ -2851,7 +2889,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     std::memset(&key, 0, sizeof(key));
     key.dbl = dbl ? 1 : 0;
     key.w = this->W;
-    key.fused = (fused ? 1 : 0) + (reg ? 2 : 0);
+    key.fused = (fused ? 1 : 0) + (reg ? 2 : 0) + (general ? 4 : 0);
     key.cross = cross_rounds ? 1 : 0;
     key.batch = batch;
     key.p = p;

@@ -30,21 +30,27 @@ struct JacobiEngine {
   bool res_round(int nchunk_x, int nchunk_w) const {
     return single && nchunk_x * 64 <= 512 && nchunk_w * 64 <= 512;
   }
-  // Cross rounds of problems of at most 512 rows run as one launch with the
-  // block pair in registers (jac_round_reg)
+  // FP64 cross rounds of problems of at most 512 rows run as one launch with
+  // the block pair in registers (jac_round_reg)
   bool reg_round(int nchunk_x, int nchunk_w, int r) const {
     return reg && cross_rounds && p > 1 && r > 0 && nchunk_x * 64 <= 512 &&
            nchunk_w * 64 <= 512;
   }
   bool reg = false;
+  // FP64 problems of one block pair are solved whole (jac_inner_whole)
+  bool whole() const { return W == 64 && p == 1 && !single && !general; }
+  // Set before reserve(): every round as jac_gram, jac_inner and jac_update
+  // (or their fused forms), whose arithmetic the FP32 sweeps share.  The
+  // FP64 engine next to FP32 sweeps runs so: FP32 rounding reaches the
+  // amplitudes at 1e-6 to 1e-4, and a change in the last bit of any gate
+  // before an FP32 one draws it anew, so a circuit only keeps its result as
+  // long as all of its gates keep their arithmetic.
+  bool general = false;
   // the inner sweeps of outer rounds 1.. rotate only the cross pairs of
   // their two column blocks (round 0 of every outer sweep rotates all)
   bool cross_rounds = false;
   int64_t ldw = 0;     // leading dimension of W (0: cols_p)
   const int64_t* chimax_per = nullptr;  // host, per-problem cap (optional)
-  // > 0: the sweeps stop at this square of the largest scaled off-diagonal
-  // (for a caller that refines the vectors itself) instead of at tol
-  double conv2_refined = 0.0;
   int64_t* chimax_dev = nullptr;
   // device arrays (valid after reserve); Gram partials and rotation blocks
   // are complex double, or complex float when `single`

@@ -1,10 +1,10 @@
-"""The FP64 refinement of the chosen form's FP32 vectors: one capped layer on
-random states of square, wide and tall two-site matrices, flat and steeply
-decaying spectra (columns below the FP32 floor), caps next to the full rank
-and well below it.  What first order leaves of an FP32 error of 1e-4 is its
-square; the FP32 rounding of the two-site matrix itself (6e-8 per entry, a
-few 1e-6 over the sweeps) stays: amplitudes, i.e. states within 1e-10
-infidelity of the FP64 layer, spectra within 1e-6 and weights within 1e-8."""
+"""One capped layer in the chosen form on random states of square, wide and
+tall two-site matrices, flat and steeply decaying spectra (columns below the
+FP32 floor), caps next to the full rank and well below it, against the FP64
+layer.  The FP32 vectors mix kept and discarded directions by at most some
+1e-5: states within 1e-10 infidelity, spectra within 1e-6; values below the
+floor (2e-5 |X|, 4e-10 of the weight each) count as zeros, so weights agree
+within 1e-8; Newton-Schulz leaves the vectors orthonormal to 1e-12."""
 import numpy as np
 import pytest
 
