@@ -184,6 +184,9 @@ struct qtn_ctx {
   // destroyed with it.  parent is set on workers.
   qtn_ctx* parent = nullptr;
   std::vector<qtn_ctx*> workers;
+  // columns of the two-site matrices that the other executors of a layer
+  // solve meanwhile (0 outside a layer)
+  int64_t beside_cols = 0;
   int32_t worker(int i, qtn_ctx** out);
 };
 

@@ -1477,13 +1477,14 @@ int32_t apply_gates_grouped(qtn_ctx* ctx, int32_t ngates,
   struct Group {
     std::vector<int> idx;
     double cost;
+    int64_t cols;  // padded columns of a gate's problem
   };
   std::vector<Group> groups;
   double total = 0.0;
   for (auto& kv : bucket) {
     const double c = (double)kv.second.size() * (double)kv.first *
                      (double)kv.first;
-    groups.push_back({kv.second, c});
+    groups.push_back({kv.second, c, kv.first});
     total += c;
   }
   for (;;) {
@@ -1494,7 +1495,8 @@ int32_t apply_gates_grouped(qtn_ctx* ctx, int32_t ngates,
     if (g.cost * kExec <= total || (int)g.idx.size() < 2 * kMinChunk) break;
     const size_t half = g.idx.size() / 2;
     Group h{std::vector<int>(g.idx.begin() + half, g.idx.end()),
-            g.cost * (double)(g.idx.size() - half) / (double)g.idx.size()};
+            g.cost * (double)(g.idx.size() - half) / (double)g.idx.size(),
+            g.cols};
     g.cost -= h.cost;
     g.idx.resize(half);
     groups.push_back(std::move(h));
@@ -1558,6 +1560,18 @@ int32_t apply_gates_grouped(qtn_ctx* ctx, int32_t ngates,
     QTN_TRY(ctx->worker(e - 1, &exec[e]));
     exec[e]->jac_tiling = ctx->jac_tiling;  // the context's tuned tilings
   }
+  for (int e = 0; e < nexec; ++e)
+    for (int f = 0; f < nexec; ++f)
+      if (f != e)
+        for (int gi : plan[f])
+          exec[e]->beside_cols +=
+              groups[gi].cols * (int64_t)groups[gi].idx.size();
+  struct Alone {  // whichever way this returns
+    std::vector<qtn_ctx*>& exec;
+    ~Alone() {
+      for (qtn_ctx* c : exec) c->beside_cols = 0;
+    }
+  } alone{exec};
   // the workers' streams start after everything queued on this one
   QTN_CHECK_HIP(hipStreamSynchronize(ctx->stream));
   std::vector<int32_t> status(nexec, QTN_OK);

@@ -2459,9 +2459,19 @@ int32_t JacobiEngine::reserve(qtn_ctx* ctx, int batch_, int64_t rows_p_,
   // FP64 cross rounds of at most 512 rows keep the block pair in registers
   // unless a fused tiling was tuned in or QTN_JACOBI_FUSED forces either of
   // the others.  Against three launches a round: the 40-qubit chi-256 circuit
-  // 370 -> 292 ms, 24 uneven circuits 340 -> 302 ms, single problems of 256
-  // rows even.
-  reg = !single && !general && !fused;
+  // 370 -> 292 ms, 24 uneven circuits 340 -> 302 ms.
+  // Above 256 rows that takes the block pairs of five square problems, those
+  // that other executors of a layer solve meanwhile among them: a pair is
+  // one workgroup, and the three launches spread few pairs over more CUs.  512 x 512 alone, three launches / registers, ms per problem: one
+  // 11.0 / 20.9, four 4.7 / 5.4, six 3.8 / 3.7, twelve 3.2 / 2.1; 384 x 384:
+  // 8.7 / 11.6, 2.9 / 3.3, 2.3 / 2.2, 1.6 / 1.2.  Up to 256 rows the two are
+  // within 15% alone (256 x 256: 5.0 / 5.7, 1.36 / 1.58, 1.00 / 1.08, 0.63 /
+  // 0.55; 128 x 128: 2.2 / 1.9, .., 0.22 / 0.18) and beside the other groups
+  // of a layer registers are faster (24 qubits at chi 120: 66.7 / 61.0 ms).
+  const int64_t tall = std::max(rows_p, cols_p);
+  const int64_t solved = n_active >= 0 ? n_active : batch;
+  reg = !single && !general && !fused &&
+        (tall <= 256 || solved * cols_p + ctx->beside_cols >= 5 * tall);
   if (const char* e = getenv("QTN_JACOBI_FUSED")) {
     fused = atoi(e) != 0;
     reg = false;
