@@ -386,33 +386,35 @@ __device__ __forceinline__ void net_reduce(const double2* __restrict__ dev,
 // dependent launches, so independent steps share one (the 20-qubit QFT
 // network in its treewidth order, 249 steps in 26 levels: 7.26 ms -> 1.99 ms
 // per contract(); the 17-qubit one in the default order, a chain of 170
-// steps closed by a 1 x 1 x 131072 product: 40.4 ms -> 2.01 ms).  dev is the arena (the operands of a level and
-// its results are disjoint), steps its nsteps descriptors with ascending
-// first blocks, pool the legs.  kHeavy: the level holds tile or long steps,
-// whose accumulators allow two waves per SIMD; the levels without them take
-// the lighter instance.
+// steps closed by a 1 x 1 x 131072 product: 40.4 ms -> 2.01 ms).  dev is the
+// arena (the operands of a level and its results are disjoint), steps its
+// nsteps descriptors with ascending first blocks, pool the legs; this launch
+// takes the level's blocks from base on.  kHeavy: the level holds tile or
+// long steps, whose accumulators allow two waves per SIMD; the levels without
+// them take the lighter instance.
 template <bool kHeavy>
 __global__ __launch_bounds__(256) void net_level(
     const double2* __restrict__ dev, double2* __restrict__ out,
     const NetStep* __restrict__ steps, int nsteps,
-    const NetLeg* __restrict__ pool) {
+    const NetLeg* __restrict__ pool, uint32_t base) {
   __shared__ NetShared sh;
   __shared__ int s_at;
   const int tid = threadIdx.x;
+  const uint32_t bid = base + blockIdx.x;
   int at = 0;
   if (nsteps > 1) {
     // the last step whose first block is not after this one
     if (tid == 0) s_at = 0;
     __syncthreads();
     for (int i = tid; i < nsteps; i += 256)
-      if (steps[i].first <= blockIdx.x &&
-          (i + 1 == nsteps || steps[i + 1].first > blockIdx.x))
+      if (steps[i].first <= bid &&
+          (i + 1 == nsteps || steps[i + 1].first > bid))
         s_at = i;
     __syncthreads();
     at = __builtin_amdgcn_readfirstlane(s_at);
   }
   const NetStep st = steps[at];
-  const uint32_t blk = blockIdx.x - st.first;
+  const uint32_t blk = bid - st.first;
   const int nl = st.n_am + st.n_k + st.n_bn;
   if (tid < nl) sh.leg[tid] = pool[st.legs + tid];
   __syncthreads();
@@ -920,9 +922,12 @@ int32_t qtn_contract_network(qtn_ctx* ctx, int32_t ntensors,
     bool heavy = false;
     for (int i : lev[l])
       heavy = heavy || steps[i].d.kind == kTile || steps[i].d.kind == kLong;
-    hipLaunchKernelGGL(heavy ? net_level<true> : net_level<false>,
-                       dim3(blocks[l]), dim3(256), 0, s, (const double2*)dev,
-                       dev, ds, ns, dl);
+    // a grid holds fewer than 2^32 threads
+    constexpr uint32_t kMost = 1u << 23;
+    for (uint32_t at = 0; at < blocks[l]; at += kMost)
+      hipLaunchKernelGGL(heavy ? net_level<true> : net_level<false>,
+                         dim3(std::min(blocks[l] - at, kMost)), dim3(256), 0,
+                         s, (const double2*)dev, dev, ds, ns, dl, at);
     ds += ns;
   }
   QTN_CHECK_HIP(hipGetLastError());

@@ -83,3 +83,27 @@ def test_levels_that_would_not_fit_run_in_the_given_order(gpu_ctx):
     f = min(abs(tensors[4 * i + 2] @ (tensors[4 * i] @ tensors[4 * i + 1]) @
                 tensors[4 * i + 3]) for i in range(12))
     assert abs(got - ref) <= bound / f * scale
+
+
+def test_level_of_more_threads_than_a_grid_holds():
+    """Three independent products of 37856 x 37856 entries (69 GB), all made
+    before the first is closed: one level of more than 2^32 threads."""
+    from qaintensor import Context
+    rng = np.random.default_rng(6)
+    d, tensors, labels, close, ref, f = 37856, [], [], [], 1.0 + 0j, 1.0
+    for i in range(3):
+        u, w = crand(rng, d, 2), crand(rng, 2, d)
+        x, y = crand(rng, d), crand(rng, d)
+        u, w, x, y = (t / np.linalg.norm(t) for t in (u, w, x, y))
+        b = 10 * (i + 1)
+        tensors += [u, w, x, y]
+        labels += [[b + 1, i + 1], [i + 1, b + 2], [b + 1], [b + 2]]
+        close += [b + 1, b + 2]
+        ref *= (x @ u) @ (w @ y)
+        f = min(f, abs((x @ u) @ (w @ y)))
+    ctx = Context()
+    got = complex(ops.contract_network(tensors, labels, [1, 2, 3] + close,
+                                       ctx=ctx))
+    ctx.close()
+    # three factors, each two contractions of d terms of unit vectors
+    assert abs(got - ref) <= 3 * 2 * (d + 8) * EPS / f * abs(ref)
