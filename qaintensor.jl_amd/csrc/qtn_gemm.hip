@@ -247,7 +247,10 @@ __global__ __launch_bounds__(256) void gemm_grouped_kernel(
 // it loses where its last round of tiles leaves CUs idle (5 products of 512
 // x 512 x 512: 320 big tiles, two rounds, 163 us; 1280 small ones, five
 // quarter rounds, 133 us).
+// From 2^29 rows on, 32x32 tiles would ask for 2^32 threads in the grid's
+// first dimension, which a launch drops without an error.
 bool big_tiles(int64_t m, int64_t n, int64_t count) {
+  if (m >= (int64_t)1 << 29) return true;
   const int64_t big = ((m + 63) / 64) * ((n + 63) / 64) * count;
   const int64_t small = ((m + 31) / 32) * ((n + 31) / 32) * count;
   return 40 * ((big + 255) / 256) <= 11 * ((small + 255) / 256);

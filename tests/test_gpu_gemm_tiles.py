@@ -68,3 +68,37 @@ def test_gemm_tiles(gpu_ctx, m, n, k, ops, single):
             np.abs(beta) * np.abs(c)
         # complex products double the terms of every inner index
         assert np.all(np.abs(g - ref) <= (2 * k + 8) * eps * size)
+
+
+@pytest.mark.parametrize("m", [2**29 - 33, 2**29 + 33])
+def test_more_rows_than_small_tiles_can_launch(m):
+    """An outer product of a long column, on both sides of the 2^24 small
+    tiles that a grid's first dimension holds."""
+    import torch
+    from qaintensor import Context
+    n = 2
+    A = torch.randn(m, dtype=torch.complex64, device="cuda")
+    B = torch.tensor([0.5 - 2j, -1 + 0.25j], dtype=torch.complex64).cuda()
+    C = torch.zeros(n, m, dtype=torch.complex64, device="cuda")
+    one = np.array([1.0, 0.0], dtype=np.float32)
+    zero = np.zeros(2, dtype=np.float32)
+    ptr = ctypes.POINTER(ctypes.c_float)
+
+    def dev(t):
+        return ctypes.cast(t.data_ptr(), ptr)
+
+    torch.cuda.synchronize()
+    ctx = Context()
+    L.check(L.load().qtn_cgemm_dev(
+        ctx.handle, b"N", b"N", m, n, 1, one.ctypes.data_as(ptr), dev(A), m,
+        0, dev(B), 1, 0, zero.ctypes.data_as(ptr), dev(C), m, 0, 1))
+    ctx.sync()
+    # one complex product per entry
+    for j in range(n):
+        err = torch.abs(C[j] - A * B[j])
+        assert bool(torch.all(err <= 10 * 2.0**-23 * torch.abs(A) *
+                              abs(complex(B[j]))))
+        del err
+    ctx.close()
+    del A, B, C
+    torch.cuda.empty_cache()
