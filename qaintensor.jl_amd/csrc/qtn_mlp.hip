@@ -234,9 +234,8 @@ __device__ __forceinline__ f4_t mfma4(float a, float b, f4_t c) {
 // The weights of a wave's two row tiles t = wave, wave + 4 of a layer, all
 // loaded together once per launch: element s of tile i is W[16 t + l % 16,
 // 4 s + l / 16] (W column-major, K columns).  Tiles and columns behind the
-// last are read as the last: such tiles are not used, such columns meet zero
-// activations (no select, which would make every load wait for the one
-// before).
+// last are read as the last and not used (layer_tile selects; a select here
+// would make every load wait for the one before).
 __device__ __forceinline__ void load_layer(const float* __restrict__ W, int w,
                                            int K, int wave,
                                            float (&r)[2][32]) {
@@ -267,7 +266,7 @@ __device__ __forceinline__ void load_layer_t(const float* __restrict__ W,
 }
 
 // 16 rows x 16 samples: the tile's weights times act (K rows, zero padded to
-// a multiple of 16).
+// a multiple of 16; kT: K is one).
 template <bool kT>
 __device__ __forceinline__ f4_t layer_tile(const float (&r)[32], int K,
                                            const float (*act)[kAct]) {
@@ -280,7 +279,8 @@ __device__ __forceinline__ f4_t layer_tile(const float (&r)[32], int K,
     for (int e = 0; e < 4; ++e) {
       const int k = kT ? 16 * g + 4 * (lane >> 4) + e
                        : 16 * g + 4 * e + (lane >> 4);
-      acc = mfma4(r[4 * g + e], act[k][lane & 15], acc);
+      // an infinite weight of the last column must not meet the padding
+      acc = mfma4(kT || k < K ? r[4 * g + e] : 0.f, act[k][lane & 15], acc);
     }
   }
   return acc;
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(256) void mlp_pass(
     for (int i = 0; i < 2; ++i) {
       const int t = wave + 4 * i;
       if (t >= wt) break;
-      const f4_t acc = layer_tile<false>(w1[i], 16 * it, A0);
+      const f4_t acc = layer_tile<false>(w1[i], nin, A0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int m = 16 * t + 4 * (lane >> 4) + e;

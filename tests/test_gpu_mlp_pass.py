@@ -42,3 +42,20 @@ def test_pass_matches_oracle(gpu_ctx, nin, width, nb):
     assert abs(hist[0] - l0) <= 2e-5 * max(l0, 1e-3)
     assert np.all(np.isfinite(hist)) and np.all(np.isfinite(m.params()))
     m.free()
+
+
+@pytest.mark.parametrize("nin", [70, 72, 80, 127])
+def test_infinite_weight_of_the_last_input(gpu_ctx, nin):
+    """Inputs that fill no feature tile: the padding takes no part, so an
+    infinite weight gives the infinite output it gives without padding."""
+    w = 32
+    p = np.abs(Lrn.init_params(5, nin, w)) + np.float32(1e-3)
+    p[w * (nin - 1) + 7] = np.inf
+    X = (np.random.default_rng(nin).random((nin, 20)) + 0.1).astype(np.float32)
+    m = Lrn.RankMLP(p, nin, w, ctx=gpu_ctx)
+    with np.errstate(all="ignore"):
+        ref = O.mlp_forward(p.astype(np.float64), X.astype(np.float64), nin,
+                            w)[0]
+    assert np.all(ref == np.inf)
+    assert np.all(m.forward(X) == np.inf)
+    m.free()
