@@ -544,6 +544,22 @@ int32_t forward(qtn_mlp* m, int64_t nb, const float* X, Acts& a, bool keep) {
   hipStream_t s = ctx->stream;
   const int w = m->width, nin = m->nin;
   void* p;
+  QTN_TRY(ctx->buffer(kSlotY, (size_t)nb * sizeof(float), &p));
+  a.Y = (float*)p;
+  const Offsets o = offsets(nin, w);
+  const float* P = m->params;
+  if (!keep && one_pass(nin, w)) {
+    // Two workgroups per CU walk the samples with the weights they loaded.
+    // One per 16 samples against 512, us at 262144 samples: 335 / 237
+    // (72-128-128-1), 146 / 65 (10-16-16-1; layer by layer 84); even up to
+    // 8192 samples.
+    const int groups = (int)std::min<int64_t>((nb + 15) / 16, 512);
+    hipLaunchKernelGGL(mlp_pass<false>, dim3(groups), dim3(256), 0, s, P, o,
+                       m->np, nin, w, X, (const float*)nullptr, nb, a.Y,
+                       (float*)nullptr);
+    QTN_CHECK_HIP(hipGetLastError());
+    return QTN_OK;
+  }
   QTN_TRY(ctx->buffer(kSlotA0, (size_t)nin * nb * sizeof(float), &p));
   a.A0 = (float*)p;
   QTN_TRY(ctx->buffer(kSlotZ1, (size_t)w * nb * sizeof(float), &p));
@@ -554,18 +570,6 @@ int32_t forward(qtn_mlp* m, int64_t nb, const float* X, Acts& a, bool keep) {
   a.Z2 = (float*)p;
   QTN_TRY(ctx->buffer(kSlotA2, (size_t)w * nb * sizeof(float), &p));
   a.A2 = (float*)p;
-  QTN_TRY(ctx->buffer(kSlotY, (size_t)nb * sizeof(float), &p));
-  a.Y = (float*)p;
-  const Offsets o = offsets(nin, w);
-  const float* P = m->params;
-  if (!keep && one_pass(nin, w)) {
-    const int groups = (int)std::min<int64_t>((nb + 15) / 16, 1 << 20);
-    hipLaunchKernelGGL(mlp_pass<false>, dim3(groups), dim3(256), 0, s, P, o,
-                       m->np, nin, w, X, (const float*)nullptr, nb, a.Y,
-                       (float*)nullptr);
-    QTN_CHECK_HIP(hipGetLastError());
-    return QTN_OK;
-  }
   hipLaunchKernelGGL(prep_input, dim3(grid_for((int64_t)nin * nb)),
                      dim3(256), 0, s, X, nin, nb, a.A0);
   QTN_CHECK_HIP(hipGetLastError());

@@ -59,3 +59,14 @@ def test_infinite_weight_of_the_last_input(gpu_ctx, nin):
     assert np.all(ref == np.inf)
     assert np.all(m.forward(X) == np.inf)
     m.free()
+
+
+@pytest.mark.parametrize("nb", [8192, 8193, 16400])
+def test_forward_of_more_tiles_than_workgroups(gpu_ctx, nb):
+    p = Lrn.init_params(4, 72, 128)
+    X = np.random.default_rng(nb).random((72, nb)).astype(np.float32)
+    m = Lrn.RankMLP(p, 72, 128, ctx=gpu_ctx)
+    ref = O.mlp_forward(p.astype(np.float64), X.astype(np.float64), 72, 128)[0]
+    assert np.abs(m.forward(X) - ref).max() <= \
+        2e-5 * max(1.0, np.abs(ref).max())
+    m.free()
