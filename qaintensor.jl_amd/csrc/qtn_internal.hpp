@@ -179,6 +179,16 @@ struct qtn_ctx {
   void* pin_area[kPinAreas] = {};
   size_t pin_bytes[kPinAreas] = {};
   int32_t pinned_area(int area, size_t bytes, void** out);
+  // For the time between a copy out of an input area and the next wait: a
+  // return in between (an error) waits, so that the next call does not write
+  // the area under the copy.
+  struct PinGuard {
+    hipStream_t s;
+    bool waited = false;
+    ~PinGuard() {
+      if (!waited) (void)hipStreamSynchronize(s);
+    }
+  };
   // Worker contexts (same device, own stream and scratch) that run
   // independent batches concurrently with this one; created on first use,
   // destroyed with it.  parent is set on workers.

@@ -1049,6 +1049,7 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
   GateDesc* d_gd = (GateDesc*)((char*)ddesc + gate_bytes);
   GemmDesc<double>* d_g1 = (GemmDesc<double>*)(d_gd + ng);
   GemmDesc<double>* d_g2 = d_g1 + ng;
+  qtn_ctx::PinGuard guard{s};
   {
     char* c = (char*)pin;
     std::memcpy(c, gates, gate_bytes);
@@ -1430,6 +1431,7 @@ int32_t apply_gates_core(qtn_ctx* ctx, int ng, qtn_mps* const* ms,
     if (disc_out) disc_out[g] = total[g] > 0 ? disc[g] / total[g] : 0.0;
   }
   QTN_CHECK_HIP(hipStreamSynchronize(s));
+  guard.waited = true;
   return QTN_OK;
 }
 

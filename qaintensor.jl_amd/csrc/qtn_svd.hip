@@ -2805,6 +2805,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
 
   // Inputs through pinned memory in one copy (laid out as reserve() does),
   // results and flags straight into it.
+  qtn_ctx::PinGuard guard{s};
   {
     void* pin;
     const size_t bytes =
@@ -2927,6 +2928,7 @@ int32_t JacobiEngine::run_t(qtn_ctx* ctx, typename CType<R>::type* X,
     else
       QTN_TRY(enqueue_sweep());
     QTN_CHECK_HIP(hipStreamSynchronize(s));
+    guard.waited = true;
     if (ctx->prof)
       QTN_TRY(account_sweep(n_act, host_flags[2], host_flags[3], nchunk_x,
                             nchunk_w));
