@@ -807,9 +807,8 @@ int32_t qtn_mlp_train(qtn_mlp* m, int64_t nb, const float* X, const float* T,
   for (int t = 0; t < steps; ++t) {
     const int64_t start = ((int64_t)t * mb) % nb;
     const int64_t cnt = std::min(mb, nb - start);
-    m->step += 1;
-    const float c1 = 1.f - powf(b1, (float)m->step);
-    const float c2 = 1.f - powf(b2, (float)m->step);
+    const float c1 = 1.f - powf(b1, (float)(m->step + 1));
+    const float c2 = 1.f - powf(b2, (float)(m->step + 1));
     if (one_pass(m->nin, m->width)) {
       float* part;
       int parts;
@@ -821,6 +820,7 @@ int32_t qtn_mlp_train(qtn_mlp* m, int64_t nb, const float* X, const float* T,
                          (float*)pl + t, m->params, m->m1, m->m2, lr, b1, b2,
                          eps, c1, c2);
       QTN_CHECK_HIP(hipGetLastError());
+      m->step += 1;
       continue;
     }
     QTN_TRY(loss_grad(m, cnt, dX + start * m->nin, dT + start,
@@ -829,6 +829,7 @@ int32_t qtn_mlp_train(qtn_mlp* m, int64_t nb, const float* X, const float* T,
                        m->params, (const float*)m->grads, m->m1, m->m2, m->np,
                        lr, b1, b2, eps, c1, c2);
     QTN_CHECK_HIP(hipGetLastError());
+    m->step += 1;
   }
   if (loss_hist && steps > 0)
     QTN_CHECK_HIP(hipMemcpyAsync(loss_hist, pl, steps * sizeof(float),
