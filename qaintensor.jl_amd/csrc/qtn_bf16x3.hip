@@ -116,13 +116,16 @@ __global__ void split_b(const double2* __restrict__ B, int64_t ldb, int64_t K,
 //
 // The FP32 accumulators are added to FP64 ones every kFlush steps: over 2048
 // embedded inner indices the 384 FP32 additions per entry cost far more
-// accuracy than the operands' 24 bits.  The conversions run on the vector
-// units beside the other wave's MFMAs and cost what the prefetch gains.  Bound
-// by the matrix cores and the LDS reads that feed them (18 KB per wave and
-// step).  <psi|H|psi> of 24 sites at chi 1024 (the largest products 6144 x
-// 2048 x 2048): 298 us per product, about 1000 TF of bf16, and a relative
-// error of 2e-8..1e-7; one buffer, no prefetch and FP32 accumulation: 293 us
-// and 3e-7..7e-6.  128 x 64 tiles with three workgroups per CU: 339 us.
+// accuracy than the operands' 24 bits.  Bound by the matrix cores and the LDS
+// reads that feed them (18 KB per wave and step).  Against one buffer, no
+// prefetch, 64 x 64 per wave and FP32 accumulation, us (TF of bf16, relative
+// error on Gaussian operands): 512^3 73 / 54 (119), 1024^3 147 / 110 (468), 3072
+// x 2048 x 1024 377 / 379 (816), 1024 x 3072 x 2048 399 / 433 (714), 2048^3 424
+// / 462 (892), 2048 x 8192 x 2048 1730 / 1841 (896); 5e-7..1e-6 / 1.0e-7 at
+// every size.  <psi|H|psi> at chi 512, 1024, 2048: 2.48 / 1.90, 6.75 / 6.10,
+// 36.1 / 34.2 ms and 2e-7..6e-6 / 2e-8..4e-7.  128 x 64 tiles with three
+// workgroups per CU were slower (339 us against 298 at chi 1024), 64 x 64 per
+// wave with two buffers too (2048^3 686 us).
 constexpr int kFlush = 2;
 constexpr int kGemmThreads = 512;
 
@@ -133,13 +136,11 @@ __global__ __launch_bounds__(kGemmThreads) void gemm_bf16x3(
   __shared__ __attribute__((aligned(16))) uint16_t As[2][3][kBM][kLdsK];
   __shared__ __attribute__((aligned(16))) uint16_t Bs[2][3][kBN][kLdsK];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  // consecutive workgroups go to the 8 XCDs in turn: each takes a contiguous
-  // run of tiles
-  const uint32_t nt = gridDim.x * gridDim.y;
-  uint32_t t = blockIdx.x + gridDim.x * blockIdx.y;
-  t = (t % 8) * (nt / 8) + min(t % 8, nt % 8) + t / 8;
-  const int64_t m0 = (int64_t)(t % gridDim.x) * kBM;
-  const int64_t n0 = (int64_t)(t / gridDim.x) * kBN;
+  // Tiles in launch order: consecutive workgroups go to the 8 XCDs in turn,
+  // so that those of one XCD share every eighth row of tiles over several
+  // columns.  A contiguous run of tiles per XCD is one column with all rows of
+  // A (2048 x 8192 x 2048: 1993 us against 1841; 2048^3 474 against 462).
+  const int64_t m0 = (int64_t)blockIdx.x * kBM, n0 = (int64_t)blockIdx.y * kBN;
   const int wm = (wave & 3) * 32, wn = (wave >> 2) * 64;
   const int64_t planeA = Mp * Kp, planeB = Np * Kp;
   f32x4 acc[2][4];
