@@ -234,8 +234,9 @@ __device__ __forceinline__ f4_t mfma4(float a, float b, f4_t c) {
 // The weights of a wave's two row tiles t = wave, wave + 4 of a layer, all
 // loaded together once per launch: element s of tile i is W[16 t + l % 16,
 // 4 s + l / 16] (W column-major, K columns).  Tiles and columns behind the
-// last are read as the last and not used (layer_tile selects; a select here
-// would make every load wait for the one before).
+// last are read as the last (no select, which would make every load wait for
+// the one before): such tiles are not used, such columns are cleared once all
+// loads are under way (clear_behind).
 __device__ __forceinline__ void load_layer(const float* __restrict__ W, int w,
                                            int K, int wave,
                                            float (&r)[2][32]) {
@@ -265,8 +266,21 @@ __device__ __forceinline__ void load_layer_t(const float* __restrict__ W,
   }
 }
 
+// Zero in place of the columns from K on: against zero activations an
+// infinite weight read there would give NaN.
+__device__ __forceinline__ void clear_behind(int K, float (&r)[2][32]) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int s = 0; s < 32; ++s)
+    if (4 * s + 4 > K) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        r[i][s] = 4 * s + (lane >> 4) < K ? r[i][s] : 0.f;
+    }
+}
+
 // 16 rows x 16 samples: the tile's weights times act (K rows, zero padded to
-// a multiple of 16; kT: K is one).
+// a multiple of 16).
 template <bool kT>
 __device__ __forceinline__ f4_t layer_tile(const float (&r)[32], int K,
                                            const float (*act)[kAct]) {
@@ -279,8 +293,7 @@ __device__ __forceinline__ f4_t layer_tile(const float (&r)[32], int K,
     for (int e = 0; e < 4; ++e) {
       const int k = kT ? 16 * g + 4 * (lane >> 4) + e
                        : 16 * g + 4 * e + (lane >> 4);
-      // an infinite weight of the last column must not meet the padding
-      acc = mfma4(kT || k < K ? r[4 * g + e] : 0.f, act[k][lane & 15], acc);
+      acc = mfma4(r[4 * g + e], act[k][lane & 15], acc);
     }
   }
   return acc;
@@ -338,6 +351,7 @@ __global__ __launch_bounds__(256) void mlp_pass(
   load_layer(P + o.W1, w, nin, wave, w1);
   load_layer(P + o.W2, w, w, wave, w2);
   if constexpr (kGrad) load_layer_t(P + o.W2, w, wave, w2t);
+  clear_behind(nin, w1);
   const float inv = 1.0f / (float)nb;
   for (int64_t n0 = (int64_t)blockIdx.x * 16; n0 < nb;
        n0 += (int64_t)gridDim.x * 16) {
@@ -362,7 +376,7 @@ __global__ __launch_bounds__(256) void mlp_pass(
     for (int i = 0; i < 2; ++i) {
       const int t = wave + 4 * i;
       if (t >= wt) break;
-      const f4_t acc = layer_tile<false>(w1[i], nin, A0);
+      const f4_t acc = layer_tile<false>(w1[i], 16 * it, A0);
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int m = 16 * t + 4 * (lane >> 4) + e;
