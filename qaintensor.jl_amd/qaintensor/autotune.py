@@ -4,7 +4,8 @@ For every column bucket (the padded width of the two-site matrix, a
 multiple of 64), sweep precision and batch class (floor(log2) of the number
 of problems one batched SVD solves, capped at 6) the library can run three
 tilings:
-32x32 Gram blocks in three launches a round (QTN_TILING_W32), the same in
+32x32 Gram blocks in three launches a round (QTN_TILING_W32; in FP64 most
+rounds in one where their block pairs fill the card), the same in
 one fused launch (QTN_TILING_W32_FUSED), or 64x64 Gram blocks
 (QTN_TILING_W64).  qtn_tune_jacobi times each on a batch of synthetic
 complex Gaussian problems of the bucket's size with HIP events and keeps
