@@ -223,6 +223,10 @@ __host__ __device__ inline int64_t share_size(int64_t np) {
   return (np + 4) / 4 * 4;
 }
 
+// At every batch: gradient of 72-128-128-1, host copies included, layer by
+// layer / one pass: 1 sample 0.19 / 0.12 ms, 256 0.29 / 0.17, 4096 1.8 / 0.6,
+// 65536 26 / 8.7, 262144 117 / 35 (256 workgroups walk their tiles in series,
+// the layers' FP32 products do not use the matrix cores).
 bool one_pass(int nin, int w) {
   return w % 16 == 0 && w <= kMaxW && nin <= kMaxIn;
 }
